@@ -34,6 +34,7 @@ ROOT = os.path.dirname(os.path.abspath(__file__))
 sys.path.insert(0, ROOT)
 
 FP32_PEAK_TFLOPS = 157.3
+F16_PEAK_TFLOPS = 2516.6   # dense 16-bit matrix peak: 1024 FLOP per cycle and SIMD at 2.4 GHz
 VALU_F32_PEAK_TFLOPS = 78.6   # one FP32 FMA per lane per cycle (no packed instructions)
 METRIC = "member·pixel evals/sec + ES iterations/sec (512² 4-tex, pop 8192), % roofline"
 KERNELS = ("batch", "perturb", "pop_eval", "es_grad", "adam", "lat_eps", "lat_pair", "lat_gather", "qat_search", "decode",
@@ -390,7 +391,7 @@ def run_gpu(w, steps, warmup, fd_steps=0, seconds=0.0, settle=0.0):
     assert np.isfinite(img).all() and np.isfinite(loss)
     name = "k_pop_eval"
     if tr.on_matrix_cores("pop_eval"):
-        name = ("k_pop_pair_own" if tr.on_matrix_cores("pop_pair_own") else "k_pop_pair") if tr.on_matrix_cores("pop_pair") else "k_pop_mfma"
+        name = "k_pop_split" if tr.on_matrix_cores("pop_split") else "k_pop_mfma"
     out = {"z": z, "p": p, "tgt": tgt, "steps": steps, "el": el, "kernels": kernels, "fd": fd, "loss": loss, "pop_kernel": name,
            "refit": refit, "dct_codes": getattr(tr, "dct_codes", None), "settle": {"seconds": settle, "iterations": settle_iters}}
     if w.dct_q:
@@ -406,6 +407,8 @@ def roofline_of(w, r):
     achieved = pop_flop / (pe["ms_mean"] * 1e-3) / 1e12
     # the VALU kernels (--valu) against the FP32 VALU peak without packed instructions
     bound, peak = ("mfma", FP32_PEAK_TFLOPS) if r["pop_kernel"] != "k_pop_eval" else ("valu", VALU_F32_PEAK_TFLOPS)
+    if r["pop_kernel"] == "k_pop_split":   # each multiply-add is three 16-bit products
+        peak = round(F16_PEAK_TFLOPS / 3, 1)
     roof = {"bound": bound, "achieved": round(achieved, 3), "peak": peak, "unit": "TFLOP/s",
             "frac": round(achieved / peak, 4), "traffic": None, "kernel": r["pop_kernel"],
             "flop_per_launch": pop_flop, "ms_per_launch": pe["ms_mean"]}

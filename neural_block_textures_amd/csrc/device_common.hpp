@@ -27,6 +27,19 @@ constexpr int kMaxLevels = 3, kMaxPos = 16, kMaxOut = 12, kMaxHidden = 8, kMaxWi
 constexpr int kMinibatchSlack = 256;
 __host__ __device__ constexpr int minibatch_rows(int nin) { return 4 * ((nin + 3) / 4); }
 
+// The minibatch as the split population kernel reads it (split_mlp.hpp), slot by slot: the features times kSplitFeat in
+// two 16-bit parts, split_inputs(nin) hi parts then as many lo parts (zero past nin), and the targets, split_targets(nout)
+// floats. Both arrays carry kSplitSlack slots past the last one.
+// At most 16 inputs: a first layer of more would need another operand layout (no compiled shape has them). At most two
+// hidden layers: the values of a third, scaled as the first two are, would leave the 16-bit range.
+__host__ __device__ constexpr bool split_pays(int nin, int nl) { return nin <= 16 && nl <= 2; }
+__host__ __device__ constexpr int split_inputs(int nin) { return nin <= 8 ? 8 : 16; }
+__host__ __device__ constexpr int split_targets(int nout) { return nout <= 4 ? nout : 4 * ((nout + 3) / 4); }
+constexpr int kSplitSlack = 256;
+constexpr float kSplitFeat = 1.0f;
+// the power of two that the largest weight of the first hidden layer, the second and the output layer is scaled below
+constexpr int kSplitExp[3] = { 4, 4, 12 };
+
 // ---------------------------------------------------------------- model description
 struct DevLevel {
     int W, H, C, nearest;
@@ -70,6 +83,7 @@ __host__ __device__ __forceinline__ uint64_t noise_head(uint64_t seed, uint32_t 
 __host__ __device__ __forceinline__ uint64_t noise_bits(uint64_t head, uint64_t index) { return mix64(head + index * kPhi64); }
 // x is not a NaN, decided on its bits (valid in code compiled to assume no NaNs, where a float test folds away)
 __device__ __forceinline__ bool not_nan_bits(float x) { return (__float_as_uint(x) & 0x7fffffffu) <= 0x7f800000u; }
+__device__ __forceinline__ bool not_nan_bits_d(double x) { return ((uint64_t)__double_as_longlong(x) & 0x7fffffffffffffffull) <= 0x7ff0000000000000ull; }
 __host__ __device__ __forceinline__ uint32_t noise_uniform(uint32_t u, uint32_t n) { return (uint32_t)(((uint64_t)u * (uint64_t)n) >> 32); }
 // One standard normal draw: the 24-bit halves of the key select the two factors, whose product
 // is the reference's sqrtf(-2 logf(u1)) * cosf(2 pi u2) bit for bit (one IEEE multiply).

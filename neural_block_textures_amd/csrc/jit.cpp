@@ -90,6 +90,8 @@ std::vector<std::string> expressions(const std::string& shape, const DevModel& m
         v.push_back(e("k_pop_mfma", std::to_string(a_fd) + ", " + c + ", 0"));
         v.push_back(e("k_pop_mfma", std::to_string(a_es) + ", " + c + ", 1"));
         v.push_back(e("k_pop_mfma", std::to_string(a_es) + ", " + c + ", 2"));
+        if (split_pays(m.nin, m.nl))
+            for (int from : { 1, 2 }) v.push_back(e("k_pop_split", c + ", " + std::to_string(from) + ", false"));
         v.push_back(e("k_lat_pair_mfma", std::to_string(a_es) + ", " + c));
     }
     v.push_back(e("k_qat_mfma", std::to_string(unit ? kActFold : kActAny) + ", " + c));
@@ -207,7 +209,7 @@ bool jit_prepare(Impl& I, std::string& why) {
     const std::string shape = jit_shape_name(js);
     const std::string csrc = source_dir();
     std::string key_src;
-    for (const char* f : { "kern_pop.hpp", "kern_valu.hpp", "mfma_mlp.hpp", "device_common.hpp", "noise_math.hpp" }) {
+    for (const char* f : { "kern_pop.hpp", "kern_valu.hpp", "split_mlp.hpp", "mfma_mlp.hpp", "device_common.hpp", "noise_math.hpp" }) {
         std::string t;
         if (csrc.empty() || !read_file(csrc + "/" + f, t)) { why = "the kernel sources are not next to the library (" + csrc + ")"; return false; }
         key_src += t;

@@ -1,10 +1,12 @@
 // Device code only (compiled into libntc_hip.so for the fixed shapes of shapes.hpp, and by hipRTC at
 // init for the shape of a model that is none of them, jit.cpp); the launchers are in kernels_pop.hip.
 //
-// The population evaluation (MlpTrainer::step's member losses, main.cpp:1848-1861) on the FP32
+// The population evaluation (MlpTrainer::step's member losses, main.cpp:1848-1861) on the
 // matrix cores of gfx950, for the fixed shapes the matrix cores pay off for (MfmaShape::kOk) and
 // 0 <= leak <= 1; other models use the VALU kernel of kernels_mlp.hip. In an ES step the kernel
-// stages the pair's perturbed weights itself (no member weight sets in memory).
+// stages the pair's perturbed weights itself (no member weight sets in memory). ES steps of the shapes split_pays
+// takes run on k_pop_split (16-bit instructions, operands in two parts); central differences, and the ES steps of
+// the other shapes, on k_pop_mfma (32-bit instructions), which the following is about.
 //
 // On this chip an FP32 matrix instruction and a VALU instruction do not run concurrently on a
 // SIMD (a 16x16x4 f32 step costs 32 cycles, a VALU instruction 4, and their mixes take the sum),
@@ -25,7 +27,7 @@
 // while the current ones compute. Each lane adds the float terms cw (d d) (main.cpp:1747) of its
 // output channels into a double; the two waves of a member are added in a fixed order.
 #pragma once
-#include "mfma_mlp.hpp"
+#include "split_mlp.hpp"
 
 namespace ntc_hip {
 
@@ -99,6 +101,7 @@ __device__ __forceinline__ void pop_load(PopTileIn<S>& in, __amdgpu_buffer_rsrc_
 // s2 = -log2(e) s: the kernels scale the output layer by kNegLog2e (scale_output), so the matrix
 // instruction delivers s2 directly
 constexpr float kNegLog2e = -1.44269504088896341f;
+constexpr double kNegLog2eD = -1.44269504088896340736;
 __device__ __forceinline__ float sigmoid_hw2(float s2) { return __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(s2)); }
 
 // the output of a pre-activation: clamp(s + 0.5) with --clamp, else the sigmoid of a pre-activation
@@ -285,56 +288,26 @@ __global__ void __launch_bounds__(64 * kPopWaves) __attribute__((amdgpu_waves_pe
     }
 }
 
-// ---- The ES population with the pair's first layer shared (models with one or two 16-unit hidden tiles, except the
-// pixel-per-lane shapes; the launch takes it where a chunk's first-layer pre-activations stay in the L2). More than 4
-// outputs: the output tile on the matrix cores, its rows packed (out_at); at most 4: valu_out_g's sums and
-// reduce-scatter on the VALU, both members' output weights read from an LDS table (in registers they would cost a
-// wave per SIMD). The two members of a pair differ
-// in every weight by +-sigma eps, so their first layers are h+- = u +- d with u the unperturbed layer's pre-activations
-// (bias + w x, the same for every pair; the minibatch launch computes it once per step, lay1[unit][slot]) and d the
-// perturbation's: h- = 2 u - h+, one fused multiply-add per value instead of the - member's first-layer matrix
-// instructions. A wave evaluates both members of its pair on one 16-slot tile at a time (two independent chains
-// after the first layer), on tiles wave, wave + 4, ... of the chunk; the member's A operands stay in VGPRs, the
-// biases come from LDS rows in operand layout (every lane of a group reads the same 16 bytes), so the two members'
-// weights fit the four waves per SIMD the chains need. Every parameter is the reference's w0 +- sigma eps
-// (main.cpp:1852-1856) scaled as k_pop_mfma scales it; the - member's first layer is within a few roundings of its
-// own chain's, inside the 1e-5 member-loss bar.
-template <class S, bool = MfmaShape<S>::kOk>
-struct PopPairOk { static constexpr bool value = false; };
+// waves per SIMD the split kernel's register allocation aims at (more would spill)
 template <class S>
-struct PopPairOk<S, true> {
-    static constexpr bool value = MfmaShape<S>::kHt <= 2 && MfmaShape<S>::kH % 16 == 0 && !pop_own<S>();
+constexpr int split_occupancy() { return MfmaShape<S>::kH > 48 ? 2 : ((MfmaShape<S>::kIn <= 8 && MfmaShape<S>::kH <= 32 && (!valu_out<S>() || MfmaShape<S>::kHt == 1)) ? 4 : 3); }
+// the minibatch slot by slot (device_common.hpp, split_inputs) and the step's layer scales (split_mlp.hpp)
+struct SplitIn {
+    const u4v* feat;
+    const float* tgt;
+    const float* scales;
 };
-template <class S>
-constexpr bool pop_pair_ok() { return PopPairOk<S>::value; }
-// bias rows per member: the first layer's kHt tiles, each deeper hidden layer's kHt, the output tile
-template <class S>
-constexpr int pair_bias_rows() { return MfmaShape<S>::kHt * MfmaShape<S>::kNL + 1; }
-// a member's parameters in LDS, padded to whole 16-byte pieces
-template <class S>
-constexpr int pair_p_pad() { return (MfmaShape<S>::kP + 3) & ~3; }
 
-// UnitCw: every channel weight is 1 (a single texture, or equally weighted ones), so cw (d d) is d d without a multiply
-// Stages both members of an ES pair in LDS: wpm_s = w0 + sigma eps, then (PP floats on) w0 - sigma eps (main.cpp:1852-1856),
-// scaled as k_pop_mfma scales its registers (the hidden layers by the folded activation's (1 + leak) / 2, the output
-// layer by -log2 e for the hardware sigmoid); the biases also to their operand rows bias_s [member][row][4 g + r]
-// (the output tile's padding rows zero), and cw_s[4 g + r] = the channel weight of output register r of lane group g.
-// The Gaussians are drawn here (kDraw: the chunk-0 block writes them for the update) or read (kReadEps).
-template <class S, bool Clamp, int From>
-__device__ __forceinline__ void pair_stage(const DevModel& m, const PopSource& src, int pair, int ch, float* __restrict__ wpm_s,
-                                           float* __restrict__ bias_s, float* __restrict__ cw_s) {
-    using Q = MfmaShape<S>;
-    constexpr int H = Q::kH, NIN = Q::kIn, NO = Q::kNout, RO = out_regs<S>(), NB = pair_bias_rows<S>(), PP = pair_p_pad<S>();
-    constexpr int kPout = H * NIN + H + (Q::kNL - 1) * (H * H + H);   // the first output-layer parameter
+// Stages both members of an ES pair in LDS (SplitLds): w0 + sigma eps, then w0 - sigma eps (main.cpp:1852-1856), in two
+// parts with their factors. The Gaussians are drawn here (kDraw: the chunk-0 block writes them for the update) or read
+// (kReadEps).
+template <class S, int From>
+__device__ __forceinline__ void split_stage(const PopSource& src, const SplitFactors f, int pair, int ch, unsigned* __restrict__ lds) {
+    using L = SplitLds<S>;
+    constexpr int kP = MfmaShape<S>::kP;
     const uint64_t head = noise_head(src.seed, NS_MLP, src.step, (uint32_t)pair);
-    float* eg = src.eps + (size_t)pair * Q::kP;
-    const float fb = fold_scale(m.leak);
-    if (tid_x() < 16) {   // the output tile's padding rows; the channel weights (zero on padding)
-        const int gg = tid_x() >> 2, r = tid_x() & 3, c = out_at<S>(gg, r);
-        if (c < 0) { bias_s[(NB - 1) * 16 + tid_x()] = 0.0f; bias_s[(2 * NB - 1) * 16 + tid_x()] = 0.0f; }
-        cw_s[tid_x()] = c < 0 ? 0.0f : m.cw[c];
-    }
-    for (int k = tid_x(); k < Q::kP; k += 64 * kPopWaves) {
+    float* eg = src.eps + (size_t)pair * kP;
+    for (int k = tid_x(); k < kP; k += 64 * kPopWaves) {
         float e;
         if constexpr (From == kDraw) {
             e = gauss_at(src.nt, head, (uint64_t)k);
@@ -343,325 +316,196 @@ __device__ __forceinline__ void pair_stage(const DevModel& m, const PopSource& s
             e = eg[k];
         }
         const float w0 = src.w0[k];
-        const float sc = k < kPout ? fb : (Clamp ? 1.0f : kNegLog2e);
-        const float vp = __builtin_fmaf(src.sigma, e, w0) * sc, vm = __builtin_fmaf(-src.sigma, e, w0) * sc;
-        wpm_s[k] = vp;
-        wpm_s[PP + k] = vm;
-        int row = -1, col = 0;   // a bias: its operand row and column
-        if (k >= H * NIN && k < H * NIN + H) {
-            row = (k - H * NIN) >> 4; col = (k - H * NIN) & 15;
-        } else if (k >= H * NIN + H && k < kPout) {
-            const int q = k - (H * NIN + H), l = q / (H * H + H), o = q - l * (H * H + H) - H * H;
-            if (o >= 0) { row = Q::kHt * (1 + l) + (o >> 4); col = o & 15; }
-        } else if (k >= kPout + NO * H) {
-            const int c = k - (kPout + NO * H);
-            row = NB - 1; col = 4 * (c / RO) + c % RO;   // output c sits in register c % RO of lane group c / RO
-        }
-        if (row >= 0) { bias_s[row * 16 + col] = vp; bias_s[(NB + row) * 16 + col] = vm; }
+        const int l = L::layer(k), at = L::pos(k);
+        const bool b = L::bias(k);
+        const double fw = l == 0 ? f.w1 : (l == 1 ? f.w2 : f.w3), fb = l == 0 ? f.b1 : (l == 1 ? f.b2 : f.b3), ff = b ? fb : fw;
+        lds[at] = split_param(w0, src.sigma, e, ff, b);
+        lds[L::kWords + at] = split_param(w0, -src.sigma, e, ff, b);
     }
 }
 
+// Flat parameter k of a member staged in LDS as the 32-bit evaluation takes it (the layers' factors without their powers of
+// two): both parts' sum; hi alone where that is an infinity.
+template <class S>
+struct SplitParam32 {
+    const unsigned* lds;
+    SplitScale sc;
+    __device__ __forceinline__ float operator()(int k) const {
+        using L = SplitLds<S>;
+        const int l = L::layer(k);
+        const unsigned v = lds[L::pos(k)];
+        if (L::bias(k)) return __uint_as_float(v) / (kSplitFeat * sc.s1 * (l > 0 ? sc.s2 : 1.0f) * (l > 1 ? sc.s3 : 1.0f));
+        const float h = (float)__builtin_bit_cast(_Float16, (unsigned short)v), lo = (float)__builtin_bit_cast(_Float16, (unsigned short)(v >> 16));
+        return ((v & 0x7fffu) == 0x7c00u ? h : h + lo) / (l == 0 ? sc.s1 : (l == 1 ? sc.s2 : sc.s3));
+    }
+};
+
+// ---- The ES population on the 16-bit matrix instructions with 32-bit operands in two parts (split_mlp.hpp), for the shapes
+// of at most 16 inputs and two hidden layers.
+//
+// Block (pair, chunk) has four waves: wave w evaluates member 2 pair + (w & 1) on the passes 2 q + (w >> 1) of the chunk's
+// slots, 32 slots a pass (two 16-slot tiles) for the models with more than 4 outputs, 64 (four tiles) for the others, whose
+// four output tiles meet in one accumulator so that every lane ends with the outputs of its own slot. A member's operands and
+// biases stay in VGPRs for the whole chunk (both parts of every weight: 32 VGPRs for the 32-wide models, 112 for the 64-wide
+// ones), so a pass reads only its inputs, the next pass's while it computes: 16 bytes of features per lane and tile and the
+// lane's targets, both laid out slot by slot by the minibatch launch.
+// What bounds it is the issue of matrix and VALU instructions, which hardly overlap: a 32-wide, 12-output tile takes 11
+// matrix instructions of 16 cycles and about 75 VALU ones (300 cycles: 2.5 each, conversions 4.5, exp2 and the reciprocal 8.6),
+// where the 32-bit instructions of k_pop_mfma take 28 of 32 cycles beside their VALU work; material512's population takes 530
+// cycles a tile, the staging of its members' weights among them. Whole launches against the 32-bit kernels (MI355X, ms):
+// material512 0.95 -> 0.47, two levels with 512 pairs on 65536 slots 1.57 -> 0.72, 36-wide with 777 pairs on 5001 slots 0.38
+// -> 0.16, 64-wide with 8192 pairs on 262144 slots 386 -> 119.
+// A lane adds its channel terms cw (d d) in float over a pass's slots, then into a double, as the other population kernels.
+// Values past the 16-bit range make NaN outputs (split_mlp.hpp), so a wave whose sum is a NaN evaluates its slots again in
+// 32 bits as k_pop_mfma does; with --clamp, where a NaN output becomes 0, the output pre-activations are tested.
+template <class S>
+constexpr int split_u() { return valu_out<S>() ? 4 : 2; }
+
 template <class S, bool Clamp, int From, bool UnitCw>
-__global__ void __launch_bounds__(64 * kPopWaves) __attribute__((amdgpu_waves_per_eu(pop_occupancy<S>()))) k_pop_pair(DevModel m, PopSource src, int M, int Mcap,
-                                                            int chunk, int chunks, const float* __restrict__ feat,
-                                                            const float* __restrict__ btgt, const float* __restrict__ lay1,
+__global__ void __launch_bounds__(64 * kPopWaves) __attribute__((amdgpu_waves_per_eu(split_occupancy<S>()))) k_pop_split(DevModel m, PopSource src, int M, int Mcap,
+                                                            int chunk, int chunks, SplitIn in, const float* __restrict__ feat,
                                                             double* __restrict__ part) {
     using Q = MfmaShape<S>;
-    static_assert(From != kSets && pop_pair_ok<S>(), "an ES step of a shape the pair kernel takes");
-    constexpr int H = Q::kH, NIN = Q::kIn, NO = Q::kNout, RO = out_regs<S>(), NB = pair_bias_rows<S>(), PP = pair_p_pad<S>();
-    constexpr int kPout = H * NIN + H + (Q::kNL - 1) * (H * H + H);   // the first output-layer parameter
-    __shared__ double red[2][kPopWaves];
-    __shared__ __attribute__((aligned(16))) float wpm_s[2 * PP];          // the + member's parameters, then the - member's
-    __shared__ __attribute__((aligned(16))) float bias_s[2 * NB * 16];    // [member][row][4 g + r]
-    __shared__ __attribute__((aligned(16))) float cw_s[16];               // the channel weight of register r of group g
-    // at most 4 outputs: the output layer on the VALU (valu_out_g's sums and reduce-scatter), its weights from LDS:
-    // [member][lane group][bias, then k-step 0 .. kKsH - 1][output 0 .. 3], and each wave's two reduce-scatter tiles
+    using P = SplitShape<S>;
+    static_assert(From != kSets && P::kOk, "an ES step of a shape the split kernel takes");
+    constexpr int NIN = Q::kIn, NO = Q::kNout, RO = out_regs<S>(), U = split_u<S>();
     constexpr bool kVOut = valu_out<S>();
-    constexpr int kWo = kVOut ? 2 * 4 * (Q::kKsH + 1) * 4 : 4;
-    __shared__ __attribute__((aligned(16))) float wo_s[kWo];
-    __shared__ __attribute__((aligned(16))) float vo_s[kVOut ? kPopWaves * 2 * kVoTile : 4];
+    constexpr int TS = split_targets(NO), FB = 4 * split_inputs(NIN);   // floats of targets and bytes of features per slot
+    constexpr int NT = kVOut ? NO : RO;                                  // target values a lane takes per read
+    constexpr int TT = kVOut ? 1 : U;                                    // reads per pass
+    __shared__ double red[kPopWaves];
+    __shared__ unsigned par_s[2 * SplitLds<S>::kWords];                  // the + member's parameters, then the - member's
+    __shared__ __attribute__((aligned(16))) float vo_s[kVOut ? kPopWaves * kVoTile : 4];   // the 32-bit evaluation's output sums
     const int lane = tid_x() & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid_x() >> 6);
-    const int pair = bid_x(), ch = bid_y();
+    const int pair = bid_x(), ch = bid_y(), sgn = wave & 1, half = wave >> 1;
     const int i16 = lane & 15, g = lane >> 4;
     const int s0 = ch * chunk, s1 = min(M, s0 + chunk);
-    const int tiles = (s1 - s0 + 15) >> 4;
-    const int mine = (tiles - wave + kPopWaves - 1) / kPopWaves;   // this wave's tiles: wave + 4 j, j < mine
-    // lane byte offsets: feature rows 4 ks + g, first-layer rows 16 ot + 4 g + r, target rows out_at(g, r) (a valid row
-    // for padding: its channel weight is zero)
-    // (register r of lane group g holds output RO g + r, so row r of a group is its first row + r)
-    static_assert(out_at<S>(3, RO - 1) == 3 * RO + RO - 1 || out_at<S>(3, RO - 1) < 0, "packed output rows");
-    const uint32_t fo = 4u * ((uint32_t)g * (uint32_t)Mcap + (uint32_t)i16);
-    const uint32_t uo = 4u * (4u * (uint32_t)g * (uint32_t)Mcap + (uint32_t)i16);
-    const uint32_t to = 4u * ((uint32_t)min(RO * g, NO - RO) * (uint32_t)Mcap + (uint32_t)i16);
-    const __amdgpu_buffer_rsrc_t rf = buffer_of(feat, 4u * ((uint32_t)minibatch_rows(NIN) * (uint32_t)Mcap + (uint32_t)kMinibatchSlack));
-    const __amdgpu_buffer_rsrc_t rt = buffer_of(btgt, 4u * ((uint32_t)NO * (uint32_t)Mcap + (uint32_t)kMinibatchSlack));
-    const __amdgpu_buffer_rsrc_t ru = buffer_of(lay1, 4u * ((uint32_t)H * (uint32_t)Mcap + (uint32_t)kMinibatchSlack));
-    // a tile's inputs, loaded one pass ahead; its targets at the start of its own pass (used at the end)
-    struct TileIn { float b1[Q::kKs1]; float u[Q::kHt][4]; };
-    auto tile_off = [&](int j) {   // tile wave + 4 j (uniform)
-        return (uint32_t)__builtin_amdgcn_readfirstlane((int)(4u * (uint32_t)(s0 + 16 * (wave + kPopWaves * j))));
+    constexpr int PS = 16 * U;                                           // slots per pass
+    const int mine = ((s1 - s0 + PS - 1) / PS - half + 1) >> 1;          // this wave's passes: 2 q + half, q < mine
+    const uint32_t slots = (uint32_t)Mcap + (uint32_t)kSplitSlack;
+    const __amdgpu_buffer_rsrc_t rf = buffer_of((const float*)in.feat, slots * (uint32_t)FB), rt = buffer_of(in.tgt, slots * 4u * TS);
+    const uint32_t fo = (uint32_t)(FB * i16 + 16 * (P::kS1 == 1 ? (g & 1) : g));
+    const uint32_t to = kVOut ? 4u * (uint32_t)(TS * lane) : 4u * (uint32_t)(TS * i16 + RO * g);
+    struct In { h8v f[U]; float t[TT][NT]; };
+    auto load = [&](In& n, int q) {
+        const uint32_t s = (uint32_t)__builtin_amdgcn_readfirstlane(s0 + PS * (2 * q + half));
+#pragma unroll
+        for (int u = 0; u < U; u++) n.f[u] = __builtin_bit_cast(h8v, __builtin_amdgcn_raw_buffer_load_b128(rf, (int)fo, (int)((s + 16u * u) * FB), 0));
+#pragma unroll
+        for (int u = 0; u < TT; u++)
+#pragma unroll
+            for (int r = 0; r < NT; r++) n.t[u][r] = buffer_f32(rt, to + 4u * r, (s + 16u * u) * (4u * TS));
     };
-    auto load = [&](TileIn& in, int j) {
-        const uint32_t so = tile_off(j);
-#pragma unroll
-        for (int ks = 0; ks < Q::kKs1; ks++) in.b1[ks] = buffer_f32(rf, fo, so + 16u * (uint32_t)ks * (uint32_t)Mcap);
-#pragma unroll
-        for (int ot = 0; ot < Q::kHt; ot++)
-#pragma unroll
-            for (int r = 0; r < 4; r++) in.u[ot][r] = buffer_f32(ru, uo, so + 4u * (uint32_t)(16 * ot + r) * (uint32_t)Mcap);
-    };
-    TileIn in0, in1;
+    In in0, in1;
     load(in0, 0);
-    pair_stage<S, Clamp, From>(m, src, pair, ch, wpm_s, bias_s, cw_s);
+    const SplitScale sc = split_scale(in.scales);
+    split_stage<S, From>(src, split_factors(sc, m.fold_c, Clamp ? 1.0 : kNegLog2eD), pair, ch, par_s);
     __syncthreads();
-    if constexpr (kVOut) {   // the output layer's table from the staged (scaled) parameters
-        for (int i = tid_x(); i < kWo; i += 64 * kPopWaves) {
-            const int c = i & 3, ks = (i >> 2) % (Q::kKsH + 1) - 1, gg = (i >> 2) / (Q::kKsH + 1) % 4, mem = i / (4 * (Q::kKsH + 1) * 4);
-            const float* wm = wpm_s + mem * PP + kPout;
-            float v = 0.0f;
-            if (c < NO) {
-                if (ks < 0) v = gg == 0 ? wm[NO * H + c] : 0.0f;   // the bias, in lane group 0 (valu_out_g's W.bo)
-                else if (hidden_input<Q>(ks, gg) < H) v = wm[c * H + hidden_input<Q>(ks, gg)];
-            }
-            wo_s[i] = v;
-        }
-        __syncthreads();
+    const unsigned* const mine_s = par_s + sgn * SplitLds<S>::kWords;
+    SplitWeights<S> W;
+    split_load<S>(W, mine_s, lane);
+    const float ak = in_vgpr(act_k_of<kActFold>(m)), neg = in_vgpr(-1.0f), inv = in_vgpr(sc.inv);
+    // the channel weight of each of this lane's output registers (0 past the last output)
+    float cw[NT];
+#pragma unroll
+    for (int r = 0; r < NT; r++) {
+        cw[r] = 0.0f;
+#pragma unroll
+        for (int c = 0; c < NO; c++)
+            if ((kVOut ? r : out_at<S>(g, r)) == c) cw[r] = m.cw[c];
     }
-    MfmaWeights<S> Wp, Wm;   // the A operands of both members (their bias fields unused)
-    mfma_load<S>(Wp, wpm_s, lane);
-    mfma_load<S>(Wm, wpm_s + PP, lane);
-    const float ak = act_k_of<kActFold>(m);
-    auto bias = [&](int mem, int row) { return *reinterpret_cast<const f4v*>(bias_s + (mem * NB + row) * 16 + 4 * g); };
-    // valu_out_g of member mem with its weights from wo_s: output g of pixel i16 in lane (g, i16), zero past nout
-    auto vout = [&](int mem, const float (&x)[Q::kKsH]) {
-        const float* wg = wo_s + (mem * 4 + g) * (Q::kKsH + 1) * 4;
-        float* t = vo_s + (wave * 2 + mem) * kVoTile;
-        f4v p = *reinterpret_cast<const f4v*>(wg);
+    constexpr bool kUnit = UnitCw && (kVOut || NO == 4 * RO);   // (padding outputs need their zero weight)
+    double e = 0.0;
+    bool bad = false;   // --clamp: an output pre-activation was a NaN
+    auto terms = [&](const f4v& o, const float (&t)[NT], float sum) {
 #pragma unroll
-        for (int ks = 0; ks < Q::kKsH; ks++) {
-            const f4v wv = *reinterpret_cast<const f4v*>(wg + 4 * (ks + 1));
-#pragma unroll
-            for (int c = 0; c < NO; c++) p[c] = __builtin_fmaf(wv[c], x[ks], p[c]);
+        for (int r = 0; r < NT; r++) {
+            const float s = o[r] * inv;
+            if constexpr (Clamp) bad |= !not_nan_bits(s);
+            const float d = out_of<S>(s, Clamp) - t[r];
+            sum = __builtin_fmaf(kUnit ? d : __fmul_rn(cw[r], d), d, sum);
         }
-#pragma unroll
-        for (int c = 0; c < 4; c++) t[i16 * kOwnRow + 4 * c + g] = p[c];
-        wave_lds_fence();
-        const f4v v = *reinterpret_cast<const f4v*>(t + i16 * kOwnRow + 4 * g);
-        wave_lds_fence();
-        return (v[0] + v[2]) + (v[1] + v[3]);
+        return sum;
     };
-    double ep = 0.0, em = 0.0;
-    float fp = 0.0f, fm = 0.0f;   // the float sums of this lane's terms over the passes since the last double add
-    auto pass = [&](TileIn& c, TileIn& n, int j) {
-        j = __builtin_amdgcn_readfirstlane(j);
-        float tt[RO];
-        {
-            const uint32_t so = tile_off(j);
-#pragma unroll
-            for (int r = 0; r < RO; r++) tt[r] = buffer_f32(rt, to, so + 4u * (uint32_t)r * (uint32_t)Mcap);
-        }
-        load(n, j + 1 < mine ? j + 1 : j);
-        // first layer: the + member's chain, the - member as 2 u - h+
-        f4v hp[Q::kHt], hm[Q::kHt];
-#pragma unroll
-        for (int ot = 0; ot < Q::kHt; ot++) hp[ot] = bias(0, ot);
-#pragma unroll
-        for (int ks = 0; ks < Q::kKs1; ks++)
-#pragma unroll
-            for (int ot = 0; ot < Q::kHt; ot++) hp[ot] = mfma4(Wp.a1[ot][ks], c.b1[ks], hp[ot]);
-#pragma unroll
-        for (int ot = 0; ot < Q::kHt; ot++)
-#pragma unroll
-            for (int r = 0; r < 4; r++) hm[ot][r] = __builtin_fmaf(2.0f, c.u[ot][r], -hp[ot][r]);
-        float xp[Q::kKsH], xm[Q::kKsH];
-#pragma unroll
-        for (int ot = 0; ot < Q::kHt; ot++)
-#pragma unroll
-            for (int r = 0; r < 4; r++) { xp[4 * ot + r] = act<kActFold>(hp[ot][r], ak); xm[4 * ot + r] = act<kActFold>(hm[ot][r], ak); }
-#pragma unroll
-        for (int l = 0; l < Q::kNL - 1; l++) {
-            f4v ap[Q::kHt], am[Q::kHt];
-#pragma unroll
-            for (int ot = 0; ot < Q::kHt; ot++) { ap[ot] = bias(0, Q::kHt * (1 + l) + ot); am[ot] = bias(1, Q::kHt * (1 + l) + ot); }
-#pragma unroll
-            for (int ks = 0; ks < Q::kKsH; ks++)
-#pragma unroll
-                for (int ot = 0; ot < Q::kHt; ot++) {
-                    ap[ot] = mfma4(Wp.ah[l][ot][ks], xp[ks], ap[ot]);
-                    am[ot] = mfma4(Wm.ah[l][ot][ks], xm[ks], am[ot]);
-                }
-#pragma unroll
-            for (int ot = 0; ot < Q::kHt; ot++)
-#pragma unroll
-                for (int r = 0; r < 4; r++) { xp[4 * ot + r] = act<kActFold>(ap[ot][r], ak); xm[4 * ot + r] = act<kActFold>(am[ot][r], ak); }
-        }
-        f4v op, om;
+    auto pass = [&](In& c, In& n, int q) {
+        q = __builtin_amdgcn_readfirstlane(q);
+        load(n, q + 1 < mine ? q + 1 : q);
+        const int s = s0 + PS * (2 * q + half);   // the pass's first slot
         if constexpr (kVOut) {
-            op[0] = vout(0, xp);
-            om[0] = vout(1, xm);
-        } else {
-            op = bias(0, NB - 1);
-            om = bias(1, NB - 1);
+            f4v o = W.co;
 #pragma unroll
-            for (int ks = 0; ks < Q::kKsH; ks++) {
-                op = mfma4(Wp.ao[ks], xp[ks], op);
-                om = mfma4(Wm.ao[ks], xm[ks], om);
+            for (int u = 0; u < U; u++) {
+                h8v b[P::kB];
+                split_hidden<S>(W, c.f[u], ak, neg, b);
+                o = split_dot<S>(W.ao[u], b, o);
+            }
+            const float ts = terms(o, c.t[0], 0.0f);
+            if (s + lane < s1) e += (double)ts;
+        } else {
+            f4v o[U];
+#pragma unroll
+            for (int u = 0; u < U; u++) {
+                h8v b[P::kB];
+                split_hidden<S>(W, c.f[u], ak, neg, b);
+                o[u] = split_dot<S>(W.ao[0], b, W.co);
+            }
+            if (s + PS <= s1) {   // every slot inside the chunk (uniform)
+                float ts = 0.0f;
+#pragma unroll
+                for (int u = 0; u < U; u++) ts = terms(o[u], c.t[u], ts);
+                e += (double)ts;
+            } else {
+#pragma unroll
+                for (int u = 0; u < U; u++) {
+                    const float ts = terms(o[u], c.t[u], 0.0f);
+                    if (s + 16 * u + i16 < s1) e += (double)ts;
+                }
             }
         }
-        // each member's channel terms cw (d d) (a multiply, unless every cw is 1, and a fused multiply-add each), summed
-        // in float over this lane's outputs of the tile and over the loop's two passes, then into the member's double
-        float tp = 0.0f, tm = 0.0f;
-        const f4v cw = *reinterpret_cast<const f4v*>(cw_s + 4 * g);
-        constexpr bool kUnit = UnitCw && NO == 4 * RO;   // (with padding rows their zero weight is still needed)
-#pragma unroll
-        for (int r = 0; r < RO; r++) {
-            const float dp = out_of<S>(op[r], Clamp) - tt[r], dm = out_of<S>(om[r], Clamp) - tt[r];
-            tp = __builtin_fmaf(kUnit ? dp : __fmul_rn(cw[r], dp), dp, tp);
-            tm = __builtin_fmaf(kUnit ? dm : __fmul_rn(cw[r], dm), dm, tm);
-        }
-        if (s0 + 16 * (wave + kPopWaves * j) + i16 < s1) { fp += tp; fm += tm; }
     };
-    for (int j = 0; j < mine; j += 2) {
-        pass(in0, in1, j);
-        if (j + 1 < mine) pass(in1, in0, j + 1);
-        ep += (double)fp; em += (double)fm;
-        fp = 0.0f; fm = 0.0f;
+    for (int q = 0; q < mine; q += 2) {
+        pass(in0, in1, q);
+        if (q + 1 < mine) pass(in1, in0, q + 1);
     }
-    ep = wave_sum(ep);
-    em = wave_sum(em);
-    if (lane == 0) { red[0][wave] = ep; red[1][wave] = em; }
+    if (__builtin_amdgcn_ballot_w64(bad || !not_nan_bits_d(e)) != 0) {
+        // 32 bits: the wave's slots again, a 16-slot tile at a time, from the minibatch's 32-bit feature rows
+        e = 0.0;
+        MfmaWeights<S> F;
+        mfma_load_from<S>(F, SplitParam32<S>{ mine_s, sc }, lane);
+        const __amdgpu_buffer_rsrc_t r32 = buffer_of(feat, 4u * ((uint32_t)minibatch_rows(NIN) * (uint32_t)Mcap + (uint32_t)kMinibatchSlack));
+        for (int q = 0; q < mine; q++)
+            for (int u = 0; u < U; u++) {
+                const int st = s0 + PS * (2 * q + half) + 16 * u;
+                if (st >= s1) break;
+                float b1[1][Q::kKs1], x[1][Q::kKsH];
+#pragma unroll
+                for (int ks = 0; ks < Q::kKs1; ks++)
+                    b1[0][ks] = buffer_f32(r32, 4u * ((uint32_t)(4 * ks + g) * (uint32_t)Mcap + (uint32_t)i16), 4u * (uint32_t)st);
+                mfma_hidden<S, 1, kActFold>(F, b1, ak, x);
+                float ts = 0.0f;
+                if constexpr (kVOut) {
+                    const float d = out_of<S>(valu_out_g<S>(F, x[0], vo_s + wave * kVoTile, g, i16), Clamp) -
+                                    buffer_f32(rt, 4u * (uint32_t)(TS * i16 + min(g, NO - 1)), (uint32_t)st * (4u * TS));
+                    ts = g < NO ? __fmul_rn(__fmul_rn(m.cw[min(g, NO - 1)], d), d) : 0.0f;
+                } else {
+                    f4v o[1];
+                    mfma_output<S, 1>(F, x, o);
+#pragma unroll
+                    for (int r = 0; r < RO; r++) {
+                        const float d = out_of<S>(o[0][r], Clamp) - buffer_f32(rt, to + 4u * r, (uint32_t)st * (4u * TS));
+                        ts = __builtin_fmaf(__fmul_rn(cw[r], d), d, ts);
+                    }
+                }
+                if (st + i16 < s1) e += (double)ts;
+            }
+    }
+    e = wave_sum(e);
+    if (lane == 0) red[wave] = e;
     __syncthreads();
     if (tid_x() == 0) {
-        part[(size_t)(2 * pair) * chunks + ch] = (red[0][0] + red[0][1]) + (red[0][2] + red[0][3]);
-        part[(size_t)(2 * pair + 1) * chunks + ch] = (red[1][0] + red[1][1]) + (red[1][2] + red[1][3]);
-    }
-}
-
-// ---- The pair population kernel of the pixel-per-lane shapes (at most 4 outputs, one 16-unit hidden tile: rgb256's
-// 6-16-16-3). As k_pop_pair, both members of the pair in each wave and the - member's first layer as 2 u - h+; a pass
-// takes two of the wave's tiles, so four chains run after the first layer. The output layer's exchange (mfma_out_own)
-// takes the + member's two tiles as its tiles 0 and 1 and the - member's as 2 and 3, and each lane's 4x4x1 A operands
-// are the output weights of the member its lane group holds: lane (g, j) ends with the outputs of pixel j of the pass's
-// tile g & 1 for member g >> 1, and adds that pixel's channel terms to its member's sum.
-template <class S, bool = MfmaShape<S>::kOk>
-struct PopPairOwnOk { static constexpr bool value = false; };
-template <class S>
-struct PopPairOwnOk<S, true> { static constexpr bool value = pop_own<S>() && MfmaShape<S>::kH == 16; };
-template <class S>
-constexpr bool pop_pair_own_ok() { return PopPairOwnOk<S>::value; }
-
-template <class S, bool Clamp, int From, bool UnitCw>
-__global__ void __launch_bounds__(64 * kPopWaves) __attribute__((amdgpu_waves_per_eu(pop_occupancy<S>()))) k_pop_pair_own(
-        DevModel m, PopSource src, int M, int Mcap, int chunk, int chunks, const float* __restrict__ feat, const float* __restrict__ btgt,
-        const float* __restrict__ lay1, double* __restrict__ part) {
-    using Q = MfmaShape<S>;
-    static_assert(From != kSets && pop_pair_own_ok<S>() && Q::kHt == 1, "an ES step of a pixel-per-lane shape");
-    constexpr int H = Q::kH, NIN = Q::kIn, NO = Q::kNout, NB = pair_bias_rows<S>(), PP = pair_p_pad<S>();
-    __shared__ double red[2][kPopWaves];
-    __shared__ __attribute__((aligned(16))) float wpm_s[2 * PP];          // the + member's parameters, then the - member's
-    __shared__ __attribute__((aligned(16))) float bias_s[2 * NB * 16];    // [member][row][4 g + r]
-    __shared__ __attribute__((aligned(16))) float cw_s[16];
-    __shared__ __attribute__((aligned(16))) float own_s[kPopWaves * kOwnWave];   // each wave's output-layer exchange
-    const int lane = tid_x() & 63;
-    const int wave = __builtin_amdgcn_readfirstlane(tid_x() >> 6);
-    const int pair = bid_x(), ch = bid_y();
-    const int i16 = lane & 15, g = lane >> 4;
-    const int s0 = ch * chunk, s1 = min(M, s0 + chunk);
-    const int tiles = (s1 - s0 + 15) >> 4;
-    const int mine = (tiles - wave + kPopWaves - 1) / kPopWaves;   // this wave's tiles: wave + 4 q, q < mine
-    // lane byte offsets: feature rows 4 ks + g, first-layer rows 4 g + r, and the targets of pixel i16 of the pass's tile
-    // g & 1 (64 slots after its tile 0)
-    const uint32_t fo = 4u * ((uint32_t)g * (uint32_t)Mcap + (uint32_t)i16);
-    const uint32_t uo = 4u * (4u * (uint32_t)g * (uint32_t)Mcap + (uint32_t)i16);
-    const uint32_t to = 4u * ((uint32_t)i16 + 64u * (uint32_t)(g & 1));
-    const __amdgpu_buffer_rsrc_t rf = buffer_of(feat, 4u * ((uint32_t)minibatch_rows(NIN) * (uint32_t)Mcap + (uint32_t)kMinibatchSlack));
-    const __amdgpu_buffer_rsrc_t rt = buffer_of(btgt, 4u * ((uint32_t)NO * (uint32_t)Mcap + (uint32_t)kMinibatchSlack));
-    const __amdgpu_buffer_rsrc_t ru = buffer_of(lay1, 4u * ((uint32_t)H * (uint32_t)Mcap + (uint32_t)kMinibatchSlack));
-    // the inputs of a pass's two tiles, loaded one pass ahead; the targets at the start of their own pass
-    struct TileIn { float b1[2][Q::kKs1]; float u[2][4]; };
-    auto tile_off = [&](int q) {   // tile wave + 4 q (uniform)
-        return (uint32_t)__builtin_amdgcn_readfirstlane((int)(4u * (uint32_t)(s0 + 16 * (wave + kPopWaves * q))));
-    };
-    auto load = [&](TileIn& in, int j) {   // tiles 2 j and 2 j + 1 (a tile past the wave's last reads its last)
-#pragma unroll
-        for (int v = 0; v < 2; v++) {
-            const uint32_t so = tile_off(min(2 * j + v, mine - 1));
-#pragma unroll
-            for (int ks = 0; ks < Q::kKs1; ks++) in.b1[v][ks] = buffer_f32(rf, fo, so + 16u * (uint32_t)ks * (uint32_t)Mcap);
-#pragma unroll
-            for (int r = 0; r < 4; r++) in.u[v][r] = buffer_f32(ru, uo, so + 4u * (uint32_t)r * (uint32_t)Mcap);
-        }
-    };
-    TileIn in0, in1;
-    if (mine > 0) load(in0, 0);
-    pair_stage<S, Clamp, From>(m, src, pair, ch, wpm_s, bias_s, cw_s);
-    __syncthreads();
-    MfmaWeights<S> Wp, Wm, Wo;   // the A operands of both members; the output layer of the member of this lane group
-    mfma_load<S>(Wp, wpm_s, lane);
-    mfma_load<S>(Wm, wpm_s + PP, lane);
-    mfma_load<S>(Wo, wpm_s + (g >> 1) * PP, lane);
-    const float ak = act_k_of<kActFold>(m);
-    auto bias = [&](int mem, int row) { return *reinterpret_cast<const f4v*>(bias_s + (mem * NB + row) * 16 + 4 * g); };
-    float cw[NO];
-#pragma unroll
-    for (int r = 0; r < NO; r++) cw[r] = m.cw[r];
-    double e = 0.0;   // this lane's member's sum
-    auto pass = [&](TileIn& c, TileIn& n, int j) {
-        j = __builtin_amdgcn_readfirstlane(j);
-        float tt[NO];
-        {
-            const uint32_t so = tile_off(2 * j);
-#pragma unroll
-            for (int r = 0; r < NO; r++) tt[r] = buffer_f32(rt, to, so + 4u * (uint32_t)r * (uint32_t)Mcap);
-        }
-        load(n, 2 * j + 2 < mine ? j + 1 : j);
-        float x[4][Q::kKsH];   // the last hidden layer: + member's tiles 0, 1, then the - member's
-#pragma unroll
-        for (int v = 0; v < 2; v++) {
-            f4v hp = bias(0, 0), hm;
-#pragma unroll
-            for (int ks = 0; ks < Q::kKs1; ks++) hp = mfma4(Wp.a1[0][ks], c.b1[v][ks], hp);
-#pragma unroll
-            for (int r = 0; r < 4; r++) hm[r] = __builtin_fmaf(2.0f, c.u[v][r], -hp[r]);
-#pragma unroll
-            for (int r = 0; r < 4; r++) { x[v][r] = act<kActFold>(hp[r], ak); x[2 + v][r] = act<kActFold>(hm[r], ak); }
-        }
-#pragma unroll
-        for (int l = 0; l < Q::kNL - 1; l++) {
-            f4v a[4];
-#pragma unroll
-            for (int t = 0; t < 4; t++) a[t] = bias(t >> 1, 1 + l);
-#pragma unroll
-            for (int ks = 0; ks < Q::kKsH; ks++)
-#pragma unroll
-                for (int t = 0; t < 4; t++) a[t] = mfma4(t < 2 ? Wp.ah[l][0][ks] : Wm.ah[l][0][ks], x[t][ks], a[t]);
-#pragma unroll
-            for (int t = 0; t < 4; t++)
-#pragma unroll
-                for (int r = 0; r < 4; r++) x[t][r] = act<kActFold>(a[t][r], ak);
-        }
-        const f4v o = mfma_out_own<S>(Wo, x, own_s + wave * kOwnWave, g, i16);
-        // the lane's pixel: its channel terms cw (d d) (a multiply, unless every cw is 1, and a fused multiply-add each)
-        float tsum = 0.0f;
-#pragma unroll
-        for (int r = 0; r < NO; r++) {
-            const float d = out_of<S>(o[r], Clamp) - tt[r];
-            tsum = __builtin_fmaf(UnitCw ? d : __fmul_rn(cw[r], d), d, tsum);
-        }
-        const int q = 2 * j + (g & 1);
-        if (q < mine && s0 + 16 * (wave + kPopWaves * q) + i16 < s1) e += (double)tsum;
-    };
-    for (int j = 0; 2 * j < mine; j += 2) {
-        pass(in0, in1, j);
-        if (2 * j + 2 < mine) pass(in1, in0, j + 1);
-    }
-    const double ep = wave_sum(g < 2 ? e : 0.0), em = wave_sum(g < 2 ? 0.0 : e);
-    if (lane == 0) { red[0][wave] = ep; red[1][wave] = em; }
-    __syncthreads();
-    if (tid_x() == 0) {
-        part[(size_t)(2 * pair) * chunks + ch] = (red[0][0] + red[0][1]) + (red[0][2] + red[0][3]);
-        part[(size_t)(2 * pair + 1) * chunks + ch] = (red[1][0] + red[1][1]) + (red[1][2] + red[1][3]);
+        part[(size_t)(2 * pair) * chunks + ch] = red[0] + red[2];
+        part[(size_t)(2 * pair + 1) * chunks + ch] = red[1] + red[3];
     }
 }
 

@@ -26,26 +26,55 @@ struct EpsJob {
     int first_block;
 };
 
-// The unperturbed first layer of every minibatch slot, for the population kernel that shares it between the members of
-// a pair (k_pop_pair): out[u][s] = fl(b_u fb) + sum_i fl(w_ui fb) f_i as one chain of fused multiply-adds in input order
-// (the matrix instructions' order), fb the folded activation's scale. w null: none.
-struct Lay1Job {
+// The minibatch slot by slot for the split population kernel (device_common.hpp, split_inputs), and the layers' power-of-two
+// scales (split_mlp.hpp), which block `block` finds: scales[l] brings layer l's largest possible member weight (|w| + 6
+// sigma, more than the draw reaches, times the layer's factor: fold for hidden layers, out for the output layer) below
+// 2^kSplitExp[l]. feat null: none.
+struct SplitJob {
+    uint4* feat;
+    float* tgt;
+    float* scales;
     const float* w;
-    float* out;
+    float sigma, fold, out;
+    int block;
 };
 
-// floats of the first layer's weights and biases (fixed shapes of one hidden width; 1 otherwise)
-template <class S, bool = S::kFixed && S::kUniform>
-struct FirstLayerSize { static constexpr int value = 1; };
-template <class S>
-struct FirstLayerSize<S, true> { static constexpr int value = S::kH * (S::kNin + 1); };
+// a power of two in 2^-30 .. 2^30 that brings v below 2^e (1 for zero, an infinity or a NaN)
+__device__ __forceinline__ float split_pow2(float v, int e) {
+    const int x = (int)((__float_as_uint(v) >> 23) & 255u);   // v < 2^(x - 126)
+    return x == 0 || x == 255 ? 1.0f : __uint_as_float((uint32_t)(127 + clampi(e + 126 - x, -30, 30)) << 23);
+}
+__device__ inline void split_scales(const DevModel& m, const SplitJob& sj) {
+    __shared__ float red[kTPB / 64];
+    float total = kSplitFeat;
+    if (threadIdx.x == 0) sj.scales[1] = 1.0f;   // (a single hidden layer has no second)
+    int p = 0, in = m.nin;
+    for (int l = 0; l <= m.nl; l++) {
+        const bool last = l == m.nl;
+        const int out = last ? m.nout : m.hidden[l];
+        float v = 0.0f;
+        for (int k = (int)threadIdx.x; k < out * in; k += kTPB) v = fmaxf(v, fabsf(sj.w[p + k]));
+        for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, 64));
+        if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
+        __syncthreads();
+        v = red[0];
+        for (int q = 1; q < kTPB / 64; q++) v = fmaxf(v, red[q]);
+        __syncthreads();
+        const float s = split_pow2((v + 6.0f * fabsf(sj.sigma)) * fabsf(last ? sj.out : sj.fold), kSplitExp[last ? 2 : l]);
+        total *= s;
+        if (threadIdx.x == 0) sj.scales[last ? 2 : l] = s;
+        p += out * in + out; in = out;
+    }
+    if (threadIdx.x == 0) sj.scales[3] = 1.0f / total;
+}
 
 // The minibatch (draw_batch with the counter draw): slot s -> pixel, its feature column
 // feat[.][s] and target column btgt[.][s] (structure of arrays, so the evaluation reads coalesced).
 template <class S>
 __global__ void __launch_bounds__(kTPB) k_batch(DevModel m, uint64_t head, int M, int Mcap, const float* __restrict__ zdec,
                                                const float* __restrict__ tgt, int* __restrict__ bidx,
-                                               float* __restrict__ feat, float* __restrict__ btgt, EpsJob ej, Lay1Job l1) {
+                                               float* __restrict__ feat, float* __restrict__ btgt, EpsJob ej, SplitJob sj) {
+    if (sj.feat && (int)blockIdx.x == sj.block) { split_scales(m, sj); return; }
     if ((int)blockIdx.x >= ej.first_block) {
         const long long t = (long long)(blockIdx.x - ej.first_block) * kTPB + threadIdx.x;
         if (t < (long long)ej.N * ej.P) {
@@ -53,16 +82,6 @@ __global__ void __launch_bounds__(kTPB) k_batch(DevModel m, uint64_t head, int M
             ej.eps[t] = gauss_at(ej.nt, noise_head(ej.seed, NS_MLP, ej.step, (uint32_t)i), (uint64_t)k);
         }
         return;
-    }
-    // the first layer's weights and biases times fb, once per block (the Lay1Job below reads them from LDS)
-    constexpr int kW1 = FirstLayerSize<S>::value;
-    __shared__ float w1_s[kW1];
-    if constexpr (S::kFixed && S::kUniform) {
-        if (l1.w) {   // uniform: the whole block stages, before any thread leaves
-            const float fb = 0.5f * (1.0f + m.leak);
-            for (int k = (int)threadIdx.x; k < kW1; k += kTPB) w1_s[k] = l1.w[k] * fb;
-            __syncthreads();
-        }
     }
     const int s = blockIdx.x * kTPB + threadIdx.x;
     if (s >= M) return;
@@ -78,19 +97,24 @@ __global__ void __launch_bounds__(kTPB) k_batch(DevModel m, uint64_t head, int M
         for (int i = 0; i < m.nin; i++) feat[(size_t)i * Mcap + s] = f[i];
     }
     const float* t = tgt + (size_t)idx * m.nout;
-    for (int c = 0; c < m.nout; c++) btgt[(size_t)c * Mcap + s] = t[c];
     if constexpr (S::kFixed && S::kUniform) {
-        if (l1.w) {
-            constexpr int H = S::kH, NIN = S::kNin;
+        if (sj.feat) {
+            constexpr int N = split_inputs(S::kNin), TS = split_targets(S::kNout);
+            union { _Float16 h[2 * N]; uint4 q[N / 4]; } v;
 #pragma unroll
-            for (int u = 0; u < H; u++) {
-                float a = w1_s[H * NIN + u];
-#pragma unroll
-                for (int i = 0; i < NIN; i++) a = __builtin_fmaf(w1_s[u * NIN + i], f[i], a);
-                l1.out[(size_t)u * Mcap + s] = a;
+            for (int i = 0; i < N; i++) {
+                const float x = i < S::kNin ? f[i < S::kNin ? i : 0] * kSplitFeat : 0.0f;
+                v.h[i] = (_Float16)x;
+                v.h[N + i] = (_Float16)(x - (float)v.h[i]);
             }
+#pragma unroll
+            for (int i = 0; i < N / 4; i++) sj.feat[(size_t)s * (N / 4) + i] = v.q[i];
+#pragma unroll
+            for (int c = 0; c < TS; c++) sj.tgt[(size_t)s * TS + c] = c < S::kNout ? t[c < S::kNout ? c : 0] : 0.0f;
+            return;
         }
     }
+    for (int c = 0; c < m.nout; c++) btgt[(size_t)c * Mcap + s] = t[c];
 }
 
 // The population evaluation: block (pair, chunk) evaluates both members of the pair on the

@@ -100,44 +100,59 @@ void launch_pop_eval(Impl& I, int pairs, int M, int chunk, int chunks) {
     launch_pop_matrix<kSets>(I, src, pairs, M, chunk, chunks);
 }
 
-// The pair-sharing population kernels (k_pop_pair, k_pop_pair_own) take the ES steps of the fixed shapes they support
-// (pop_pair_possible: the trainer then keeps a first-layer array of H x Mcap floats) whose chunks' first layers stay
-// in the L2 (pop_pair_step: H x chunk floats within 2 MiB of an XCD's 4 MiB; the blocks of one chunk run together,
-// so an XCD's working set is about one chunk's minibatch). NTC_HIP_POP_PAIR=0 keeps k_pop_mfma for every step.
+// The split population kernel takes every ES step that the matrix cores take, of the shapes it has an operand layout for
+// (split_pays). Against the 32-bit kernel on the MI355X: see k_pop_split. NTC_HIP_POP_PAIR=0 keeps k_pop_mfma for every step.
+bool pop_split_possible(const Impl& I) {
+    if (!pop_on_matrix_cores(I)) return false;
+    const char* env = getenv("NTC_HIP_POP_PAIR");
+    return !(env && env[0] == '0') && split_pays(I.dm.nin, I.dm.nl);
+}
+bool pop_split_step(const Impl& I) { return I.pop_split && pop_on_matrix_cores(I); }
+
+// ntc_trainer_on_matrix_cores' "pop_pair" and "pop_pair_own": the fixed shapes of one or two whole 16-unit hidden tiles
+// whose chunks' first layers take at most 2 MiB, and those of them with at most 4 outputs and one tile.
+template <class S, bool = MfmaShape<S>::kOk>
+struct PairShape { static constexpr bool kOk = false, kOwn = false; };
+template <class S>
+struct PairShape<S, true> {
+    using Q = MfmaShape<S>;
+    static constexpr bool kOk = Q::kHt <= 2 && Q::kH % 16 == 0, kOwn = kOk && pop_own<S>();
+};
 bool pop_pair_possible(const Impl& I) {
     if (I.jit || I.valu_only || !(I.dm.leak >= 0.0f && I.dm.leak <= 1.0f)) return false;
     const char* env = getenv("NTC_HIP_POP_PAIR");
     if (env && env[0] == '0') return false;
     bool ok = false;
-    dispatch_shape(I.dm, [&](auto s) { ok = pop_pair_ok<decltype(s)>() || pop_pair_own_ok<decltype(s)>(); });
+    dispatch_shape(I.dm, [&](auto s) { ok = PairShape<decltype(s)>::kOk; });
     return ok;
 }
-
 bool pop_pair_own_shape(const Impl& I) {
     bool own = false;
-    dispatch_shape(I.dm, [&](auto s) { own = pop_pair_own_ok<decltype(s)>(); });
+    dispatch_shape(I.dm, [&](auto s) { own = PairShape<decltype(s)>::kOwn; });
     return own;
 }
-
 bool pop_pair_step(const Impl& I, int chunk) {
     return I.pop_pair && pop_on_matrix_cores(I) && (size_t)I.d.hidden[0] * (size_t)chunk * sizeof(float) <= ((size_t)2 << 20);
 }
 
 template <int From>
-static void launch_pop_pair(Impl& I, const PopSource& src, int N, int M, int chunk, int chunks) {
+static void launch_pop_split(Impl& I, const PopSource& src, int N, int M, int chunk, int chunks) {
     const bool unit = unit_cw(I);
+    const SplitIn in{ (const u4v*)I.sfeat, I.stgt, I.sscale };
+    if (I.jit) {
+        jit_launch(k_pop_split<ShapeMaterial, false, From, false>, I, "k_pop_split",
+                   std::string(I.dm.clamp_out ? "true, " : "false, ") + std::to_string(From) + ", false", dim3(N, chunks), dim3(64 * kPopWaves), 0,
+                   I.dm, src, M, I.Mcap, chunk, chunks, in, (const float*)I.feat, I.part);
+        NTC_CHECK(hipGetLastError());
+        return;
+    }
     dispatch_shape(I.dm, [&](auto s) {
         using S = decltype(s);
-        if constexpr (pop_pair_ok<S>()) {
-            auto kern = I.dm.clamp_out ? (unit ? k_pop_pair<S, true, From, true> : k_pop_pair<S, true, From, false>)
-                                       : (unit ? k_pop_pair<S, false, From, true> : k_pop_pair<S, false, From, false>);
-            launch_timed(kern, I, dim3(N, chunks), dim3(64 * kPopWaves), 0, I.dm, src, M, I.Mcap, chunk, chunks, I.feat, I.btgt,
-                         (const float*)I.lay1, I.part);
-        } else if constexpr (pop_pair_own_ok<S>()) {
-            auto kern = I.dm.clamp_out ? (unit ? k_pop_pair_own<S, true, From, true> : k_pop_pair_own<S, true, From, false>)
-                                       : (unit ? k_pop_pair_own<S, false, From, true> : k_pop_pair_own<S, false, From, false>);
-            launch_timed(kern, I, dim3(N, chunks), dim3(64 * kPopWaves), 0, I.dm, src, M, I.Mcap, chunk, chunks, I.feat, I.btgt,
-                         (const float*)I.lay1, I.part);
+        if constexpr (SplitShape<S>::kOk) {
+            auto kern = I.dm.clamp_out ? k_pop_split<S, true, From, false>
+                                       : (unit ? k_pop_split<S, false, From, true> : k_pop_split<S, false, From, false>);
+            launch_timed(kern, I, dim3(N, chunks), dim3(64 * kPopWaves), 0, I.dm, src, M, I.Mcap, chunk, chunks, in, (const float*)I.feat,
+                         I.part);
         }
     });
     NTC_CHECK(hipGetLastError());
@@ -149,9 +164,9 @@ void launch_pop_eval_es(Impl& I, int it, float sigma, int N, int M, int chunk, i
     src.nt = I.noise; src.seed = I.d.seed; src.step = (uint32_t)it; src.sigma = sigma;
     src.w0 = I.w; src.eps = I.eps_mlp;
     ProfScope ps(I, "pop_eval", true);
-    if (pop_pair_step(I, chunk)) {   // the step's minibatch launch wrote the first layer
-        if (pop_reads_eps(chunks)) launch_pop_pair<kReadEps>(I, src, N, M, chunk, chunks);
-        else launch_pop_pair<kDraw>(I, src, N, M, chunk, chunks);
+    if (pop_split_step(I)) {
+        if (pop_reads_eps(chunks)) launch_pop_split<kReadEps>(I, src, N, M, chunk, chunks);
+        else launch_pop_split<kDraw>(I, src, N, M, chunk, chunks);
         return;
     }
     if (pop_reads_eps(chunks)) launch_pop_matrix<kReadEps>(I, src, N, M, chunk, chunks);   // drawn by the minibatch launch

@@ -85,10 +85,12 @@ struct ntc_cuda::Trainer::Impl {
     float *feat = nullptr, *btgt = nullptr;
     int* bidx = nullptr;
     int Mcap = 0;
-    // the minibatch's unperturbed first-layer pre-activations (H x Mcap + slack), for the population kernel that
-    // shares them between a pair's members (k_pop_pair; pop_pair: the model's shape takes it)
-    float* lay1 = nullptr;
-    bool pop_pair = false;
+    // the minibatch slot by slot, and the layer scales, for the split population kernel (k_pop_split; pop_split: the
+    // model's ES steps take it), in one allocation: Mcap + kSplitSlack slots of split_inputs(nin) pairs of 16-bit parts,
+    // the 4 scales, as many slots of split_targets(nout) floats
+    uint4* sfeat = nullptr;
+    float *stgt = nullptr, *sscale = nullptr;
+    bool pop_split = false, pop_pair = false;
     float* wsets = nullptr;
     size_t wsets_cap = 0;      // floats
     float* eps_mlp = nullptr;
@@ -212,12 +214,15 @@ std::vector<uint32_t> noise_fix_summary(const std::vector<uint32_t>& fix);
 // kernels_mlp.hip
 void launch_fill(Impl& I, float* p, size_t n, float v);
 // the minibatch of step it; eps_pairs > 0: the same launch draws the step's Gaussians of that many pairs (EpsJob)
-void launch_batch(Impl& I, int it, int M, int eps_pairs = 0, bool lay1 = false);
-// whether this model's shape takes the pair-sharing population kernel (k_pop_pair; the trainer then keeps the
-// minibatch's first layer, lay1), and whether an ES step with chunks of `chunk` slots does
+// split: slot by slot for k_pop_split in an ES step of that sigma, in place of btgt
+void launch_batch(Impl& I, int it, int M, int eps_pairs = 0, bool split = false, float sigma = 0.0f);
+// whether this model's ES steps take the split population kernel (k_pop_split; decided at init, the trainer then keeps
+// its arrays), and whether the next one does
+bool pop_split_possible(const Impl& I);
+bool pop_split_step(const Impl& I);
+// ntc_trainer_on_matrix_cores' "pop_pair" and "pop_pair_own"
 bool pop_pair_possible(const Impl& I);
 bool pop_pair_step(const Impl& I, int chunk);
-// whether that kernel is the pixel-per-lane shapes' k_pop_pair_own
 bool pop_pair_own_shape(const Impl& I);
 void launch_perturb(Impl& I, int it, float sigma, int N);
 // the Gaussians of one ES step (NS_MLP, it, pair, k) into eps_mlp, N x P

@@ -1,0 +1,87 @@
+"""The ES population on the 16-bit matrix instructions with two-part operands (k_pop_split), at the sizes and values where
+it can go wrong: minibatches around its 16-slot tiles and its 32- and 64-slot passes, every operand layout of a hidden
+layer (7 to 64 units, one and two hidden layers), and models whose values leave the 16-bit range."""
+import numpy as np
+import pytest
+
+from gpu_common import LAYOUTS, data, rel, say, trainer
+from neural_block_textures_amd.trainer import Layout
+
+pytestmark = pytest.mark.gpu
+
+# Outputs are within 2e-6 of the reference's (the bar of the decode; a 32-bit pre-activation of size up to 8 is itself
+# within 5e-7). A member's loss is the mean of squared differences d, so it moves by at most 2 sqrt(loss) 2e-6 + (2e-6)^2.
+DELTA = 2e-6
+
+
+def check(orc, lay, z, p, tgt, pairs, batch, sigma=0.02, seed=5):
+    tr = trainer(lay, z, p, tgt, max_pairs=pairs, max_batch=batch, seed=seed)
+    tr.mlp_step(3, sigma, 0.005, pairs, batch)
+    idx = tr.debug_last_batch()
+    lp, lm = tr.debug_last_losses()
+    _, _, lp_o, lm_o = orc.mlp_es_eval(lay, p, z, tgt, seed, 3, sigma, pairs, idx)
+    worst = 0.0
+    for got, want in ((lp, lp_o), (lm, lm_o)):
+        bound = 2 * np.sqrt(want) * DELTA + DELTA ** 2
+        worst = max(worst, float((np.abs(got - want) / bound).max()))
+    say("pairs", pairs, "batch", batch, "largest error over its bound", worst)
+    assert worst <= 1.0
+    tr.close()
+
+
+@pytest.mark.parametrize("name", ["rgb_16x2", "rgb_24x2", "two_level", "material", "material_clamp", "dct_plane", "large",
+                                  "chief1_36", "mat_qat_36", "image3_27", "dct_17", "dct_11", "run8x3", "jit_mfma_28",
+                                  "jit_own_13"])
+def test_split_population_edges(orc, name):
+    lay = LAYOUTS[name]
+    z, p, tgt = data(lay, 21)
+    say("split edges", name)
+    for pairs, batch in ((1, 1), (2, 15), (1, 16), (3, 17), (2, 33), (2, 63), (1, 64), (2, 65), (5, 257), (2, 1000), (40, 300)):
+        check(orc, lay, z, p, tgt, pairs, batch)
+
+
+@pytest.mark.parametrize("hidden,nout", [(16, 1), (48, 1), (24, 3)])
+def test_split_population_one_hidden_layer(orc, hidden, nout):
+    lay = Layout(40, 24, [(10, 6, 4, False)], [hidden], T=nout, leak=0.1)
+    z, p, tgt = data(lay, 22)
+    say("split one hidden layer", hidden, nout)
+    check(orc, lay, z, p, tgt, 3, 100)
+
+
+@pytest.mark.parametrize("name", ["rgb_16x2", "material", "material_clamp", "large", "chief1_36", "two_level"])
+@pytest.mark.parametrize("scale", [2.0 ** 14, 2.0 ** -14])
+def test_split_population_range(orc, name, scale):
+    """Latents whose hidden values pass 65504 (the kernel then evaluates its slots in 32 bits), and layers whose sizes are far
+    from one another: the first layer's weights and biases scaled, the output layer scaled back, so the outputs are those of
+    an ordinary model and the bound is the same."""
+    lay = LAYOUTS[name]
+    z, p, tgt = data(lay, 23)
+    nin, h = lay.nin, lay.hidden[0]
+    p = p.copy()
+    n1, n2 = h * nin + h, h * nin + h + h * h + h
+    p[:n1] *= np.float32(scale)
+    p[n1 + h * h:n2] *= np.float32(scale)
+    p[n2:n2 + lay.nout * h] *= np.float32(1.0 / scale)
+    say("split range", name, scale)
+    # sigma follows the smallest layer's scale
+    check(orc, lay, z, p, tgt, 3, 200, sigma=0.02 * min(scale, 1.0 / scale))
+    if scale > 1:   # large features in place of large weights: the layers' scales cannot take them
+        z2, p2 = z * np.float32(scale), data(lay, 23)[1].copy()
+        p2[h * nin:n1] *= np.float32(scale)
+        p2[n1 + h * h:n2] *= np.float32(scale)
+        p2[n2:n2 + lay.nout * h] /= np.float32(scale)
+        check(orc, lay, z2, p2, tgt, 3, 200, sigma=0.02 / scale)
+
+
+def test_split_population_infinite_bias(orc):
+    """an infinite output bias saturates its output (main.cpp:624): a finite loss, as the oracle's"""
+    lay = LAYOUTS["material"]
+    z, p, tgt = data(lay, 24)
+    p = p.copy()
+    p[-1] = np.inf
+    tr = trainer(lay, z, p, tgt, max_pairs=2, max_batch=100)
+    tr.mlp_step(1, 0.02, 0.005, 2, 100)
+    lp, lm = tr.debug_last_losses()
+    _, _, lp_o, lm_o = orc.mlp_es_eval(lay, p, z, tgt, 5, 1, 0.02, 2, tr.debug_last_batch())
+    assert np.isfinite(lp_o).all() and rel(lp, lp_o).max() < 1e-5 and rel(lm, lm_o).max() < 1e-5
+    tr.close()
