@@ -300,7 +300,8 @@ struct SplitIn {
 
 // Stages both members of an ES pair in LDS (SplitLds): w0 + sigma eps, then w0 - sigma eps (main.cpp:1852-1856), in two
 // parts with their factors. The Gaussians are drawn here (kDraw: the chunk-0 block writes them for the update) or read
-// (kReadEps).
+// (kReadEps). Central differences (kSets): pair j < P is w0 with weight j at w + h and w - h (h = sigma; the 32-bit sums,
+// main.cpp:1905), pair P two copies of w0.
 template <class S, int From>
 __device__ __forceinline__ void split_stage(const PopSource& src, const SplitFactors f, int pair, int ch, unsigned* __restrict__ lds) {
     using L = SplitLds<S>;
@@ -308,19 +309,22 @@ __device__ __forceinline__ void split_stage(const PopSource& src, const SplitFac
     const uint64_t head = noise_head(src.seed, NS_MLP, src.step, (uint32_t)pair);
     float* eg = src.eps + (size_t)pair * kP;
     for (int k = tid_x(); k < kP; k += 64 * kPopWaves) {
-        float e;
-        if constexpr (From == kDraw) {
+        const float w0 = src.w0[k];
+        float wp = w0, wm = w0, s = src.sigma, e = 0.0f;
+        if constexpr (From == kSets) {
+            if (k == pair) { wp = w0 + s; wm = w0 - s; }
+            s = 0.0f;
+        } else if constexpr (From == kDraw) {
             e = gauss_at(src.nt, head, (uint64_t)k);
             if (ch == 0) eg[k] = e;
         } else {
             e = eg[k];
         }
-        const float w0 = src.w0[k];
         const int l = L::layer(k), at = L::pos(k);
         const bool b = L::bias(k);
         const double fw = l == 0 ? f.w1 : (l == 1 ? f.w2 : f.w3), fb = l == 0 ? f.b1 : (l == 1 ? f.b2 : f.b3), ff = b ? fb : fw;
-        lds[at] = split_param(w0, src.sigma, e, ff, b);
-        lds[L::kWords + at] = split_param(w0, -src.sigma, e, ff, b);
+        lds[at] = split_param(wp, s, e, ff, b);
+        lds[L::kWords + at] = split_param(wm, -s, e, ff, b);
     }
 }
 
@@ -340,8 +344,9 @@ struct SplitParam32 {
     }
 };
 
-// ---- The ES population on the 16-bit matrix instructions with 32-bit operands in two parts (split_mlp.hpp), for the shapes
-// of at most 16 inputs and two hidden layers.
+// ---- The population on the 16-bit matrix instructions with 32-bit operands in two parts (split_mlp.hpp), for the shapes
+// of at most 16 inputs and two hidden layers: ES steps, and central differences (kSets), whose members it forms from the
+// weights themselves (no weight sets in memory).
 //
 // Block (pair, chunk) has four waves: wave w evaluates member 2 pair + (w & 1) on the passes 2 q + (w >> 1) of the chunk's
 // slots, 32 slots a pass (two 16-slot tiles) for the models with more than 4 outputs, 64 (four tiles) for the others, whose
@@ -367,7 +372,7 @@ __global__ void __launch_bounds__(64 * kPopWaves) __attribute__((amdgpu_waves_pe
                                                             double* __restrict__ part) {
     using Q = MfmaShape<S>;
     using P = SplitShape<S>;
-    static_assert(From != kSets && P::kOk, "an ES step of a shape the split kernel takes");
+    static_assert(P::kOk, "a shape the split kernel takes");
     constexpr int NIN = Q::kIn, NO = Q::kNout, RO = out_regs<S>(), U = split_u<S>();
     constexpr bool kVOut = valu_out<S>();
     constexpr int TS = split_targets(NO), FB = 4 * split_inputs(NIN);   // floats of targets and bytes of features per slot

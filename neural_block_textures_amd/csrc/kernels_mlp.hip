@@ -32,9 +32,8 @@ __global__ void __launch_bounds__(kTPB) k_perturb(NoiseFix nt, uint64_t seed, ui
 }
 
 // Weight sets of one central-difference step: set pair j < P has w_j + h and w_j - h (float-realized,
-// main.cpp:1905), pair P holds two copies of w for the unperturbed loss; hh[j] = wp - wm in double.
-__global__ void __launch_bounds__(kTPB) k_fd_sets(int P, float h, const float* __restrict__ w0, float* __restrict__ wsets,
-                                                 double* __restrict__ hh) {
+// main.cpp:1905), pair P holds two copies of w for the unperturbed loss.
+__global__ void __launch_bounds__(kTPB) k_fd_sets(int P, float h, const float* __restrict__ w0, float* __restrict__ wsets) {
     const long long t = (long long)blockIdx.x * kTPB + threadIdx.x;
     if (t >= (long long)(P + 1) * P) return;
     const int j = (int)(t / P), k = (int)(t - (long long)j * P);
@@ -43,7 +42,6 @@ __global__ void __launch_bounds__(kTPB) k_fd_sets(int P, float h, const float* _
     const float wp = w + h, wm = w - h;
     wsets[(size_t)(2 * j) * P + k] = hit ? wp : w;
     wsets[(size_t)(2 * j + 1) * P + k] = hit ? wm : w;
-    if (hit) hh[j] = (double)wp - (double)wm;
 }
 
 // ES update direction (main.cpp:1868-1873): g[k] = sum over pairs of ((float)dl_i * scale) * eps_ik, one
@@ -167,11 +165,13 @@ __global__ void __launch_bounds__(kTPB) k_es_grad_final(int P, int segs, const f
     adam_at(theta, m, v, (size_t)k, g, lr, c1, c2);
 }
 
-// Central differences: dl_j = L(w_j + h) - L(w_j - h), g_j = dl_j / hh_j; pair P gives L(w).
-__global__ void __launch_bounds__(kTPB) k_fd_finish(const double* __restrict__ part, int chunks, int P, double norm,
-                                                   const double* __restrict__ hh, double* __restrict__ dl,
-                                                   double* __restrict__ lsum, float* __restrict__ grad) {
-    const int j = blockIdx.x * kTPB + threadIdx.x;
+// Central differences: dl_j = L(w_j + h) - L(w_j - h), g_j = dl_j / hh_j with hh_j = (w_j + h) - (w_j - h) in double of the
+// 32-bit sums, then Adam on the weight; pair P gives L(w).
+__global__ void __launch_bounds__(64) k_fd_finish(const double* __restrict__ part, int chunks, int P, double norm, float h,
+                                                   double* __restrict__ dl, double* __restrict__ lsum, float* __restrict__ grad,
+                                                   float* __restrict__ theta, float* __restrict__ m, float* __restrict__ v, float lr,
+                                                   float c1, float c2) {
+    const int j = blockIdx.x * 64 + threadIdx.x;
     if (j > P) return;
     double lp = 0.0, lm = 0.0;
     for (int c = 0; c < chunks; c++) { lp += part[(size_t)(2 * j) * chunks + c]; lm += part[(size_t)(2 * j + 1) * chunks + c]; }
@@ -179,7 +179,10 @@ __global__ void __launch_bounds__(kTPB) k_fd_finish(const double* __restrict__ p
     if (j == P) { lsum[0] = lp; return; }
     const double d = lp - lm;
     dl[j] = d;
-    grad[j] = (float)(d / hh[j]);
+    const float w = theta[j], wp = w + h, wm = w - h;
+    const float g = (float)(d / ((double)wp - (double)wm));
+    grad[j] = g;
+    adam_at(theta, m, v, (size_t)j, g, lr, c1, c2);
 }
 
 // Adam (main.cpp:1799-1809): m = fma(b1, m, (1 - b1) g), v = fma(b2, v, ((1 - b2) g) g),
@@ -301,7 +304,7 @@ void launch_perturb(Impl& I, int it, float sigma, int N) {
 void launch_fd_sets(Impl& I, float h) {
     const size_t n = (size_t)(I.P + 1) * I.P;
     ProfScope ps(I, "fd_sets");
-    hipLaunchKernelGGL(k_fd_sets, dim3(blocks_for(n, kTPB)), dim3(kTPB), 0, I.stream, I.P, h, I.w, I.wsets, I.hh);
+    hipLaunchKernelGGL(k_fd_sets, dim3(blocks_for(n, kTPB)), dim3(kTPB), 0, I.stream, I.P, h, I.w, I.wsets);
     NTC_CHECK(hipGetLastError());
 }
 
@@ -339,9 +342,11 @@ void launch_es_update(Impl& I, int chunks, double norm, float sigma, int N, floa
     }
 }
 
-void launch_fd_finish(Impl& I, int chunks, double norm) {
-    hipLaunchKernelGGL(k_fd_finish, dim3(blocks_for(I.P + 1, kTPB)), dim3(kTPB), 0, I.stream, I.part, chunks, I.P, norm, I.hh,
-                       I.dl, I.lsum, I.wgrad);
+void launch_fd_finish(Impl& I, int chunks, double norm, float h, float lr, int t) {
+    const float c1 = 1.0f - powf(0.9f, (float)t), c2 = 1.0f - powf(0.999f, (float)t);
+    ProfScope ps(I, "adam");
+    hipLaunchKernelGGL(k_fd_finish, dim3(blocks_for(I.P + 1, 64)), dim3(64), 0, I.stream, I.part, chunks, I.P, norm, h,
+                       I.dl, I.lsum, I.wgrad, I.w, I.wm, I.wv, lr, c1, c2);
     NTC_CHECK(hipGetLastError());
 }
 

@@ -83,6 +83,9 @@ static void launch_pop_matrix(Impl& I, const PopSource& src, int pairs, int M, i
     NTC_CHECK(hipGetLastError());
 }
 
+template <int From>
+static void launch_pop_split(Impl& I, const PopSource& src, int N, int M, int chunk, int chunks);
+
 void launch_pop_eval(Impl& I, int pairs, int M, int chunk, int chunks) {
     ProfScope ps(I, "pop_eval", pop_on_matrix_cores(I));   // the matrix path is one launch
     if (!pop_on_matrix_cores(I)) {
@@ -100,7 +103,16 @@ void launch_pop_eval(Impl& I, int pairs, int M, int chunk, int chunks) {
     launch_pop_matrix<kSets>(I, src, pairs, M, chunk, chunks);
 }
 
-// The split population kernel takes every ES step that the matrix cores take, of the shapes it has an operand layout for
+// the central-difference population (P + 1 pairs) of a model on the split kernel, from the weights and h
+void launch_pop_eval_fd(Impl& I, float h, int M, int chunk, int chunks) {
+    check_pop_launch(I, I.P + 1, chunk, chunks);
+    PopSource src{};
+    src.w0 = I.w; src.sigma = h;
+    ProfScope ps(I, "pop_eval", true);
+    launch_pop_split<kSets>(I, src, I.P + 1, M, chunk, chunks);
+}
+
+// The split population kernel takes every step that the matrix cores take, of the shapes it has an operand layout for
 // (split_pays). Against the 32-bit kernel on the MI355X: see k_pop_split. NTC_HIP_POP_PAIR=0 keeps k_pop_mfma for every step.
 bool pop_split_possible(const Impl& I) {
     if (!pop_on_matrix_cores(I)) return false;

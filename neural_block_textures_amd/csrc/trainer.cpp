@@ -201,7 +201,7 @@ Trainer::~Trainer() {
         dev_free(I.z); dev_free(I.zq); dev_free(I.zgrad); dev_free(I.zm); dev_free(I.zv); dev_free(I.ztmp);
         dev_free(I.w); dev_free(I.wgrad); dev_free(I.wm); dev_free(I.wv);
         dev_free(I.tgt); dev_free(I.img); dev_free(I.feat); dev_free(I.btgt); dev_free(I.bidx); dev_free(I.sfeat);
-        dev_free(I.wsets); dev_free(I.eps_mlp); dev_free(I.gpart); dev_free(I.part); dev_free(I.dl); dev_free(I.lsum); dev_free(I.hh);
+        dev_free(I.wsets); dev_free(I.eps_mlp); dev_free(I.gpart); dev_free(I.part); dev_free(I.dl); dev_free(I.lsum);
         dev_free(I.eps_lat); dev_free(I.eps_ahead); dev_free(I.dpix); dev_free(I.ranges); dev_free(I.qat_grid); dev_free(I.qat_bits);
         dev_free(I.qes_dev); dev_free(I.qgrid);
         dev_free(I.zpost); dev_free(I.st_part); dev_free(I.st_keys); dev_free(I.st_hist); dev_free(I.st_dct); dev_free(I.st_sse);
@@ -371,7 +371,7 @@ bool Trainer::init(const ModelDesc& d, const float* z, const float* p, const flo
     dev_alloc(&I.gpart, I.gpart_cap);
     if (!pop_on_matrix_cores(I)) ensure_wsets(I, (size_t)2 * I.pairs_cap * I.P);   // the matrix-core ES step needs none
     ensure_part(I, (size_t)2 * (std::max(I.pairs_cap, I.P + 1) * 4 + 2048));
-    dev_alloc(&I.dl, (size_t)std::max(I.pairs_cap, I.P)); dev_alloc(&I.lsum, (size_t)I.pairs_cap); dev_alloc(&I.hh, (size_t)I.P);
+    dev_alloc(&I.dl, (size_t)std::max(I.pairs_cap, I.P)); dev_alloc(&I.lsum, (size_t)I.pairs_cap);
     if (d.qat > 0) {
         dev_alloc(&I.qat_grid, 9 * 257); dev_alloc(&I.qat_bits, MAX_CH);
         NTC_CHECK(hipMemcpy(I.qat_grid, d.qat_grid, sizeof(float) * 9 * 257, hipMemcpyHostToDevice));
@@ -547,14 +547,18 @@ void Trainer::mlp_step_fd(int it, float h, float lr, int M) {
         fprintf(stderr, "ntc_hip backend: FD step with %d pixels outside the buffers sized at init (%d)\n", M, I.Mcap);
         exit(1);
     }
-    launch_batch(I, it, M);
-    ensure_wsets(I, (size_t)2 * (I.P + 1) * I.P);
-    launch_fd_sets(I, h);
+    const bool split = pop_split_step(I);
+    launch_batch(I, it, M, 0, split, h);
     const int chunk = pop_chunk(I, I.P + 1, M), chunks = (M + chunk - 1) / chunk;
     ensure_part(I, (size_t)2 * (I.P + 1) * chunks);
-    launch_pop_eval(I, I.P + 1, M, chunk, chunks);
-    launch_fd_finish(I, chunks, 3.0 * (double)I.d.wsum * (double)M);
-    launch_adam(I, I.w, I.wgrad, I.wm, I.wv, I.P, lr, ++I.mlp_t);
+    if (split) {
+        launch_pop_eval_fd(I, h, M, chunk, chunks);
+    } else {
+        ensure_wsets(I, (size_t)2 * (I.P + 1) * I.P);
+        launch_fd_sets(I, h);
+        launch_pop_eval(I, I.P + 1, M, chunk, chunks);
+    }
+    launch_fd_finish(I, chunks, 3.0 * (double)I.d.wsum * (double)M, h, lr, ++I.mlp_t);
     I.last_N = I.P; I.last_fd = true; I.last_M = M; I.last_chunk = chunk;
 }
 

@@ -96,7 +96,7 @@ struct ntc_cuda::Trainer::Impl {
     float* eps_mlp = nullptr;
     float* gpart = nullptr;    // segment partials of the ES update: ceil(max_pairs / 128) x P
     size_t gpart_cap = 0;
-    double *part = nullptr, *dl = nullptr, *lsum = nullptr, *hh = nullptr;
+    double *part = nullptr, *dl = nullptr, *lsum = nullptr;
     size_t part_cap = 0;
     int pairs_cap = 0;
     float *eps_lat = nullptr, *dpix = nullptr;   // one group of pairs of a latent step: Kcap x nz, Kcap x W*H
@@ -240,9 +240,11 @@ void launch_pop_eval(Impl& I, int pairs, int M, int chunk, int chunks);
 // (launch_batch with eps_pairs = N), else each chunk-0 block draws its pair's and writes them to eps_mlp
 inline bool pop_reads_eps(int chunks) { return chunks >= 3; }
 void launch_pop_eval_es(Impl& I, int it, float sigma, int N, int M, int chunk, int chunks);
+void launch_pop_eval_fd(Impl& I, float h, int M, int chunk, int chunks);
 void launch_pop_eval_valu(Impl& I, int pairs, int M, int chunk, int chunks);
 void launch_es_update(Impl& I, int chunks, double norm, float sigma, int N, float lr, int t);
-void launch_fd_finish(Impl& I, int chunks, double norm);
+// the central differences' gradient and Adam step t
+void launch_fd_finish(Impl& I, int chunks, double norm, float h, float lr, int t);
 void launch_adam(Impl& I, float* theta, const float* g, float* m, float* v, size_t n, float lr, int t);
 void launch_decode(Impl& I, const float* z);
 void launch_debug_gauss(Impl& I, uint32_t stream, uint32_t step, uint32_t pair, uint64_t index0, size_t n, float* out);

@@ -85,3 +85,28 @@ def test_split_population_infinite_bias(orc):
     _, _, lp_o, lm_o = orc.mlp_es_eval(lay, p, z, tgt, 5, 1, 0.02, 2, tr.debug_last_batch())
     assert np.isfinite(lp_o).all() and rel(lp, lp_o).max() < 1e-5 and rel(lm, lm_o).max() < 1e-5
     tr.close()
+
+
+@pytest.mark.parametrize("name", ["rgb_16x2", "dct_11", "material", "chief1_36", "jit_mfma_28"])
+def test_split_central_differences_edges(orc, name):
+    """The central-difference population on the split kernel, which forms its members from the weights itself. A loss
+    difference carries the rounding of both losses: as in the full-size check, at most 1e-3 of the differences' RMS, or
+    where the minibatch is small (few roundings average out) twice the bound of one loss."""
+    lay = LAYOUTS[name]
+    z, p, tgt = data(lay, 25)
+    h = np.float32(1e-3)
+    for batch in (1, 17, 65, 1000):
+        tr = trainer(lay, z, p, tgt, max_pairs=4, max_batch=batch)
+        tr.mlp_step_fd(2, h, 0.005, batch)
+        dl = tr.debug_last_dl()
+        dl_o, hh, l0 = orc.mlp_fd_eval(lay, p, z, tgt, h, tr.debug_last_batch())
+        rms = np.sqrt((dl_o ** 2).mean())
+        worst = np.abs(dl - dl_o).max()
+        say("fd", name, "batch", batch, "largest error over the RMS", worst / rms)
+        assert worst <= max(1e-3 * rms, 2 * (2 * np.sqrt(l0) * DELTA / np.sqrt(batch) + DELTA ** 2))
+        g = tr.debug_last_wgrad()
+        assert np.array_equal(g, orc.fd_grad(dl, hh))          # the realized 32-bit steps
+        w, m, v = p.copy(), np.zeros_like(p), np.zeros_like(p)
+        orc.adam(w, g, m, v, 0.005, 1)
+        assert np.array_equal(tr.download_model()[1], w)
+        tr.close()
