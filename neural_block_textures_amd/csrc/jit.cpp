@@ -15,7 +15,7 @@
 #include <sstream>
 #include <vector>
 
-#include "mfma_mlp.hpp"
+#include "kern_decode.hpp"
 
 namespace ntc_hip {
 
@@ -81,6 +81,10 @@ std::vector<std::string> expressions(const std::string& shape, const DevModel& m
     std::vector<std::string> v;
     if (!pop) {
         for (const char* k : { "k_batch", "k_pop_eval", "k_decode", "k_lat_pair", "k_qat_search", "k_dct_probe" }) v.push_back(e(k, ""));
+        bool one = true;
+        for (int l = 1; l < m.nl; l++) one = one && m.hidden[l] == m.hidden[0];
+        if (one && decode_pays(m.nin, m.hidden[0], m.nl, m.nout))
+            for (int to : { 0, 1, 2 }) v.push_back(e("k_decode_mfma", std::to_string(to)));
         return v;
     }
     const std::string c = m.clamp_out ? "true" : "false";
@@ -209,7 +213,7 @@ bool jit_prepare(Impl& I, std::string& why) {
     const std::string shape = jit_shape_name(js);
     const std::string csrc = source_dir();
     std::string key_src;
-    for (const char* f : { "kern_pop.hpp", "kern_valu.hpp", "split_mlp.hpp", "mfma_mlp.hpp", "device_common.hpp", "noise_math.hpp" }) {
+    for (const char* f : { "kern_pop.hpp", "kern_decode.hpp", "kern_valu.hpp", "split_mlp.hpp", "mfma_mlp.hpp", "device_common.hpp", "noise_math.hpp" }) {
         std::string t;
         if (csrc.empty() || !read_file(csrc + "/" + f, t)) { why = "the kernel sources are not next to the library (" + csrc + ")"; return false; }
         key_src += t;
@@ -230,7 +234,7 @@ bool jit_prepare(Impl& I, std::string& why) {
         const auto exprs = expressions(shape, I.dm, pop != 0);
         std::string code;
         std::vector<std::string> lowered;
-        if (!build_program(csrc, arch, pop ? "kern_pop.hpp" : "kern_valu.hpp", exprs, pop != 0, key_src, code, lowered, why)) {
+        if (!build_program(csrc, arch, pop ? "kern_pop.hpp" : "kern_decode.hpp", exprs, pop != 0, key_src, code, lowered, why)) {
             delete set;
             return false;
         }
@@ -258,7 +262,7 @@ bool jit_compile_only(const DevModel& m, const std::string& arch, std::string& w
     for (int pop = 0; pop < (mfma ? 2 : 1); pop++) {
         std::string code;
         std::vector<std::string> lowered;
-        if (!build_program(csrc, arch, pop ? "kern_pop.hpp" : "kern_valu.hpp", expressions(shape, m, pop != 0), pop != 0, "", code, lowered,
+        if (!build_program(csrc, arch, pop ? "kern_pop.hpp" : "kern_decode.hpp", expressions(shape, m, pop != 0), pop != 0, "", code, lowered,
                            why, false))   // compiled every time, never cached
             return false;
         if (code.empty()) { why = "empty code object"; return false; }

@@ -3,7 +3,7 @@
 //
 // Reference semantics (main.cpp): MlpTrainer::draw_batch 1825-1833, MlpTrainer::step 1836-1876,
 // MlpTrainer::step_fd 1890-1920, Adam::step 1799-1809, Decoder::decode_full 1712-1718.
-#include "kern_valu.hpp"
+#include "kern_decode.hpp"
 #include "jit.hpp"
 #include "shapes.hpp"
 #include "trainer_impl.hpp"
@@ -211,7 +211,7 @@ void launch_copy_calibration(Impl& I, const float* src, float* dst, size_t n) {
 // A decode rounded to 8 bits as save_png writes it (lround of the [0, 1]-clamped value times 255).
 __global__ void __launch_bounds__(kTPB) k_pack_u8(const float* __restrict__ img, size_t n, uint8_t* __restrict__ out) {
     const size_t i = (size_t)blockIdx.x * kTPB + threadIdx.x;
-    if (i < n) out[i] = (uint8_t)(int)roundf(__fmul_rn(fminf(1.0f, fmaxf(0.0f, img[i])), 255.0f));
+    if (i < n) out[i] = (uint8_t)to_byte(img[i]);
 }
 
 // The printed error of a decode (mse_of, main.cpp:1764-1788): both images rounded to 8 bits as save_png
@@ -229,8 +229,7 @@ __global__ void __launch_bounds__(kTPB) k_u8_sse(const float* __restrict__ img, 
         for (int t = 0; t < T; t++)
             for (int c = 0; c < 3; c++) {
                 const float x = img[p * nout + 3 * t + c], y = tgt[p * nout + 3 * t + c];
-                const int xi = (int)roundf(__fmul_rn(fminf(1.0f, fmaxf(0.0f, x)), 255.0f));
-                const int yi = (int)roundf(__fmul_rn(fminf(1.0f, fmaxf(0.0f, y)), 255.0f));
+                const int xi = to_byte(x), yi = to_byte(y);
                 s[t] += (unsigned long long)((xi - yi) * (xi - yi));
             }
     }
@@ -357,8 +356,36 @@ void launch_adam(Impl& I, float* theta, const float* g, float* m, float* v, size
     NTC_CHECK(hipGetLastError());
 }
 
+// The matrix-core decode of the extent ew x eh into out, for the shapes it pays for (decode_pays; any leak): enough blocks to
+// fill the chip, each taking 256-pixel rounds until the extent ends. Returns the blocks launched, 0 where the VALU kernel
+// takes the model (trainers set to the VALU kernels among them).
+template <int To>
+static size_t launch_decode_mfma(Impl& I, const float* z, int ew, int eh, void* out) {
+    if (I.valu_only || I.dm.nl < 1) return 0;
+    const int H = I.dm.hidden[0];
+    for (int l = 1; l < I.dm.nl; l++) if (I.dm.hidden[l] != H) return 0;
+    if (!decode_pays(I.dm.nin, H, I.dm.nl, I.dm.nout)) return 0;
+    const size_t groups = ((size_t)ew * eh + kTPB - 1) / kTPB, fill = (size_t)I.cus * decode_waves(H);
+    const size_t rounds = (groups + fill - 1) / fill, blocks = (groups + rounds - 1) / rounds;
+    bool done = false;
+    if (I.jit) {
+        jit_launch(k_decode_mfma<ShapeMaterial, To>, I, "k_decode_mfma", std::to_string(To), dim3((unsigned)blocks), dim3(kTPB), 0, I.dm, I.w, z,
+                   I.tgt, ew, eh, out);
+        done = true;
+    } else dispatch_shape(I.dm, [&](auto s) {
+        using S = decltype(s);
+        if constexpr (DecodeOk<S>::value) {
+            hipLaunchKernelGGL((k_decode_mfma<S, To>), dim3((unsigned)blocks), dim3(kTPB), 0, I.stream, I.dm, I.w, z, I.tgt, ew, eh, out);
+            done = true;
+        }
+    });
+    NTC_CHECK(hipGetLastError());
+    return done ? blocks : 0;
+}
+
 void launch_decode(Impl& I, const float* z) {
     ProfScope ps(I, "decode");
+    if (launch_decode_mfma<kToFloat>(I, z, I.d.W, I.d.H, I.img)) return;
     if (I.jit) {
         jit_launch(k_decode<ShapeDefault>, I, "k_decode", "", dim3(blocks_for(I.npix, kTPB)), dim3(kTPB), 0, I.dm, I.w, z, I.img);
     } else dispatch_shape(I.dm, [&](auto s) {
@@ -380,13 +407,24 @@ void launch_debug_factors(Impl& I, uint32_t k0, size_t n, float* rad, float* cos
     NTC_CHECK(hipGetLastError());
 }
 
-void launch_u8_sse(Impl& I, int ew, int eh, unsigned long long* part) {
-    hipLaunchKernelGGL(k_u8_sse, dim3(blocks_for((size_t)ew * eh, kTPB)), dim3(kTPB), 0, I.stream, I.img, I.tgt, I.d.W, ew, eh, I.d.nout,
-                       part);
+size_t launch_decode_sse(Impl& I, const float* z, int ew, int eh, unsigned long long* part) {
+    {
+        ProfScope ps(I, "decode");
+        if (const size_t blocks = launch_decode_mfma<kToError>(I, z, ew, eh, part)) return blocks;
+    }
+    launch_decode(I, z);
+    const size_t blocks = blocks_for((size_t)ew * eh, kTPB);
+    hipLaunchKernelGGL(k_u8_sse, dim3((unsigned)blocks), dim3(kTPB), 0, I.stream, I.img, I.tgt, I.d.W, ew, eh, I.d.nout, part);
     NTC_CHECK(hipGetLastError());
+    return blocks;
 }
 
-void launch_pack_u8(Impl& I, uint8_t* out) {
+void launch_decode_u8(Impl& I, const float* z, uint8_t* out) {
+    {
+        ProfScope ps(I, "decode");
+        if (launch_decode_mfma<kToBytes>(I, z, I.d.W, I.d.H, out)) return;
+    }
+    launch_decode(I, z);
     ProfScope ps(I, "pack_u8");
     const size_t n = (size_t)I.npix * I.d.nout;
     hipLaunchKernelGGL(k_pack_u8, dim3(blocks_for(n, kTPB)), dim3(kTPB), 0, I.stream, I.img, n, out);

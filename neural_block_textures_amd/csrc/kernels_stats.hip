@@ -316,9 +316,8 @@ void print_stats_impl(Impl& I, int qbits, int ew, int eh, ntc_print_stats* out) 
     if (eh <= 0 || eh > I.d.H) eh = I.d.H;
     const size_t sblocks = ((size_t)ew * eh + 255) / 256;
     ensure(&I.st_sse, I.st_sse_cap, sblocks * 4);
-    launch_decode(I, I.zpost);
-    launch_u8_sse(I, ew, eh, I.st_sse);
-    std::vector<unsigned long long> sse(sblocks * 4);
+    const size_t written = launch_decode_sse(I, I.zpost, ew, eh, I.st_sse);
+    std::vector<unsigned long long> sse(written * 4);
     NTC_CHECK(hipMemcpyAsync(sse.data(), I.st_sse, sse.size() * sizeof(unsigned long long), hipMemcpyDeviceToHost, I.stream));
     NTC_CHECK(hipStreamSynchronize(I.stream));
     {
@@ -327,7 +326,7 @@ void print_stats_impl(Impl& I, int qbits, int ew, int eh, ntc_print_stats* out) 
         double ws = 0.0;
         for (int t = 0; t < T; t++) {
             unsigned long long s = 0;
-            for (size_t b = 0; b < sblocks; b++) s += sse[b * 4 + t];
+            for (size_t b = 0; b < written; b++) s += sse[b * 4 + t];
             o.q_tex_mse[t] = (double)s / (3.0 * np);
             ws += (double)I.d.cw[3 * t] * (double)s;
         }

@@ -72,7 +72,7 @@ void decode_error_noalloc_impl(Impl& I, const float* z_host, int ew, int eh, dou
     if (I.d.nout % 3 != 0) { fprintf(stderr, "ntc_hip backend: decode_error needs RGB textures (nout a multiple of 3)\n"); exit(1); }
     if (ew <= 0 || ew > I.d.W) ew = I.d.W;
     if (eh <= 0 || eh > I.d.H) eh = I.d.H;
-    const size_t npx = (size_t)ew * eh, blocks = (npx + 255) / 256;
+    const size_t npx = (size_t)ew * eh;
     if (npx > kNoallocMaxPixels) {
         fprintf(stderr, "ntc_hip backend: decode_error_noalloc evaluates at most %zu pixels (its static scratch); the extent "
                         "%d x %d has %zu (decode_error has no such limit)\n", kNoallocMaxPixels, ew, eh, npx);
@@ -85,10 +85,9 @@ void decode_error_noalloc_impl(Impl& I, const float* z_host, int ew, int eh, dou
         NTC_CHECK(hipMemcpyAsync(I.ztmp, z_host, I.nz * sizeof(float), hipMemcpyHostToDevice, I.stream));
         zsrc = I.ztmp;
     }
-    launch_decode(I, zsrc);
-    launch_u8_sse(I, ew, eh, sp);
+    const size_t written = launch_decode_sse(I, zsrc, ew, eh, sp);
     unsigned long long* tot = sp + kNoallocBlocks * 4;
-    hipLaunchKernelGGL(k_sse_totals, dim3(1), dim3(256), 0, I.stream, sp, blocks, tot);
+    hipLaunchKernelGGL(k_sse_totals, dim3(1), dim3(256), 0, I.stream, sp, written, tot);
     NTC_CHECK(hipGetLastError());
     unsigned long long h[4];
     NTC_CHECK(hipMemcpyAsync(h, tot, sizeof(h), hipMemcpyDeviceToHost, I.stream));

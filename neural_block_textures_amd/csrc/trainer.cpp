@@ -139,9 +139,8 @@ void decode_error_impl(Impl& I, const float* z_host, int ew, int eh, double* tex
         NTC_CHECK(hipMemcpyAsync(I.ztmp, z_host, I.nz * sizeof(float), hipMemcpyHostToDevice, I.stream));
         zsrc = I.ztmp;
     }
-    launch_decode(I, zsrc);
-    launch_u8_sse(I, ew, eh, part);
-    std::vector<unsigned long long> h(blocks * 4);
+    const size_t written = launch_decode_sse(I, zsrc, ew, eh, part);
+    std::vector<unsigned long long> h(written * 4);
     NTC_CHECK(hipMemcpyAsync(h.data(), part, h.size() * sizeof(unsigned long long), hipMemcpyDeviceToHost, I.stream));
     sync(I);
     NTC_CHECK(ntc_hip::ntc_free(part));
@@ -150,7 +149,7 @@ void decode_error_impl(Impl& I, const float* z_host, int ew, int eh, double* tex
     double ws = 0.0;
     for (int t = 0; t < T; t++) {
         unsigned long long sse = 0;
-        for (size_t b = 0; b < blocks; b++) sse += h[b * 4 + t];
+        for (size_t b = 0; b < written; b++) sse += h[b * 4 + t];
         if (tex_mse) tex_mse[t] = (double)sse / (3.0 * npix);
         ws += (double)I.d.cw[3 * t] * (double)sse;
     }
@@ -163,8 +162,7 @@ void decode_rgb8_impl(Impl& I, uint8_t* out) {
     const size_t n = (size_t)I.npix * I.d.nout;
     uint8_t* d = nullptr;
     NTC_CHECK(ntc_hip::ntc_malloc(&d, n));
-    launch_decode(I, I.zdec);
-    launch_pack_u8(I, d);
+    launch_decode_u8(I, I.zdec, d);
     NTC_CHECK(hipMemcpyAsync(out, d, n, hipMemcpyDeviceToHost, I.stream));
     sync(I);
     NTC_CHECK(ntc_hip::ntc_free(d));

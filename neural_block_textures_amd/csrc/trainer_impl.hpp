@@ -273,10 +273,11 @@ void launch_dct_snap(Impl& I, float pull = 0.0f);
 void launch_dct_recon(Impl& I);
 // the decoder sensitivity probe over the decode buffer: codes (and block gains, when gain != null) into device buffers
 void launch_dct_probe(Impl& I, uint8_t* code, float* gain);
-// per-block, per-texture 8-bit squared-error sums of the decode in img against the target (ceil(ew eh / 256) x 4)
-void launch_u8_sse(Impl& I, int ew, int eh, unsigned long long* part);
-// img rounded to 8 bits (save_png) into out (device, npix x nout)
-void launch_pack_u8(Impl& I, uint8_t* out);
+// the decode of z over the extent ew x eh: per-block, per-texture 8-bit squared-error sums against the target; returns the
+// blocks, at most ceil(ew eh / 256), 4 sums each (img may be written, or not)
+size_t launch_decode_sse(Impl& I, const float* z, int ew, int eh, unsigned long long* part);
+// the decode of z rounded to 8 bits (save_png) into out (device, npix x nout)
+void launch_decode_u8(Impl& I, const float* z, uint8_t* out);
 // decode the decode buffer and download it as 8-bit values
 void decode_rgb8_impl(Impl& I, uint8_t* out);
 // decode the decode buffer on the device and return mse_of's per-texture and weighted figures
