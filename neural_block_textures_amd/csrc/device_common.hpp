@@ -92,6 +92,12 @@ __device__ __forceinline__ float gauss_at(const NoiseFix& fx, uint64_t head, uin
     return __fmul_rn(nm_radius(fx, (uint32_t)(h >> 40)), nm_cosine(fx, (uint32_t)(h & 0xFFFFFFull)));
 }
 
+// a power of two in 2^-30 .. 2^30 that brings v below 2^e (1 for zero, an infinity or a NaN)
+__device__ __forceinline__ float split_pow2(float v, int e) {
+    const int x = (int)((__float_as_uint(v) >> 23) & 255u);   // v < 2^(x - 126)
+    return x == 0 || x == 255 ? 1.0f : __uint_as_float((uint32_t)(127 + min(30, max(-30, e + 126 - x))) << 23);
+}
+
 // ---------------------------------------------------------------- geometry (main.cpp:507-547)
 struct Tap { int x0, x1, y0, y1; float fx, fy; };
 

@@ -96,7 +96,8 @@ std::vector<std::string> expressions(const std::string& shape, const DevModel& m
         v.push_back(e("k_pop_mfma", std::to_string(a_es) + ", " + c + ", 2"));
         if (split_pays(m.nin, m.nl))
             for (int from : { 0, 1, 2 }) v.push_back(e("k_pop_split", c + ", " + std::to_string(from) + ", false"));
-        v.push_back(e("k_lat_pair_mfma", std::to_string(a_es) + ", " + c));
+        if (split_pays(m.nin, m.nl)) v.push_back(e("k_lat_split", c + ", false"));
+        else v.push_back(e("k_lat_pair_mfma", std::to_string(a_es) + ", " + c));
     }
     v.push_back(e("k_qat_mfma", std::to_string(unit ? kActFold : kActAny) + ", " + c));
     return v;

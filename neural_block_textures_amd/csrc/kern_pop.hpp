@@ -289,8 +289,9 @@ __global__ void __launch_bounds__(64 * kPopWaves) __attribute__((amdgpu_waves_pe
 }
 
 // waves per SIMD the split kernel's register allocation aims at (more would spill)
+constexpr int split_waves(int nin, int H, int nout) { return H > 48 ? 2 : ((nin <= 8 && H <= 32 && (nout > 4 || H <= 16)) ? 4 : 3); }
 template <class S>
-constexpr int split_occupancy() { return MfmaShape<S>::kH > 48 ? 2 : ((MfmaShape<S>::kIn <= 8 && MfmaShape<S>::kH <= 32 && (!valu_out<S>() || MfmaShape<S>::kHt == 1)) ? 4 : 3); }
+constexpr int split_occupancy() { return split_waves(MfmaShape<S>::kIn, MfmaShape<S>::kH, MfmaShape<S>::kNout); }
 // the minibatch slot by slot (device_common.hpp, split_inputs) and the step's layer scales (split_mlp.hpp)
 struct SplitIn {
     const u4v* feat;
@@ -597,66 +598,6 @@ __device__ __forceinline__ void features_pm(const DevModel& m, __amdgpu_buffer_r
     }
 }
 
-// Models whose latent step perturbs level 1 only (level 0 searched under --qat, so the step's mask is 2) and whose
-// level-0 channels and positional features fill whole k-steps of the first layer: the latent pair takes those
-// inputs first (level 0, then the positional features, then level 1), so the k-steps over them are one chain of
-// matrix instructions for both members of a pair, which each member's level-1 k-steps continue. Each unit's
-// first-layer sum then adds the same products in that order instead of the reference's (main.cpp:603-627).
-// The shared k-steps, or 0 where the layout has none.
-template <class S>
-constexpr int lat_shared_ksteps() {
-    return (S::kFixed && S::kC2 == 0 && S::kC1 > 0 && (S::kC0 + 2 * S::kNpos) % 4 == 0) ? (S::kC0 + 2 * S::kNpos) / 4 : 0;
-}
-// position p of that order holds input map(p) of the reference's order
-template <class S>
-struct InLatShared {
-    __host__ __device__ static constexpr int map(int p) {
-        return p < S::kC0 ? p : (p < S::kC0 + 2 * S::kNpos ? S::kC0 + S::kC1 + (p - S::kC0) : S::kC0 + (p - S::kC0 - 2 * S::kNpos));
-    }
-};
-template <bool B, class A, class C> struct PickType { using type = A; };
-template <class A, class C> struct PickType<false, A, C> { using type = C; };
-
-// sample_latent of an unperturbed level through its raw buffer (sample_level_pm's loads and blend, one member)
-template <int C>
-__device__ __forceinline__ void sample_level_plain(const DevLevel& L, __amdgpu_buffer_rsrc_t rz, const Tap& t, float* f) {
-    const uint32_t off = (uint32_t)L.off, LW = (uint32_t)L.W, LC = (uint32_t)L.C;
-    const uint32_t a = 4u * (off + ((uint32_t)t.y0 * LW + (uint32_t)t.x0) * LC);
-    if (L.nearest) {
-#pragma unroll
-        for (int c = 0; c < C; c++) f[c] = buffer_f32(rz, a + 4u * c, 0u);
-        return;
-    }
-    const uint32_t tap[4] = { a, 4u * (off + ((uint32_t)t.y0 * LW + (uint32_t)t.x1) * LC),
-                              4u * (off + ((uint32_t)t.y1 * LW + (uint32_t)t.x0) * LC),
-                              4u * (off + ((uint32_t)t.y1 * LW + (uint32_t)t.x1) * LC) };
-    const Blend w = blend_of(t);
-#pragma unroll
-    for (int c = 0; c < C; c++)
-        f[c] = blend(w, buffer_f32(rz, tap[0] + 4u * c, 0u), buffer_f32(rz, tap[1] + 4u * c, 0u), buffer_f32(rz, tap[2] + 4u * c, 0u),
-                     buffer_f32(rz, tap[3] + 4u * c, 0u));
-}
-
-// The features of one pixel for a latent pair in the shared order (lat_shared_ksteps): fs = level 0 and the
-// positional features, common to both members; fp / fm = level 1 perturbed by +sg eps / -sg eps (features_pm's
-// values, in another arrangement).
-template <class S>
-__device__ __forceinline__ void features_lat_shared(const DevModel& m, __amdgpu_buffer_rsrc_t rz, __amdgpu_buffer_rsrc_t re, float sg,
-                                                    int px, int py, float (&fs)[S::kC0 + 2 * S::kNpos], float (&fp)[S::kC1],
-                                                    float (&fm)[S::kC1]) {
-    const float u = pixel_u(px, m.W), v = pixel_u(py, m.H);
-    const Tap t0 = tap_of(m.lv[0].W, m.lv[0].H, m.lv[0].nearest != 0, u, v);
-    const Tap t1 = tap_of(m.lv[1].W, m.lv[1].H, m.lv[1].nearest != 0, u, v);
-    sample_level_plain<S::kC0>(m.lv[0], rz, t0, fs);
-    sample_level_pm<S::kC1>(m.lv[1], rz, re, sg, t1, fp, fm);
-#pragma unroll
-    for (int q = 0; q < S::kNpos; q++) {
-        const bool uv = m.pos[q] == 0;
-        fs[S::kC0 + 2 * q] = __builtin_fmaf(uv ? u : t1.fx, 2.0f, -1.0f);
-        fs[S::kC0 + 2 * q + 1] = __builtin_fmaf(uv ? v : t1.fy, 2.0f, -1.0f);
-    }
-}
-
 // The column and row of pixel base + lane for a wave's 64 pixels from base (a multiple of 64): when the
 // image's width is a multiple of 64 they share one row (a scalar division), else each lane divides (pixels
 // past the last clamped to it).
@@ -673,39 +614,19 @@ __device__ __forceinline__ void round_pixel(const DevModel& m, int base, int lan
 }
 
 
-// One 16-pixel tile of a latent pair: both members' MLPs on the tile's first-layer operands (Sh > 0: the shared
-// k-steps' bs, continued by each member's own bp / bm; Sh = 0: each member's whole first layer bp / bm), each lane's
+// One 16-pixel tile of a latent pair: both members' MLPs on the tile's first-layer operands bp / bm, each lane's
 // channel terms cw (d d) (its out_regs in ascending order, or its one on the VALU output layer), the pixel's four
 // lane groups added pairwise for each member (group_sums), and (e+ - e-) inv_px written to out[p] by lane group 0.
-template <class S, int Act, bool Clamp, int Sh, bool UnitCw>
+template <class S, int Act, bool Clamp>
 __device__ __forceinline__ void lat_pair_tile(const DevModel& m, const MfmaWeights<S>& W, float ak, const float (&cw)[4],
-                                              const float (&bs)[Sh > 0 ? Sh : 1],
-                                              const float (&bp)[Sh > 0 ? MfmaShape<S>::kKs1 - Sh : MfmaShape<S>::kKs1],
-                                              const float (&bm)[Sh > 0 ? MfmaShape<S>::kKs1 - Sh : MfmaShape<S>::kKs1],
+                                              const float (&bp)[MfmaShape<S>::kKs1], const float (&bm)[MfmaShape<S>::kKs1],
                                               const float (&tt)[4], float* vo, float* sums, int g, int i16, int p,
                                               float* __restrict__ out) {
     using Q = MfmaShape<S>;
-    constexpr int NO = Q::kNout, kM = Q::kKs1 - Sh;
     constexpr bool kVOut = valu_out<S>();
     // the first layer's pre-activations of both members (D layout)
     f4v a1[2][Q::kHt];
-    if constexpr (Sh > 0) {
-        f4v as[Q::kHt];
-#pragma unroll
-        for (int ot = 0; ot < Q::kHt; ot++) as[ot] = W.c1[ot];
-#pragma unroll
-        for (int ks = 0; ks < Sh; ks++)
-#pragma unroll
-            for (int ot = 0; ot < Q::kHt; ot++) as[ot] = mfma4(W.a1[ot][ks], bs[ks], as[ot]);
-#pragma unroll
-        for (int ot = 0; ot < Q::kHt; ot++) { a1[0][ot] = as[ot]; a1[1][ot] = as[ot]; }
-#pragma unroll
-        for (int ks = 0; ks < kM; ks++)
-#pragma unroll
-            for (int v = 0; v < 2; v++)
-#pragma unroll
-                for (int ot = 0; ot < Q::kHt; ot++) a1[v][ot] = mfma4(W.a1[ot][Sh + ks], v ? bm[ks] : bp[ks], a1[v][ot]);
-    } else {
+    {
         float b1[2][Q::kKs1];
 #pragma unroll
         for (int ks = 0; ks < Q::kKs1; ks++) { b1[0][ks] = bp[ks]; b1[1][ks] = bm[ks]; }
@@ -717,9 +638,8 @@ __device__ __forceinline__ void lat_pair_tile(const DevModel& m, const MfmaWeigh
         mfma_hidden_from1<S, 2, Act>(W, a1, ak, x);
         const float dp = out_of<S>(valu_out_g<S>(W, x[0], vo, g, i16), Clamp) - tt[0],
                     dm = out_of<S>(valu_out_g<S>(W, x[1], vo + kVoTile, g, i16), Clamp) - tt[0];
-        constexpr bool kUnit = UnitCw && NO == 4;   // (lane groups past nout need their zero weight)
-        ep = kUnit ? __fmul_rn(dp, dp) : __fmul_rn(cw[0], __fmul_rn(dp, dp));
-        em = kUnit ? __fmul_rn(dm, dm) : __fmul_rn(cw[0], __fmul_rn(dm, dm));
+        ep = __fmul_rn(cw[0], __fmul_rn(dp, dp));
+        em = __fmul_rn(cw[0], __fmul_rn(dm, dm));
     } else {
         float x[2][Q::kKsH];
         mfma_hidden_from1<S, 2, Act>(W, a1, ak, x);
@@ -728,9 +648,8 @@ __device__ __forceinline__ void lat_pair_tile(const DevModel& m, const MfmaWeigh
 #pragma unroll
         for (int r = 0; r < out_regs<S>(); r++) {
             const float dp = out_of<S>(o[0][r], Clamp) - tt[r], dm = out_of<S>(o[1][r], Clamp) - tt[r];
-            constexpr bool kUnit = UnitCw && NO == 4 * out_regs<S>();   // (padding rows need their zero weight)
-            ep = kUnit ? __builtin_fmaf(dp, dp, ep) : __builtin_fmaf(cw[r], __fmul_rn(dp, dp), ep);
-            em = kUnit ? __builtin_fmaf(dm, dm, em) : __builtin_fmaf(cw[r], __fmul_rn(dm, dm), em);
+            ep = __builtin_fmaf(cw[r], __fmul_rn(dp, dp), ep);
+            em = __builtin_fmaf(cw[r], __fmul_rn(dm, dm), em);
         }
     }
     float sp, sm;
@@ -738,24 +657,19 @@ __device__ __forceinline__ void lat_pair_tile(const DevModel& m, const MfmaWeigh
     if (g == 0 && p < m.npix) out[p] = __fmul_rn(sp - sm, m.inv_px);
 }
 
-// Sh > 0: the shared first-layer k-steps of lat_shared_ksteps (the launch's mask must be 2: level 1 perturbed only).
-// UnitCw: every channel weight is 1, so a pixel's error terms are d d (fused into the sum where a lane holds several)
-template <class S, int Act, bool Clamp, int Sh = 0, bool UnitCw = false>
+template <class S, int Act, bool Clamp>
 __global__ void __launch_bounds__(256) k_lat_pair_mfma(DevModel m, const float* __restrict__ w, const float* __restrict__ zdec,
                                                       const float* __restrict__ eps, const float* __restrict__ tgt, float sg,
                                                       unsigned mask, float* __restrict__ dpix, int rounds) {
     using Q = MfmaShape<S>;
     constexpr int NO = Q::kNout, kRounds = lat_rounds<S>();
-    static_assert(Sh == 0 || Sh == lat_shared_ksteps<S>(), "the shared k-steps of the layout");
-    constexpr int kM = Q::kKs1 - Sh;   // each member's own k-steps of the first layer
     // at most 4 outputs: the output layer on the VALU leaves output g of pixel j in lane (g, j)
     constexpr bool kVOut = valu_out<S>();
     const int k = bid_y();
     const int lane = tid_x() & 63, wave = __builtin_amdgcn_readfirstlane(tid_x() >> 6), i16 = lane & 15, g = lane >> 4;
-    // each wave's LDS exchanges (in place of lane swaps): the tile operands (both members', or the shared k-steps
-    // and both members' own), the VALU output layer's reduce-scatters of both members, the pixel sums of both
-    // members' errors
-    constexpr int kTileLds = Sh > 0 ? 4 * 64 * (Sh + 2 * kM) : 2 * kTilesLds<S>;
+    // each wave's LDS exchanges (in place of lane swaps): both members' tile operands, the VALU output layer's
+    // reduce-scatters of both members, the pixel sums of both members' errors
+    constexpr int kTileLds = 2 * kTilesLds<S>;
     constexpr int kWaveLds = kTileLds + (kVOut ? 2 * kVoTile : 0) + kSumsLds;
     __shared__ __attribute__((aligned(16))) float lds[4 * kWaveLds];
     float* const tl = lds + wave * kWaveLds;
@@ -765,7 +679,7 @@ __global__ void __launch_bounds__(256) k_lat_pair_mfma(DevModel m, const float* 
                                  rn = buffer_of(eps, 0u);   // a level outside the mask: no Gaussians (every load 0)
     float* out = dpix + (size_t)k * m.npix;
     MfmaWeights<S> W;
-    mfma_load<S, typename PickType<(Sh > 0), InLatShared<S>, InIdentity>::type>(W, w, lane);
+    mfma_load<S>(W, w, lane);
     if constexpr (!Clamp) scale_output<S>(W, kNegLog2e);
     if constexpr (Act == kActFold) scale_hidden<S>(W, fold_scale(m.leak));
     const float ak = act_k_of<Act>(m);
@@ -794,23 +708,15 @@ __global__ void __launch_bounds__(256) k_lat_pair_mfma(DevModel m, const float* 
         const int base = bid_x() * 256 * rounds + 64 * rounds * wave + 64 * rd;   // tile t: pixels base + 16 t + j
         float tn[4];
         load_t(base, tn);
-        // both members' first-layer operands (Sh = 0), or the shared k-steps' and each member's own (Sh > 0)
-        float bp[4][Sh > 0 ? kM : Q::kKs1], bm[4][Sh > 0 ? kM : Q::kKs1], bs[4][Sh > 0 ? Sh : 1];
+        // both members' first-layer operands
+        float bp[4][Q::kKs1], bm[4][Q::kKs1];
         {
             int px, py;
             round_pixel(m, base, lane, px, py);
-            if constexpr (Sh > 0) {
-                float fs[S::kC0 + 2 * S::kNpos], fp[S::kC1], fm[S::kC1];
-                features_lat_shared<S>(m, rz, re, sg, px, py, fs, fp, fm);
-                tiles_of_n<Sh>(fs, bs, tl, g, i16);
-                tiles_of_n<kM>(fp, bp, tl + 4 * 64 * Sh, g, i16);
-                tiles_of_n<kM>(fm, bm, tl + 4 * 64 * (Sh + kM), g, i16);
-            } else {
-                float fp[S::kMaxIn], fm[S::kMaxIn];
-                features_pm<S>(m, rz, re, rn, sg, mask, px, py, fp, fm);
-                tiles_of<S>(fp, bp, tl, g, i16);
-                tiles_of<S>(fm, bm, tl + kTilesLds<S>, g, i16);
-            }
+            float fp[S::kMaxIn], fm[S::kMaxIn];
+            features_pm<S>(m, rz, re, rn, sg, mask, px, py, fp, fm);
+            tiles_of<S>(fp, bp, tl, g, i16);
+            tiles_of<S>(fm, bm, tl + kTilesLds<S>, g, i16);
         }
 #pragma unroll
         for (int t = 0; t < 4; t++) {
@@ -819,9 +725,231 @@ __global__ void __launch_bounds__(256) k_lat_pair_mfma(DevModel m, const float* 
             for (int r = 0; r < 4; r++) tt[r] = tn[r];
             if (t + 1 < 4) load_t(base + 16 * (t + 1), tn);
             const int p = base + 16 * t + i16;
-            lat_pair_tile<S, Act, Clamp, Sh, UnitCw>(m, W, ak, cw, bs[t], bp[t], bm[t], tt, vo, sums, g, i16, p, out);
+            lat_pair_tile<S, Act, Clamp>(m, W, ak, cw, bp[t], bm[t], tt, vo, sums, g, i16, p, out);
         }
     }
+}
+
+// ---- The latent pair evaluation on the 16-bit matrix instructions with operands in two parts (split_mlp.hpp), for the shapes
+// k_pop_split takes: as many blocks as fit the chip, each of which stages the current weights once (split_stage_plain); a
+// wave takes 64 pixels of a pair at a time, every wave's next one a whole grid further, over all pairs. Each lane builds its
+// pixel's features for both members (features_pm) and writes them split to the wave's LDS; lane group g of a 16-pixel tile
+// reads back the 16 bytes of parts that its slots of the first layer take. A lane's channel terms of the + member less those of the - member
+// are added over a pixel's four lane groups (more than 4 outputs; through LDS, so that each lane ends with one of the 64
+// pixels), or are the pixel's own (at most 4: split_mlp.hpp, ao). A wave that met a NaN evaluates its rounds again in 32 bits
+// (lat_pair_tile), as k_pop_split does.
+// What bounds it is instruction issue, as in k_pop_split, with the feature loads (two floats a tap and channel) beside it.
+// Against k_lat_pair_mfma (MI355X): 512 x 512, four maps, a searched and a 4-channel level, 4 pairs: 71 -> 40 us; RGB, levels of 8 and 4 channels,
+// 16 pairs: 292 -> 165 us. All four products of the two parts are taken (1% of the step): over seven models of three seeds the
+// gradient's error against 64 bits is 1.002 times the 32-bit kernel's, 1.004 without the product of the lo parts.
+template <class S>
+__device__ __forceinline__ SplitScale split_stage_plain(const DevModel& m, const float* __restrict__ w, double out, unsigned* __restrict__ lds) {
+    using L = SplitLds<S>;
+    constexpr int kP = MfmaShape<S>::kP, kN = (kP + 255) / 256;
+    __shared__ float top[4][3];
+    float v[kN], mx[3] = { 0.0f, 0.0f, 0.0f };
+#pragma unroll
+    for (int q = 0; q < kN; q++) v[q] = w[min(tid_x() + 256 * q, kP - 1)];
+#pragma unroll
+    for (int q = 0; q < kN; q++) {
+        const int k = min(tid_x() + 256 * q, kP - 1);
+        const float a = L::bias(k) ? 0.0f : fabsf(v[q]);
+#pragma unroll
+        for (int l = 0; l < 3; l++) mx[l] = fmaxf(mx[l], L::layer(k) == l ? a : 0.0f);
+    }
+#pragma unroll
+    for (int l = 0; l < 3; l++)
+        for (int o = 32; o > 0; o >>= 1) mx[l] = fmaxf(mx[l], __shfl_xor(mx[l], o, 64));
+    if ((tid_x() & 63) == 0)
+#pragma unroll
+        for (int l = 0; l < 3; l++) top[tid_x() >> 6][l] = mx[l];
+    __syncthreads();
+#pragma unroll
+    for (int l = 0; l < 3; l++) mx[l] = fmaxf(fmaxf(top[0][l], top[1][l]), fmaxf(top[2][l], top[3][l]));
+    const float fold = fold_scale(m.leak);
+    SplitScale sc{ split_pow2(mx[0] * fold, kSplitExp[0]), MfmaShape<S>::kNL > 1 ? split_pow2(mx[1] * fold, kSplitExp[1]) : 1.0f,
+                   split_pow2(mx[2] * (float)fabs(out), kSplitExp[2]), 0.0f };
+    sc.inv = 1.0f / (kSplitFeat * sc.s1 * sc.s2 * sc.s3);
+    const SplitFactors f = split_factors(sc, m.fold_c, out);
+#pragma unroll
+    for (int q = 0; q < kN; q++) {
+        const int k = tid_x() + 256 * q;
+        if (k < kP) {
+            const int l = L::layer(k);
+            const bool b = L::bias(k);
+            const double fw = l == 0 ? f.w1 : (l == 1 ? f.w2 : f.w3), fb = l == 0 ? f.b1 : (l == 1 ? f.b2 : f.b3);
+            lds[L::pos(k)] = split_param(v[q], 0.0f, 0.0f, b ? fb : fw, b);
+        }
+    }
+    __syncthreads();
+    return sc;
+}
+
+// A wave's 64 pixels' features f (lane: one pixel) split to t: per pixel split_inputs hi parts, then as many lo parts
+template <class S>
+__device__ __forceinline__ void split_write(const float (&f)[S::kMaxIn], float neg, u4v* __restrict__ t, int lane) {
+    constexpr int N = split_inputs(S::kNin), C = N / 8;   // 16-byte pieces per part
+#pragma unroll
+    for (int q = 0; q < C; q++) {
+        h2v hi[4], lo[4];
+#pragma unroll
+        for (int j = 0; j < 4; j++) {
+            const int i = 8 * q + 2 * j;
+            const float x = i < S::kNin ? f[i < S::kNin ? i : 0] * kSplitFeat : 0.0f, y = i + 1 < S::kNin ? f[i + 1 < S::kNin ? i + 1 : 0] * kSplitFeat : 0.0f;
+            split2(x, y, neg, hi[j], lo[j]);
+        }
+        u4v a, b;
+#pragma unroll
+        for (int j = 0; j < 4; j++) { a[j] = __builtin_bit_cast(unsigned, hi[j]); b[j] = __builtin_bit_cast(unsigned, lo[j]); }
+        t[lane * 2 * C + q] = a;
+        t[lane * 2 * C + C + q] = b;
+    }
+}
+// the first-layer operand of pixel `px` (of the wave's 64) for lane group g
+template <class S>
+__device__ __forceinline__ h8v split_read(const u4v* __restrict__ t, int px, int g) {
+    constexpr int C = split_inputs(S::kNin) / 8;
+    return __builtin_bit_cast(h8v, t[px * 2 * C + (C == 1 ? (g & 1) : g)]);
+}
+
+template <class S, bool Clamp, bool UnitCw>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(split_occupancy<S>()))) k_lat_split(DevModel m, const float* __restrict__ w, const float* __restrict__ zdec,
+                                                      const float* __restrict__ eps, const float* __restrict__ tgt, float sg,
+                                                      unsigned mask, float* __restrict__ dpix, int K, int blocks) {
+    using Q = MfmaShape<S>;
+    using P = SplitShape<S>;
+    constexpr int NO = Q::kNout, RO = out_regs<S>(), kEx = 64 * split_inputs(Q::kIn);   // floats of one member's exchange
+    constexpr bool kVOut = valu_out<S>();
+    constexpr int NT = kVOut ? NO : RO;
+    static_assert(2 * kTilesLds<S> <= 2 * kEx && (!kVOut || 2 * kVoTile + kSumsLds <= 2 * kEx), "the 32-bit evaluation's exchanges fit");
+    __shared__ unsigned par_s[SplitLds<S>::kWords];
+    __shared__ __attribute__((aligned(16))) float ex_s[4][2 * kEx];
+    __shared__ __attribute__((aligned(16))) float sum_s[kVOut ? 1 : 4][kVOut ? 4 : 256];
+    const int lane = tid_x() & 63, wave = __builtin_amdgcn_readfirstlane(tid_x() >> 6), i16 = lane & 15, g = lane >> 4;
+    const SplitScale sc = split_stage_plain<S>(m, w, Clamp ? 1.0 : kNegLog2eD, par_s);
+    SplitWeights<S> W;
+    split_load<S>(W, par_s, lane);
+    const float ak = in_vgpr(act_k_of<kActFold>(m)), neg = in_vgpr(-1.0f), inv = in_vgpr(sc.inv);
+    float cw[NT];
+#pragma unroll
+    for (int r = 0; r < NT; r++) {
+        cw[r] = 0.0f;
+#pragma unroll
+        for (int c = 0; c < NO; c++)
+            if ((kVOut ? r : out_at<S>(g, r)) == c) cw[r] = m.cw[c];
+    }
+    constexpr bool kUnit = UnitCw && (kVOut || NO == 4 * RO);
+    const __amdgpu_buffer_rsrc_t rz = buffer_of(zdec, 4u * (uint32_t)m.nz), rn = buffer_of(eps, 0u);
+    float* const ex = ex_s[wave];
+    const int R = (m.npix + 63) >> 6;                       // 64-pixel rounds of an image
+    const int stride = 4 * blocks;
+    // this wave's rounds: f(pair, first pixel)
+    auto rounds = [&](auto f) {
+        int k = 0;
+        for (int rd = bid_x() * 4 + wave;; rd += stride) {
+            while (rd >= R && k < K) { rd -= R; k++; }
+            if (k >= K) break;
+            f(k, 64 * rd);
+        }
+    };
+    bool again = false;   // a round had a NaN
+    rounds([&](int k, int base) {
+        const __amdgpu_buffer_rsrc_t re = buffer_of(eps + (size_t)k * m.nz, 4u * (uint32_t)m.nz);
+        float* const out = dpix + (size_t)k * m.npix;
+        {
+            int px, py;
+            round_pixel(m, base, lane, px, py);
+            float fp[S::kMaxIn], fm[S::kMaxIn];
+            features_pm<S>(m, rz, re, rn, sg, mask, px, py, fp, fm);
+            split_write<S>(fp, neg, (u4v*)ex, lane);
+            split_write<S>(fm, neg, (u4v*)(ex + kEx), lane);
+        }
+        wave_lds_fence();
+        bool bad = false;
+        // this lane's channel terms of the + member less the - member's: cw (d+ d+ - d- d-) as cw (d+ - d-) (d+ + d-), which
+        // rounds relative to the difference and not to each square (the two members' errors are close)
+        auto terms = [&](const f4v& op, const f4v& om, const float (&t)[NT]) {
+            float e = 0.0f;
+#pragma unroll
+            for (int r = 0; r < NT; r++) {
+                const float sp = op[r] * inv, sm = om[r] * inv;
+                if constexpr (Clamp) bad |= !not_nan_bits(sp) || !not_nan_bits(sm);
+                const float vp = out_of<S>(sp, Clamp), vm = out_of<S>(sm, Clamp);
+                const float d = vp - vm, c = (vp - t[r]) + (vm - t[r]);
+                e = __builtin_fmaf(kUnit ? d : __fmul_rn(cw[r], d), c, e);
+            }
+            return e;
+        };
+        float diff;
+        if constexpr (kVOut) {
+            float t[NT];
+            const int pr = min(base + lane, m.npix - 1);
+#pragma unroll
+            for (int r = 0; r < NT; r++) t[r] = tgt[(size_t)pr * NO + r];
+            f4v o[2] = { W.co, W.co };
+#pragma unroll
+            for (int u = 0; u < 4; u++)
+#pragma unroll
+                for (int v = 0; v < 2; v++) {
+                    h8v b[P::kB];
+                    split_hidden<S, true>(W, split_read<S>((const u4v*)(ex + v * kEx), 16 * u + i16, g), ak, neg, b);
+                    o[v] = split_dot<S, true>(W.ao[u], b, o[v]);
+                }
+            diff = terms(o[0], o[1], t);
+        } else {
+            float* const sums = sum_s[wave];
+#pragma unroll
+            for (int u = 0; u < 4; u++) {
+                float t[NT];
+                const int pr = min(base + 16 * u + i16, m.npix - 1);
+#pragma unroll
+                for (int r = 0; r < NT; r++) t[r] = tgt[(size_t)pr * NO + max(out_at<S>(g, r), 0)];
+                f4v o[2];
+#pragma unroll
+                for (int v = 0; v < 2; v++) {
+                    h8v b[P::kB];
+                    split_hidden<S, true>(W, split_read<S>((const u4v*)(ex + v * kEx), 16 * u + i16, g), ak, neg, b);
+                    o[v] = split_dot<S, true>(W.ao[0], b, W.co);
+                }
+                sums[(16 * u + i16) * 4 + g] = terms(o[0], o[1], t);
+            }
+            wave_lds_fence();
+            const f4v v = *reinterpret_cast<const f4v*>(sums + 4 * lane);
+            diff = (v[0] + v[2]) + (v[1] + v[3]);
+        }
+        wave_lds_fence();
+        again |= __builtin_amdgcn_ballot_w64(bad || !not_nan_bits(diff)) != 0;
+        if (base + lane < m.npix) out[base + lane] = __fmul_rn(diff, m.inv_px);
+    });
+    if (!again) return;
+    // 32 bits, all of the wave's rounds
+    MfmaWeights<S> F;
+    mfma_load<S>(F, w, lane);
+    if constexpr (!Clamp) scale_output<S>(F, kNegLog2e);
+    scale_hidden<S>(F, fold_scale(m.leak));
+    rounds([&](int k, int base) {
+        const __amdgpu_buffer_rsrc_t re = buffer_of(eps + (size_t)k * m.nz, 4u * (uint32_t)m.nz);
+        float* const out = dpix + (size_t)k * m.npix;
+        float bp[4][Q::kKs1], bm[4][Q::kKs1], cw4[4];
+        {
+            int px, py;
+            round_pixel(m, base, lane, px, py);
+            float fp[S::kMaxIn], fm[S::kMaxIn];
+            features_pm<S>(m, rz, re, rn, sg, mask, px, py, fp, fm);
+            tiles_of<S>(fp, bp, ex, g, i16);
+            tiles_of<S>(fm, bm, ex + kTilesLds<S>, g, i16);
+        }
+#pragma unroll
+        for (int r = 0; r < 4; r++) cw4[r] = kVOut ? ((r == 0 && g < NO) ? m.cw[min(g, NO - 1)] : 0.0f) : (r < NT ? cw[r < NT ? r : 0] : 0.0f);
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+            float t[4];
+            const int pr = min(base + 16 * u + i16, m.npix - 1);
+#pragma unroll
+            for (int r = 0; r < 4; r++) t[r] = tgt[(size_t)pr * NO + (kVOut ? min(g, NO - 1) : max(out_at<S>(g, r), 0))];
+            lat_pair_tile<S, kActFold, Clamp>(m, F, ak, cw4, bp[u], bm[u], t, ex, ex + 2 * kVoTile, g, i16, base + 16 * u + i16, out);
+        }
+    });
 }
 
 // The selector search's occupancy target: four waves per SIMD for the 8-input, 32-wide models with more than 4

@@ -39,11 +39,6 @@ struct SplitJob {
     int block;
 };
 
-// a power of two in 2^-30 .. 2^30 that brings v below 2^e (1 for zero, an infinity or a NaN)
-__device__ __forceinline__ float split_pow2(float v, int e) {
-    const int x = (int)((__float_as_uint(v) >> 23) & 255u);   // v < 2^(x - 126)
-    return x == 0 || x == 255 ? 1.0f : __uint_as_float((uint32_t)(127 + clampi(e + 126 - x, -30, 30)) << 23);
-}
 __device__ inline void split_scales(const DevModel& m, const SplitJob& sj) {
     __shared__ float red[kTPB / 64];
     float total = kSplitFeat;

@@ -198,27 +198,8 @@ static int lat_rounds_for(const Impl& I, int most, int K) {
     return most;
 }
 
-bool lat_pair_on_matrix_cores(const Impl& I) { return pop_on_matrix_cores(I); }
-
-template <class S, int Act, int Sh>
-static auto lat_kernel(bool clamp, bool unit) {
-    return clamp ? (unit ? k_lat_pair_mfma<S, Act, true, Sh, true> : k_lat_pair_mfma<S, Act, true, Sh, false>)
-                 : (unit ? k_lat_pair_mfma<S, Act, false, Sh, true> : k_lat_pair_mfma<S, Act, false, Sh, false>);
-}
-
-template <class S, int Act>
-static void launch_lat_mfma(Impl& I, int K, float sigma, unsigned mask) {
-    // a step that perturbs level 1 only shares the first layer's level-0 and positional k-steps between the members
-    constexpr int Sh = lat_shared_ksteps<S>();
-    auto kern = lat_kernel<S, Act, 0>(I.dm.clamp_out, unit_cw(I));
-    if constexpr (Sh > 0) {
-        if (mask == 2u) kern = lat_kernel<S, Act, Sh>(I.dm.clamp_out, unit_cw(I));
-    }
-    static_assert(lat_rounds<S>() >= 1, "a latent pair kernel takes at least one round");
-    const int rounds = lat_rounds_for(I, lat_rounds<S>(), K), pix = 256 * rounds;
-    hipLaunchKernelGGL(kern, dim3((unsigned)((I.npix + pix - 1) / pix), K), dim3(256), 0, I.stream, I.dm, I.w, I.zdec,
-                       I.eps_lat, I.tgt, sigma, mask, I.dpix, rounds);
-}
+// (k_lat_pair_mfma, for the shapes the split kernel does not take, is compiled at init only)
+bool lat_pair_on_matrix_cores(const Impl& I) { return pop_on_matrix_cores(I) && (I.jit || split_pays(I.dm.nin, I.dm.nl)); }
 
 void launch_lat_pair(Impl& I, int K, float sigma, unsigned mask) {
     ProfScope ps(I, "lat_pair");
@@ -226,21 +207,29 @@ void launch_lat_pair(Impl& I, int K, float sigma, unsigned mask) {
         launch_lat_pair_valu(I, K, sigma, mask);
         return;
     }
-    if (I.jit) {
-        const int act = kActFold;
-        const int rounds = lat_rounds_for(I, lat_rounds_of(I.dm.nin), K), pix = 256 * rounds;
-        jit_launch(k_lat_pair_mfma<ShapeMaterial, kActFold, false>, I, "k_lat_pair_mfma",
-                   std::to_string(act) + (I.dm.clamp_out ? ", true" : ", false"), dim3((unsigned)((I.npix + pix - 1) / pix), K), dim3(256), 0,
-                   I.dm, I.w, I.zdec, I.eps_lat, I.tgt, sigma, mask, I.dpix, rounds);
+    if (split_pays(I.dm.nin, I.dm.nl)) {
+        // as many blocks as fit the chip, or as 64-pixel rounds fill
+        const size_t rounds = (I.npix + 63) / 64 * (size_t)K;
+        const unsigned blocks = (unsigned)std::min<size_t>((size_t)I.cus * split_waves(I.dm.nin, I.dm.hidden[0], I.dm.nout), (rounds + 3) / 4);
+        if (I.jit) {
+            jit_launch(k_lat_split<ShapeMaterial, false, false>, I, "k_lat_split", I.dm.clamp_out ? "true, false" : "false, false", dim3(blocks),
+                       dim3(256), 0, I.dm, I.w, I.zdec, I.eps_lat, I.tgt, sigma, mask, I.dpix, K, (int)blocks);
+        } else dispatch_shape(I.dm, [&](auto s) {
+            using S = decltype(s);
+            if constexpr (SplitShape<S>::kOk) {
+                auto kern = I.dm.clamp_out ? k_lat_split<S, true, false> : (unit_cw(I) ? k_lat_split<S, false, true> : k_lat_split<S, false, false>);
+                hipLaunchKernelGGL(kern, dim3(blocks), dim3(256), 0, I.stream, I.dm, I.w, I.zdec, I.eps_lat, I.tgt, sigma, mask, I.dpix, K,
+                                   (int)blocks);
+            }
+        });
         NTC_CHECK(hipGetLastError());
         return;
     }
-    dispatch_shape(I.dm, [&](auto s) {
-        using S = decltype(s);
-        if constexpr (MfmaShape<S>::kOk) {
-            launch_lat_mfma<S, kActFold>(I, K, sigma, mask);
-        }
-    });
+    // a shape compiled at init (every listed one is the split kernel's)
+    const int rounds = lat_rounds_for(I, lat_rounds_of(I.dm.nin), K), pix = 256 * rounds;
+    jit_launch(k_lat_pair_mfma<ShapeMaterial, kActFold, false>, I, "k_lat_pair_mfma",
+               std::to_string((int)kActFold) + (I.dm.clamp_out ? ", true" : ", false"), dim3((unsigned)((I.npix + pix - 1) / pix), K), dim3(256), 0,
+               I.dm, I.w, I.zdec, I.eps_lat, I.tgt, sigma, mask, I.dpix, rounds);
     NTC_CHECK(hipGetLastError());
 }
 

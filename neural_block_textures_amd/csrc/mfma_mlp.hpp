@@ -134,17 +134,11 @@ struct MfmaWeights {
     f4v c4;
 };
 
-// The order in which the first layer's k-steps take the model's inputs: position p of the operand rows holds
-// input InMap::map(p) (the identity: the reference's input order).
-struct InIdentity {
-    __host__ __device__ static constexpr int map(int p) { return p; }
-};
-
 // Gathers a member's flat parameter vector (per layer W[out][in] row-major, then b[out]) into
 // operand layout; lane = threadIdx.x % 64. Padding units, inputs and outputs get zero weights: every lane
 // reads a parameter (the index clamped to a valid one) and selects zero where it has none, so the gather
 // takes no branches.
-template <class S, class Get, class InMap = InIdentity>
+template <class S, class Get>
 __device__ __forceinline__ void mfma_load_from(MfmaWeights<S>& W, const Get& w, int lane) {
     using Q = MfmaShape<S>;
     constexpr int NIN = Q::kIn, H = Q::kH, NO = Q::kNout;
@@ -155,7 +149,7 @@ __device__ __forceinline__ void mfma_load_from(MfmaWeights<S>& W, const Get& w, 
         const int u = unit_of<Q>(ot, i16), uc = min(u, H - 1);
 #pragma unroll
         for (int ks = 0; ks < Q::kKs1; ks++) {
-            const int pos = 4 * ks + g, in = pos < NIN ? InMap::map(pos) : pos;
+            const int in = 4 * ks + g;
             W.a1[ot][ks] = at(in < NIN && u < H, uc * NIN + min(in, NIN - 1));
         }
 #pragma unroll
@@ -223,9 +217,9 @@ struct ParamsAt {
     __device__ __forceinline__ float operator()(int k) const { return w[k]; }
 };
 
-template <class S, class InMap = InIdentity>
+template <class S>
 __device__ __forceinline__ void mfma_load(MfmaWeights<S>& W, const float* __restrict__ w, int lane) {
-    mfma_load_from<S, ParamsAt, InMap>(W, ParamsAt{ w }, lane);
+    mfma_load_from<S>(W, ParamsAt{ w }, lane);
 }
 
 // Output weights and biases times sc (the evaluations with the hardware sigmoid fold its -log2(e)

@@ -266,8 +266,8 @@ __device__ __forceinline__ void split_act(const f4v (&acc)[MfmaShape<S>::kHt], f
     else if constexpr (P::kRem > 0) b[2 * P::kFull] = join(hi[4 * P::kFull], lo[4 * P::kFull], hi[4 * P::kFull], lo[4 * P::kFull]);
 }
 
-// c plus one tile row block's products with the values b (the small terms last)
-template <class S>
+// c plus one tile row block's products with the values b (the small terms last); All: the products of two lo parts too
+template <class S, bool All = false>
 __device__ __forceinline__ f4v split_dot(const h8v (&a)[SplitShape<S>::kA], const h8v (&b)[SplitShape<S>::kB], f4v c) {
     using P = SplitShape<S>;
 #pragma unroll
@@ -278,13 +278,14 @@ __device__ __forceinline__ f4v split_dot(const h8v (&a)[SplitShape<S>::kA], cons
     for (int f = 0; f < P::kFull; f++) {
         c = mfma_h(a[2 * f], b[2 * f + 1], c);
         c = mfma_h(a[2 * f + 1], b[2 * f], c);
+        if constexpr (All) c = mfma_h(a[2 * f + 1], b[2 * f + 1], c);
     }
     return c;
 }
 
 // the hidden layers of one tile from its first-layer operand (the split features of a slot: split_features), the last
 // one's values as operands
-template <class S>
+template <class S, bool All = false>
 __device__ __forceinline__ void split_hidden(const SplitWeights<S>& W, h8v f, float k, float neg, h8v (&b)[SplitShape<S>::kB]) {
     using Q = MfmaShape<S>;
     using P = SplitShape<S>;
@@ -298,7 +299,7 @@ __device__ __forceinline__ void split_hidden(const SplitWeights<S>& W, h8v f, fl
     if constexpr (Q::kNL > 1) {
         f4v a2[Q::kHt];
 #pragma unroll
-        for (int ot = 0; ot < Q::kHt; ot++) a2[ot] = split_dot<S>(W.ah[ot], b, W.ch[ot]);
+        for (int ot = 0; ot < Q::kHt; ot++) a2[ot] = split_dot<S, All>(W.ah[ot], b, W.ch[ot]);
         split_act<S>(a2, k, neg, b);
     }
 }

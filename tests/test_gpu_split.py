@@ -110,3 +110,43 @@ def test_split_central_differences_edges(orc, name):
         orc.adam(w, g, m, v, 0.005, 1)
         assert np.array_equal(tr.download_model()[1], w)
         tr.close()
+
+
+def latent(orc, lay, z, p, tgt, K, sigma=0.05, seed=6):
+    """the per-pixel differences of a latent step against the oracle's, at the reference's bar (1e-3 of their RMS)"""
+    tr = trainer(lay, z, p, tgt, max_pairs=1, max_batch=16, seed=seed)
+    tr.lat_step(1, np.float32(sigma), 0.0, K)
+    dpix = tr.debug_last_dpix()
+    mask = (1 << len(lay.levels)) - 1
+    _, want, _, _ = orc.lat_grad(lay, p, z, z, tgt, seed, 0, np.float32(sigma), K, mask, want_dpix=True)
+    rms = np.sqrt((want.astype(np.float64) ** 2).mean())
+    say("latent", lay.W, lay.H, "pairs", K, "largest error over the RMS", np.abs(dpix.ravel() - want).max() / rms)
+    assert np.abs(dpix.ravel() - want).max() < 1e-3 * rms
+    tr.close()
+
+
+@pytest.mark.parametrize("name", ["rgb_16x2", "two_level", "material", "material_clamp", "dct_17", "chief1_36", "large", "run8x3",
+                                  "jit_own_13"])
+def test_split_latent_edges(orc, name):
+    """image sizes around a wave's 64 pixels and a block's four rounds, one pair and several"""
+    base = LAYOUTS[name]
+    for W, H, K in ((1, 1, 1), (7, 9, 3), (64, 1, 2), (65, 1, 1), (50, 41, 5), (128, 2, 1)):
+        lay = Layout(**{k: getattr(base, k) for k in base.__dataclass_fields__})
+        lay.W, lay.H = W, H
+        lay.levels = [(max(1, W * w // base.W), max(1, H * h // base.H), c, near) for w, h, c, near in base.levels]
+        z, p, tgt = data(lay, 26)
+        latent(orc, lay, z, p, tgt, K)
+
+
+@pytest.mark.parametrize("name", ["rgb_16x2", "material", "material_clamp", "large"])
+def test_split_latent_range(orc, name):
+    """hidden values past the 16-bit range: the kernel's rounds in 32 bits, on an image of several rounds a wave"""
+    lay = LAYOUTS[name]
+    z, p, tgt = data(lay, 27)
+    nin, h, s = lay.nin, lay.hidden[0], np.float32(2.0 ** 14)
+    p = p.copy()
+    n1, n2 = h * nin + h, h * nin + h + h * h + h
+    p[h * nin:n1] *= s
+    p[n1 + h * h:n2] *= s
+    p[n2:n2 + lay.nout * h] /= s
+    latent(orc, lay, z * s, p, tgt, 3, sigma=0.05 * 2.0 ** 14)
