@@ -6,6 +6,7 @@
 // twice, raster-order scatter into the distinct taps, grad += w * eps), dct_rate_pass 1935-1952,
 // qat_search 2088-2139.
 #include "kern_valu.hpp"
+#include "mfma_mlp.hpp"
 #include "jit.hpp"
 #include "shapes.hpp"
 #include "trainer_impl.hpp"
@@ -37,22 +38,33 @@ __global__ void __launch_bounds__(kTPB) k_lat_eps(NoiseFix nt, DevModel m, uint6
 // over the pixel rectangle that reads the texel, in raster order (the rectangle comes from the host's
 // range table, built with the same tap arithmetic); then grad += (d * scale) * eps per channel, pair
 // after pair. With the --dct-lambda rate term, level 0 also receives (rate_scale * dbits) * scale * eps
-// right after each pair's mse term. Block = 16 texels x 4 pairs: the 64 threads sum the footprints
-// of four pairs at once (each sum in raster order), then apply the four pairs in order to the texels'
-// channels (four threads per texel, each on every fourth channel). A texel's gradient is then final
-// (one block owns it), so with `adam` the block also takes the texel's Adam step (the latent ES step's
+// right after each pair's mse term. A texel's gradient is final when its block has added its pairs (one block owns
+// it), so with `adam` the block also takes the texel's Adam step (the latent ES step's
 // update, main.cpp:2036-2037), and with zq_copy writes the new value to the decode copy too (a level that is neither
 // --qes nor DCT coded, where the snap would copy it). With `first` the gradient starts from zero rather than from grad
 // (the step's first group of pairs).
 //
-// Blocks past the gather's own (blockIdx.x >= gblocks) draw the next latent step's Gaussians for the perturbed
-// levels (the entries lo .. hi - 1 whose level is in `mask`; block d = pair d / eb, entries lo + 128 (d % eb) ..):
+// A block has one to four waves (four pairs a wave: as many as the step's pairs fill) and takes 16 neighbouring texels of a
+// row: lane group q of a wave sums pair q of the wave's four, lane j of it texel j. The sum is one chain of rounded adds, so
+// its length is fixed; what can be fast is what feeds it.
+// kNarrow (rectangles of at most 16 columns): each lane reads its run from memory, the 16 lanes of a pair a few lines.
+// kWide: texels lie further apart than a line, so a wave copies its pairs' rows to LDS, whole lines at a time and the next
+// row in flight while one is added, and every lane reads its texel's run from there; with four waves all 16 pairs' chains
+// run at once. Levels of 128 x 128 x 8 and 32 x 32 x 4 under 512 x 512 pixels, 16 pairs (MI355X): 190 -> 78 us (104 with the four rows a multiple of 64
+// floats apart: sixteen lanes on a bank).
+// kUnit (a level 0 of one pixel per texel): a thread per texel, its pairs in order; a 512 x 512 x 1 plane and a 128 x 128 x 4
+// level, 4 pairs: 31 -> 23 us.
+//
+// Blocks past the gather's own (blockIdx.x >= start[n]) draw the next latent step's Gaussians for the perturbed
+// levels (the entries lo .. hi - 1 whose level is in `mask`; block d = pair d / eb, entries lo + 2 blockDim (d % eb) ..):
 // the values k_lat_eps would draw for step next_step, written to eps_next. They run beside the gather's blocks,
-// which leave most of the chip idle, so the next step needs no draw launch of its own.
+// so the next step needs no draw launch of its own.
 //
 // One launch gathers every perturbed level of the step (GatherLevels: blocks start[i] .. start[i + 1] - 1 take level
 // lv[i]); the rate term goes to level 0, and zq_copy[i] (or null) is level lv[i]'s decode copy.
-constexpr int kGatherTex = 16, kGatherPairs = 4, kGatherRun = 32, kAheadPerBlock = 128;
+constexpr int kGatherTex = 16, kGatherPairs = 4, kGatherWaves = 4, kGatherRun = 32, kWideCols = 320,
+              kWideRow = kWideCols + 4;   // (the four pairs' rows in LDS: texels 16 columns apart then share a bank four at a time, not sixteen)
+enum GatherMode : int { kNarrow = 0, kUnit = 1, kWide = 2 };
 struct LatAhead {
     NoiseFix nt; uint64_t seed; uint32_t next_step; unsigned mask;
     float* eps_next; int eb; long long lo, hi;
@@ -61,117 +73,157 @@ struct GatherLevels {
     int n;
     int lv[kMaxLevels];
     int start[kMaxLevels + 1];
+    int mode[kMaxLevels];
     float* zq_copy[kMaxLevels];
 };
-__global__ void __launch_bounds__(kGatherTex * kGatherPairs) k_lat_gather(DevModel m, GatherLevels G, int K, float scale,
-                                                                         const float* __restrict__ dpix,
-                                                                         const float* __restrict__ eps, const int* __restrict__ ranges,
-                                                                         int rate0, float rate_scale, int dct_bw, int dct_n,
-                                                                         const int32_t* __restrict__ dbits, float* __restrict__ grad,
-                                                                         int first, int adam, float* __restrict__ z, float* __restrict__ zm,
-                                                                         float* __restrict__ zv, float lr, float c1, float c2, LatAhead ah) {
+// Wide: whether a level of the launch is kWide
+template <bool Wide>
+__global__ void __launch_bounds__(64 * kGatherWaves) k_lat_gather(DevModel m, GatherLevels G, int K, float scale,
+                                                                  const float* __restrict__ dpix,
+                                                                  const float* __restrict__ eps, const int* __restrict__ ranges,
+                                                                  int rate0, float rate_scale, int dct_bw, int dct_n,
+                                                                  const int32_t* __restrict__ dbits, float* __restrict__ grad,
+                                                                  int first, int adam, float* __restrict__ z, float* __restrict__ zm,
+                                                                  float* __restrict__ zv, float lr, float c1, float c2, LatAhead ah) {
+    const int threads = (int)blockDim.x;
     if ((int)blockIdx.x >= G.start[G.n]) {   // a draw-ahead block (uniform: the whole block returns here)
         const int d = (int)blockIdx.x - G.start[G.n], k = d / ah.eb;
         const uint64_t head = noise_head(ah.seed, NS_LAT, ah.next_step, (uint32_t)k);
-        const long long i0 = ah.lo + (long long)(d - k * ah.eb) * kAheadPerBlock, i1 = min(ah.hi, i0 + kAheadPerBlock);
-        for (long long i = i0 + threadIdx.x; i < i1; i += kGatherTex * kGatherPairs)
+        const long long i0 = ah.lo + (long long)(d - k * ah.eb) * 2 * threads, i1 = min(ah.hi, i0 + 2 * threads);
+        for (long long i = i0 + threadIdx.x; i < i1; i += threads)
             if ((ah.mask >> level_of(m, i)) & 1u) ah.eps_next[(size_t)k * m.nz + i] = gauss_at(ah.nt, head, (uint64_t)i);
         return;
     }
-    __shared__ float dsum[kGatherPairs][kGatherTex];
+    __shared__ float dsum[kGatherWaves * kGatherPairs][kGatherTex];
+    extern __shared__ float stage_s[];   // with a wide level: kGatherPairs x kWideRow floats per wave
     int li = 0;   // this block's level (uniform)
     while (li + 1 < G.n && (int)blockIdx.x >= G.start[li + 1]) li++;
-    const int level = G.lv[li];
+    const int level = G.lv[li], blk0 = (int)blockIdx.x - G.start[li];
     const DevLevel& L = m.lv[level];
     const int rate = rate0 && level == 0;
     float* const zq_copy = G.zq_copy[li];
-    const int j = threadIdx.x % kGatherTex, q = threadIdx.x / kGatherTex;
-    const int t = ((int)blockIdx.x - G.start[li]) * kGatherTex + j;
-    const bool live = t < L.W * L.H;
-    const int tt = live ? t : 0;
-    const int tx = tt % L.W, ty = tt / L.W;
+    // the pairs k0 .. k0 + kn - 1 (their sums d(k)) on channel c of texel (tx, ty), after the gradient so far; after the last
+    // pair the channel's Adam step
+    auto channel = [&](int tx, int ty, int c, int k0, int kn, auto d) {
+        const size_t i = (size_t)(L.off + ((long long)ty * L.W + tx) * L.C + c);
+        const int blk = (ty / 8) * dct_bw + tx / 8;
+        float gc = (first && k0 == 0) ? 0.0f : grad[i];
+#pragma unroll 4
+        for (int kk = 0; kk < kn; kk++) {
+            const float ei = eps[(size_t)(k0 + kk) * m.nz + i];
+            gc = __builtin_fmaf(d(kk) * scale, ei, gc);
+            if (rate) {
+                const int32_t db = dbits[(size_t)(k0 + kk) * dct_n + (size_t)blk * L.C + c];
+                gc = __builtin_fmaf(__fmul_rn(__fmul_rn(rate_scale, (float)db), scale), ei, gc);
+            }
+        }
+        grad[i] = gc;
+        if (adam && k0 + kn >= K) {
+            adam_at(z, zm, zv, i, gc, lr, c1, c2);
+            if (zq_copy) zq_copy[i] = z[i];   // a level the decode copy takes as it is
+        }
+    };
+    if (G.mode[li] == kUnit) {   // a thread per texel; a sum of one value (from +0, as the longer ones)
+        const int t = blk0 * threads + (int)threadIdx.x;
+        if (t >= L.W * L.H) return;
+        for (int c = 0; c < L.C; c++)
+            channel(t % L.W, t / L.W, c, 0, K, [&](int kk) { return 0.0f + dpix[(size_t)kk * m.npix + t]; });
+        return;
+    }
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, j = lane % kGatherTex, q = lane / kGatherTex;
+    const int tiles = (L.W + kGatherTex - 1) / kGatherTex, ty = blk0 / tiles, tx = (blk0 - ty * tiles) * kGatherTex + j;
+    const bool live = tx < L.W;
     const int* R = ranges + L.rng;
-    const int x0 = R[tx], x1 = R[L.W + tx], y0 = R[2 * L.W + ty], y1 = R[2 * L.W + L.H + ty];
-    const long long base = L.off + (long long)tt * L.C;
-    const int blk = (ty / 8) * dct_bw + tx / 8;
-    for (int k0 = 0; k0 < K; k0 += kGatherPairs) {
-        const int k = k0 + q;
-        if (live && k < K) {
-            // the rectangle's values in raster order, loaded in groups and then added in order (the loads of
-            // a group overlap; the sum stays one chain). A slot past the rectangle's end adds +0, which
-            // leaves the sum as it is: the sum starts at +0 and a rounded sum is -0 only when both operands
-            // are, so it is never -0. Rectangles up to 16 wide go in groups of kGatherRun values across row
-            // ends, wider ones a row at a time in runs of 16; a one-pixel rectangle is one load.
-            const float* dp = dpix + (size_t)k * m.npix;
-            const int fw = x1 - x0, n = fw * (y1 - y0);
-            float d = 0.0f;
-            if (n == 1) {
-                d += dp[(size_t)y0 * m.W + x0];
-            } else if (fw <= 16) {
-                int row = y0, col = 0;   // position of the group's first slot
-                for (int s = 0; s < n; s += kGatherRun) {
-                    float v[kGatherRun];
-                    int r = row, cc = col;
+    const int y0 = R[2 * L.W + ty], y1 = R[2 * L.W + L.H + ty];
+    const int x0 = live ? R[tx] : m.W, x1 = live ? R[L.W + tx] : 0;   // (a texel that no pixel reads has x0 >= x1)
+    const int round = kGatherPairs * (threads >> 6);
+    for (int k0 = 0; k0 < K; k0 += round) {
+        const int kw = k0 + kGatherPairs * wave, k = kw + q;   // this wave's first pair, this lane's
+        float d = 0.0f;
+        if (!Wide || G.mode[li] == kNarrow) {
+            if (k < K && x0 < x1 && y0 < y1) {
+                // the rectangle's values in raster order, loaded in groups of kGatherRun across row ends and then added in
+                // order (the loads of a group overlap; the sum stays one chain). A slot past the rectangle's end adds +0, which
+                // leaves the sum as it is: the sum starts at +0 and a rounded sum is -0 only when both operands
+                // are, so it is never -0.
+                const float* dp = dpix + (size_t)k * m.npix;
+                const int fw = x1 - x0, n = fw * (y1 - y0);
+                if (n == 1) {
+                    d += dp[(size_t)y0 * m.W + x0];
+                } else {
+                    int row = y0, col = 0;   // position of the group's first slot
+                    for (int s = 0; s < n; s += kGatherRun) {
+                        float v[kGatherRun];
+                        int r = row, cc = col;
 #pragma unroll
-                    for (int i = 0; i < kGatherRun; i++) {
-                        v[i] = s + i < n ? dp[(size_t)r * m.W + x0 + cc] : 0.0f;
-                        if (++cc == fw) { cc = 0; r++; }
+                        for (int i = 0; i < kGatherRun; i++) {
+                            v[i] = s + i < n ? dp[(size_t)r * m.W + x0 + cc] : 0.0f;
+                            if (++cc == fw) { cc = 0; r++; }
+                        }
+                        row = r; col = cc;
+#pragma unroll
+                        for (int i = 0; i < kGatherRun; i++) d += v[i];
                     }
-                    row = r; col = cc;
-#pragma unroll
-                    for (int i = 0; i < kGatherRun; i++) d += v[i];
-                }
-            } else {
-                // runs of 16 in raster order (a row's last run padded with +0), two buffers: the next run's loads are
-                // in flight while the current run is added
-                float va[16], vb[16];
-                auto load_run = [&](float (&v)[16], int py, int px) {
-                    const float* rw = dp + (size_t)py * m.W;
-#pragma unroll
-                    for (int i = 0; i < 16; i++) v[i] = px + i < x1 ? rw[px + i] : 0.0f;
-                };
-                auto step = [&](int& py, int& px) { px += 16; if (px >= x1) { px = x0; py++; } };
-                int py = y0, px = x0;
-                load_run(va, py, px);
-                while (true) {
-                    step(py, px);
-                    if (py < y1) load_run(vb, py, px);
-#pragma unroll
-                    for (int i = 0; i < 16; i++) d += va[i];
-                    if (py >= y1) break;
-                    step(py, px);
-                    if (py < y1) load_run(va, py, px);
-#pragma unroll
-                    for (int i = 0; i < 16; i++) d += vb[i];
-                    if (py >= y1) break;
                 }
             }
-            dsum[q][j] = d;
+        } else if (kw < K) {
+            // the columns under the tile's texels
+            int xa = x0 < x1 ? x0 : m.W, xb = x0 < x1 ? x1 : 0;
+            for (int o = 8; o > 0; o >>= 1) { xa = min(xa, __shfl_xor(xa, o, 64)); xb = max(xb, __shfl_xor(xb, o, 64)); }
+            xa = __builtin_amdgcn_readfirstlane(xa); xb = __builtin_amdgcn_readfirstlane(xb);
+            // kWideCols columns of a row of the wave's pairs at a time (a step), in raster order, kAhead steps in flight; what
+            // lies past the columns asked for is copied too (buffer loads: past the image's end they read 0), never added
+            constexpr int kAhead = 3, kPer = kWideCols / 64;
+            float* const st = stage_s + wave * kGatherPairs * kWideRow;
+            const int wide = max(0, xb - xa), per_row = (wide + kWideCols - 1) / kWideCols, steps = per_row * max(0, y1 - y0);
+            float v[kAhead][kGatherPairs][kPer];
+            int lc = xa, ly = y0;   // the next step to load
+            auto load = [&](float (&b)[kGatherPairs][kPer]) {
+                const uint32_t at = 4u * ((uint32_t)ly * (uint32_t)m.W + (uint32_t)lc);
+#pragma unroll
+                for (int p = 0; p < kGatherPairs; p++) {
+                    const __amdgpu_buffer_rsrc_t rd = buffer_of(dpix + (size_t)min(kw + p, K - 1) * m.npix, 4u * (uint32_t)m.npix);
+#pragma unroll
+                    for (int s = 0; s < kPer; s++) b[p][s] = buffer_f32(rd, 4u * (uint32_t)(lane + 64 * s), at);
+                }
+                lc += kWideCols;
+                if (lc >= xb) { lc = xa; ly++; }
+            };
+#pragma unroll
+            for (int b = 0; b < kAhead; b++) if (b < steps) load(v[b]);
+            int cs = xa;
+            for (int n = 0; n < steps; n += kAhead)
+#pragma unroll
+                for (int b = 0; b < kAhead; b++) {
+                    if (n + b >= steps) break;
+#pragma unroll
+                    for (int p = 0; p < kGatherPairs; p++)
+#pragma unroll
+                        for (int s = 0; s < kPer; s++) st[p * kWideRow + lane + 64 * s] = v[b][p][s];
+                    wave_lds_fence();
+                    if (n + b + kAhead < steps) load(v[b]);
+                    const int c0 = max(x0, cs), cnt = min(x1, cs + kWideCols) - c0;
+                    const float* run = st + q * kWideRow + (c0 - cs);
+                    int s = 0;
+                    for (; s + 16 <= cnt; s += 16) {
+                        float a[16];
+#pragma unroll
+                        for (int i = 0; i < 16; i++) a[i] = run[s + i];
+#pragma unroll
+                        for (int i = 0; i < 16; i++) d += a[i];
+                    }
+                    for (; s < cnt; s++) d += run[s];
+                    wave_lds_fence();
+                    cs += kWideCols;
+                    if (cs >= xb) cs = xa;
+                }
         }
+        dsum[kGatherPairs * wave + q][j] = d;
         __syncthreads();
-        // the round's pairs in order on every channel of the texel (thread q takes channels q, q + 4, ...),
-        // the channel's gradient in a register; after the last round the channel's Adam step
-        if (live) {
-            const int kn = min(K, k0 + kGatherPairs) - k0;
-            const bool last = k0 + kGatherPairs >= K;
-            for (int c = q; c < L.C; c += kGatherPairs) {
-                const size_t i = (size_t)(base + c);
-                float gc = (first && k0 == 0) ? 0.0f : grad[i];
-                for (int kk = 0; kk < kn; kk++) {
-                    const float ei = eps[(size_t)(k0 + kk) * m.nz + i];
-                    gc = __builtin_fmaf(dsum[kk][j] * scale, ei, gc);
-                    if (rate) {
-                        const int32_t db = dbits[(size_t)(k0 + kk) * dct_n + (size_t)blk * L.C + c];
-                        gc = __builtin_fmaf(__fmul_rn(__fmul_rn(rate_scale, (float)db), scale), ei, gc);
-                    }
-                }
-                grad[i] = gc;
-                if (adam && last) {
-                    adam_at(z, zm, zv, i, gc, lr, c1, c2);
-                    if (zq_copy) zq_copy[i] = z[i];   // a level the decode copy takes as it is
-                }
-            }
-        }
+        // the round's pairs in order on every channel of the texel (thread (wave, q) takes channels 4 wave + q, + round, ...)
+        if (live)
+            for (int c = kGatherPairs * wave + q; c < L.C; c += round)
+                channel(tx, ty, c, k0, min(K - k0, round), [&](int kk) { return dsum[kk][j]; });
         __syncthreads();
     }
 }
@@ -200,14 +252,21 @@ void launch_lat_gather(Impl& I, unsigned mask, int k0, int K, float scale, bool 
     const float c1 = t > 0 ? 1.0f - powf(0.9f, (float)t) : 1.0f, c2 = t > 0 ? 1.0f - powf(0.999f, (float)t) : 1.0f;
     GatherLevels G{};
     size_t grid = 0;
-    for (int l = 0; l < I.d.nlev; l++)
-        if ((mask >> l) & 1u) {
-            G.lv[G.n] = l;
-            G.start[G.n] = (int)grid;
-            G.zq_copy[G.n] = l > 0 ? zq_rest : nullptr;
-            grid += (size_t)blocks_for((size_t)I.d.lv[l].W * I.d.lv[l].H, kGatherTex);
-            G.n++;
-        }
+    bool wide = false;
+    const int threads = 64 * std::min(kGatherWaves, (K + kGatherPairs - 1) / kGatherPairs);
+    auto mode = [&](int l) { return l == 0 && I.lv0_unit_cells ? kUnit : (I.lv_cols[l] > 16 ? kWide : kNarrow); };
+    for (int pass = 0; pass < 2; pass++)   // the wide levels' blocks first: they take longest
+        for (int l = 0; l < I.d.nlev; l++)
+            if (((mask >> l) & 1u) && (mode(l) == kWide) == (pass == 0)) {
+                G.lv[G.n] = l;
+                G.start[G.n] = (int)grid;
+                G.mode[G.n] = mode(l);
+                wide = wide || pass == 0;
+                G.zq_copy[G.n] = l > 0 ? zq_rest : nullptr;
+                grid += mode(l) == kUnit ? (size_t)blocks_for((size_t)I.d.lv[l].W * I.d.lv[l].H, threads)
+                                         : (size_t)blocks_for((size_t)I.d.lv[l].W, kGatherTex) * (size_t)I.d.lv[l].H;
+                G.n++;
+            }
     G.start[G.n] = (int)grid;
     LatAhead ah{};
     ah.eb = 1;
@@ -219,7 +278,7 @@ void launch_lat_gather(Impl& I, unsigned mask, int k0, int K, float scale, bool 
                 ah.lo = std::min<long long>(ah.lo, I.dm.lv[l].off);
                 ah.hi = std::max<long long>(ah.hi, I.dm.lv[l].off + (long long)I.d.lv[l].W * I.d.lv[l].H * I.d.lv[l].C);
             }
-        ah.eb = blocks_for((size_t)(ah.hi - ah.lo), kAheadPerBlock);
+        ah.eb = blocks_for((size_t)(ah.hi - ah.lo), 2 * threads);
         grid += (size_t)ah.eb * (size_t)ahead_K;
     }
     if (grid > 0x7fffffff) {
@@ -227,7 +286,8 @@ void launch_lat_gather(Impl& I, unsigned mask, int k0, int K, float scale, bool 
         exit(1);
     }
     ProfScope ps(I, "lat_gather");
-    hipLaunchKernelGGL(k_lat_gather, dim3((unsigned)grid), dim3(kGatherTex * kGatherPairs), 0, I.stream, I.dm, G, K,
+    hipLaunchKernelGGL((wide ? k_lat_gather<true> : k_lat_gather<false>), dim3((unsigned)grid), dim3(threads),
+                       wide ? (size_t)threads / 64 * kGatherPairs * kWideRow * sizeof(float) : 0, I.stream, I.dm, G, K,
                        scale, I.dpix, I.eps_lat,
                        I.ranges, rate ? 1 : 0, I.ddct.rate_scale, I.ddct.BW, I.ddct.n, rate ? I.dct_dbits + (size_t)k0 * I.ddct.n : nullptr,
                        I.zgrad, k0 == 0 ? 1 : 0, t > 0 ? 1 : 0, I.z, I.zm,

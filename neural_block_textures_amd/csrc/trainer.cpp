@@ -303,6 +303,8 @@ bool Trainer::init(const ModelDesc& d, const float* z, const float* p, const flo
         }
         ranges.insert(ranges.end(), xb.begin(), xb.end()); ranges.insert(ranges.end(), xe.begin(), xe.end());
         ranges.insert(ranges.end(), yb.begin(), yb.end()); ranges.insert(ranges.end(), ye.begin(), ye.end());
+        I.lv_cols[l] = 0;
+        for (int x = 0; x < L.W; x++) I.lv_cols[l] = std::max(I.lv_cols[l], xe[x] - xb[x]);
         if (l == 0) {   // level 0 with one pixel per texel (texel x covers exactly pixel x): the selector search's per-pixel form
             bool unit = L.nearest && L.W == d.W && L.H == d.H;
             for (int x = 0; unit && x < L.W; x++) unit = xb[x] == x && xe[x] == x + 1;

@@ -110,6 +110,7 @@ struct ntc_cuda::Trainer::Impl {
     int* ranges = nullptr;     // per level: xb[W] xe[W] yb[H] ye[H] (pixel footprint of each texel row / column)
     float* qat_grid = nullptr; // 9 x 257
     int* qat_bits = nullptr;   // MAX_CH
+    int lv_cols[ntc_hip::kMaxLevels] = {};   // the most pixel columns that read one texel of each level
     bool lv0_unit_cells = false;   // level 0 nearest at the image's size: every texel's cell is its own pixel
     bool valu_only = false;        // instrumentation: every stage on the VALU kernels (ntc_trainer_set_matrix_cores)
 
