@@ -124,9 +124,10 @@ size_t ntc_trainer_debug_last_dl(const ntc_trainer* t, double* dl, size_t cap) {
     return v.size();
 }
 size_t ntc_trainer_debug_last_zgrad(const ntc_trainer* t, float* g, size_t cap) {
-    std::vector<float> v; t->t.debug_last_zgrad(v);
-    if (g) memcpy(g, v.data(), std::min(cap, v.size()) * sizeof(float));
-    return v.size();
+    auto& I = *t->t.im;
+    const size_t n = (size_t)I.nz;
+    if (g && cap) ntc_hip::read_back(I, { { g, I.zgrad, std::min(cap, n) * sizeof(float) } });
+    return n;
 }
 
 size_t ntc_trainer_debug_last_dpix(const ntc_trainer* t, float* d, size_t cap) {
@@ -146,8 +147,7 @@ size_t ntc_trainer_debug_last_losses(const ntc_trainer* t, double* lplus, double
     const size_t m = std::min(cap, n);
     const int chunks = (I.last_M + I.last_chunk - 1) / I.last_chunk;
     std::vector<double> part((size_t)2 * n * chunks);
-    NTC_CHECK(hipMemcpyAsync(part.data(), I.part, part.size() * sizeof(double), hipMemcpyDeviceToHost, I.stream));
-    NTC_CHECK(hipStreamSynchronize(I.stream));
+    ntc_hip::read_back(I, { { part.data(), I.part, part.size() * sizeof(double) } });
     const double norm = 3.0 * (double)I.d.wsum * (double)I.last_M;
     for (size_t i = 0; i < m; i++) {
         double a = 0.0, b = 0.0;
@@ -160,10 +160,7 @@ size_t ntc_trainer_debug_last_losses(const ntc_trainer* t, double* lplus, double
 size_t ntc_trainer_debug_last_wgrad(const ntc_trainer* t, float* g, size_t cap) {
     auto& I = *t->t.im;
     const size_t n = (size_t)I.P;
-    if (g && cap) {
-        NTC_CHECK(hipMemcpyAsync(g, I.wgrad, std::min(cap, n) * sizeof(float), hipMemcpyDeviceToHost, I.stream));
-        NTC_CHECK(hipStreamSynchronize(I.stream));
-    }
+    if (g && cap) ntc_hip::read_back(I, { { g, I.wgrad, std::min(cap, n) * sizeof(float) } });
     return n;
 }
 size_t ntc_abi_sizeof(const char* name) {

@@ -3,6 +3,8 @@
 //
 // Reference semantics (main.cpp): MlpTrainer::draw_batch 1825-1833, MlpTrainer::step 1836-1876,
 // MlpTrainer::step_fd 1890-1920, Adam::step 1799-1809, Decoder::decode_full 1712-1718.
+#include <string.h>
+
 #include "kern_decode.hpp"
 #include "jit.hpp"
 #include "shapes.hpp"
@@ -261,7 +263,45 @@ __global__ void __launch_bounds__(kTPB) k_debug_gauss(NoiseFix nt, uint64_t head
     if (i < n) out[i] = gauss_at(nt, head, index0 + i);
 }
 
+struct HostSegs {
+    int n;
+    const uint32_t* src[4];
+    uint32_t* dst[4];
+    unsigned words[4];
+};
+__global__ void __launch_bounds__(kTPB) k_to_host(HostSegs s) {
+    for (int q = 0; q < s.n; q++)
+        for (unsigned i = blockIdx.x * kTPB + threadIdx.x; i < s.words[q]; i += gridDim.x * kTPB) s.dst[q][i] = s.src[q][i];
+}
+
 // ---------------------------------------------------------------- launchers
+void read_back(Impl& I, std::initializer_list<HostSeg> segs) {
+    size_t total = 0;
+    bool words = segs.size() <= 4;
+    for (const HostSeg& g : segs) { total += g.bytes; words = words && g.bytes % 4 == 0; }
+    if (!words || total > kHostBytes || !I.host) {
+        for (const HostSeg& g : segs)
+            if (g.bytes) NTC_CHECK(hipMemcpyAsync(g.dst, g.src, g.bytes, hipMemcpyDeviceToHost, I.stream));
+        NTC_CHECK(hipStreamSynchronize(I.stream));
+        return;
+    }
+    std::lock_guard<std::mutex> lock(I.host_mu);
+    HostSegs h{};
+    size_t at = 0;
+    for (const HostSeg& g : segs) {
+        h.src[h.n] = (const uint32_t*)g.src; h.dst[h.n] = I.host + at; h.words[h.n] = (unsigned)(g.bytes / 4);
+        at += g.bytes / 4;
+        h.n++;
+    }
+    if (at) {
+        hipLaunchKernelGGL(k_to_host, dim3((unsigned)std::min<size_t>(blocks_for(at, kTPB), 64)), dim3(kTPB), 0, I.stream, h);
+        NTC_CHECK(hipGetLastError());
+    }
+    NTC_CHECK(hipStreamSynchronize(I.stream));
+    int q = 0;
+    for (const HostSeg& g : segs) { if (g.bytes) memcpy(g.dst, h.dst[q], g.bytes); q++; }
+}
+
 void launch_fill(Impl& I, float* p, size_t n, float v) {
     if (!n) return;
     hipLaunchKernelGGL(k_fill, dim3(blocks_for(n, kTPB)), dim3(kTPB), 0, I.stream, p, n, v);

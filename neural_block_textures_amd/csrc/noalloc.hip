@@ -90,8 +90,7 @@ void decode_error_noalloc_impl(Impl& I, const float* z_host, int ew, int eh, dou
     hipLaunchKernelGGL(k_sse_totals, dim3(1), dim3(256), 0, I.stream, sp, written, tot);
     NTC_CHECK(hipGetLastError());
     unsigned long long h[4];
-    NTC_CHECK(hipMemcpyAsync(h, tot, sizeof(h), hipMemcpyDeviceToHost, I.stream));
-    NTC_CHECK(hipStreamSynchronize(I.stream));
+    read_back(I, { { h, tot, sizeof(h) } });
     const int T = I.d.nout / 3;
     const double np = (double)npx;
     double ws = 0.0;

@@ -141,8 +141,7 @@ void decode_error_impl(Impl& I, const float* z_host, int ew, int eh, double* tex
     }
     const size_t written = launch_decode_sse(I, zsrc, ew, eh, part);
     std::vector<unsigned long long> h(written * 4);
-    NTC_CHECK(hipMemcpyAsync(h.data(), part, h.size() * sizeof(unsigned long long), hipMemcpyDeviceToHost, I.stream));
-    sync(I);
+    read_back(I, { { h.data(), part, h.size() * sizeof(unsigned long long) } });
     NTC_CHECK(ntc_hip::ntc_free(part));
     const int T = I.d.nout / 3;
     const double npix = (double)ew * eh;
@@ -204,6 +203,7 @@ Trainer::~Trainer() {
         dev_free(I.qes_dev); dev_free(I.qgrid);
         dev_free(I.zpost); dev_free(I.st_part); dev_free(I.st_keys); dev_free(I.st_hist); dev_free(I.st_dct); dev_free(I.st_sse);
         dev_free(I.dct_sym); dev_free(I.dct_code); dev_free(I.dct_step); dev_free(I.dct_bits); dev_free(I.dct_dbits); dev_free(I.dct_tn); dev_free(I.dct_probe_code); dev_free(I.dct_gain);
+        if (I.host) (void)hipHostFree(I.host);
         (void)hipStreamDestroy(I.stream);
     }
     delete im;
@@ -284,6 +284,7 @@ bool Trainer::init(const ModelDesc& d, const float* z, const float* p, const flo
     if (!noise_fix_for_device(I.device, I.noise, why)) return false;
     if (!noalloc_scratch_setup(I.device, why)) return false;
     NTC_CHECK(hipStreamCreateWithFlags(&I.stream, hipStreamNonBlocking));
+    NTC_CHECK(hipHostMalloc((void**)&I.host, kHostBytes, hipHostMallocDefault));
 
     // ---- model description
     I.npix = (size_t)d.W * d.H;
@@ -426,9 +427,7 @@ void Trainer::upload_model(const float* z, const float* p) {
 
 void Trainer::download_model(float* z, float* p) {
     Impl& I = *im;
-    NTC_CHECK(hipMemcpyAsync(z, I.z, I.nz * sizeof(float), hipMemcpyDeviceToHost, I.stream));
-    NTC_CHECK(hipMemcpyAsync(p, I.w, I.P * sizeof(float), hipMemcpyDeviceToHost, I.stream));
-    sync(I);
+    read_back(I, { { z, I.z, I.nz * sizeof(float) }, { p, I.w, I.P * sizeof(float) } });
 }
 
 void Trainer::set_qes(const QesDesc& q, const float* grid, size_t grid_n) {
@@ -574,9 +573,7 @@ void Trainer::mlp_stats(double& batch_loss, double& diff_std) {
     if (I.last_N == 0) { batch_loss = 0; diff_std = 0; return; }
     if (!I.last_fd) {
         std::vector<double> dl(I.last_N), lsum(I.last_N);
-        NTC_CHECK(hipMemcpyAsync(dl.data(), I.dl, I.last_N * sizeof(double), hipMemcpyDeviceToHost, I.stream));
-        NTC_CHECK(hipMemcpyAsync(lsum.data(), I.lsum, I.last_N * sizeof(double), hipMemcpyDeviceToHost, I.stream));
-        sync(I);
+        read_back(I, { { dl.data(), I.dl, I.last_N * sizeof(double) }, { lsum.data(), I.lsum, I.last_N * sizeof(double) } });
         double mean = 0, mean2 = 0, lmean = 0;
         for (int i = 0; i < I.last_N; i++) { mean += dl[i]; mean2 += dl[i] * dl[i]; lmean += lsum[i]; }
         mean /= I.last_N; mean2 /= I.last_N; lmean /= I.last_N;
@@ -585,9 +582,7 @@ void Trainer::mlp_stats(double& batch_loss, double& diff_std) {
     } else {
         std::vector<double> dl(I.P);
         double l0 = 0;
-        NTC_CHECK(hipMemcpyAsync(dl.data(), I.dl, I.P * sizeof(double), hipMemcpyDeviceToHost, I.stream));
-        NTC_CHECK(hipMemcpyAsync(&l0, I.lsum, sizeof(double), hipMemcpyDeviceToHost, I.stream));
-        sync(I);
+        read_back(I, { { dl.data(), I.dl, I.P * sizeof(double) }, { &l0, I.lsum, sizeof(double) } });
         double ss = 0;
         for (int j = 0; j < I.P; j++) ss += dl[j] * dl[j];
         diff_std = sqrt(ss / I.P);
@@ -685,20 +680,17 @@ void Trainer::print_stats(int qbits, int ew, int eh, ::ntc_print_stats* out) {
 void Trainer::debug_last_batch(std::vector<int>& bidx) const {
     Impl& I = *im;
     bidx.resize(I.last_M);
-    if (I.last_M) NTC_CHECK(hipMemcpyAsync(bidx.data(), I.bidx, I.last_M * sizeof(int), hipMemcpyDeviceToHost, I.stream));
-    sync(I);
+    read_back(I, { { bidx.data(), I.bidx, I.last_M * sizeof(int) } });
 }
 void Trainer::debug_last_dl(std::vector<double>& dl) const {
     Impl& I = *im;
     dl.resize(I.last_N);
-    if (I.last_N) NTC_CHECK(hipMemcpyAsync(dl.data(), I.dl, I.last_N * sizeof(double), hipMemcpyDeviceToHost, I.stream));
-    sync(I);
+    read_back(I, { { dl.data(), I.dl, I.last_N * sizeof(double) } });
 }
 void Trainer::debug_last_zgrad(std::vector<float>& g) const {
     Impl& I = *im;
     g.resize(I.nz);
-    NTC_CHECK(hipMemcpyAsync(g.data(), I.zgrad, I.nz * sizeof(float), hipMemcpyDeviceToHost, I.stream));
-    sync(I);
+    read_back(I, { { g.data(), I.zgrad, I.nz * sizeof(float) } });
 }
 
 }   // namespace ntc_cuda

@@ -17,7 +17,9 @@
 #include <stdio.h>
 #include <stdlib.h>
 
+#include <initializer_list>
 #include <map>
+#include <mutex>
 #include <string>
 #include <vector>
 
@@ -141,6 +143,11 @@ struct ntc_cuda::Trainer::Impl {
     std::vector<long long> st_counts, st_dct_counts;
     std::vector<float> st_lohi;
 
+    // read_back's landing place: pinned host memory that the device writes (kHostBytes, allocated at init, the trainer's
+    // own; the lock serves callers that read one trainer from several threads)
+    uint32_t* host = nullptr;
+    std::mutex host_mu;
+
     int mlp_t = 0, lat_t = 0, lat_step_no = 0;
     int last_N = 0, last_M = 0, last_chunk = 1;
     bool last_fd = false;
@@ -211,6 +218,14 @@ void launch_timed(void (*kern)(P...), Impl& I, dim3 grid, dim3 block, size_t shm
 // C library cannot be reproduced
 bool noise_fix_for_device(int device, NoiseFix& out, std::string& why);
 std::vector<uint32_t> noise_fix_summary(const std::vector<uint32_t>& fix);
+
+// Copies each segment from the device to the host and waits for the stream. Up to kHostBytes in all (whole 4-byte words) a
+// kernel writes them to the trainer's pinned host memory and the host copies them from there: one launch and one wait. A
+// copy to pageable memory stages itself and waits for each segment: a step's statistics and gradient took 43 us more than
+// the step (MI355X), 15 us more now. Larger ones are plain copies.
+struct HostSeg { void* dst; const void* src; size_t bytes; };
+constexpr size_t kHostBytes = (size_t)256 << 10;
+void read_back(Impl& I, std::initializer_list<HostSeg> segs);
 
 // kernels_mlp.hip
 void launch_fill(Impl& I, float* p, size_t n, float v);
