@@ -304,4 +304,29 @@ __device__ __forceinline__ void split_hidden(const SplitWeights<S>& W, h8v f, fl
     }
 }
 
+// split_hidden of N tiles, a layer of every tile at a time: their matrix and VALU instructions are independent
+template <class S, int N>
+__device__ __forceinline__ void split_hidden_n(const SplitWeights<S>& W, const h8v (&f)[N], float k, float neg, h8v (&b)[N][SplitShape<S>::kB]) {
+    using Q = MfmaShape<S>;
+    using P = SplitShape<S>;
+    f4v acc[N][Q::kHt];
+#pragma unroll
+    for (int s = 0; s < P::kS1; s++)
+#pragma unroll
+        for (int n = 0; n < N; n++)
+#pragma unroll
+            for (int ot = 0; ot < Q::kHt; ot++) acc[n][ot] = mfma_h(W.a1[ot][s], f[n], s == 0 ? W.c1[ot] : acc[n][ot]);
+#pragma unroll
+    for (int n = 0; n < N; n++) split_act<S>(acc[n], k, neg, b[n]);
+    if constexpr (Q::kNL > 1) {
+        f4v a2[N][Q::kHt];
+#pragma unroll
+        for (int n = 0; n < N; n++)
+#pragma unroll
+            for (int ot = 0; ot < Q::kHt; ot++) a2[n][ot] = split_dot<S>(W.ah[ot], b[n], W.ch[ot]);
+#pragma unroll
+        for (int n = 0; n < N; n++) split_act<S>(a2[n], k, neg, b[n]);
+    }
+}
+
 }   // namespace ntc_hip
