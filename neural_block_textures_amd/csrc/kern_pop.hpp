@@ -987,35 +987,16 @@ constexpr int qat_occupancy() {
 // activation of act<Act>: the reference adds the float terms in double with its own activation, so a
 // choice can differ from the reference's only between candidates whose losses agree to a few float
 // roundings (the reference's own check accepts such rounding ties, main.cpp:3143-3144).
+// The search on the 64 pixels from base (tile t: pixels base + 16 t + j) of one wave, on the 32-bit instructions.
 // UnitCw: every channel weight is 1, so a candidate's error terms are d d (fused into the sum where a lane holds several)
-template <class S, int Act, bool Clamp, bool UnitCw = false>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(qat_occupancy<S, Act>()))) k_qat_mfma(DevModel m, const float* __restrict__ w, float* __restrict__ zdec,
-                                                 const float* __restrict__ tgt, const int* __restrict__ qat_bits,
-                                                 const float* __restrict__ grid) {
+template <class S, int Act, bool Clamp, bool UnitCw>
+__device__ __forceinline__ void qat_round(const DevModel& m, const MfmaWeights<S>& W, float ak, const float (&cw)[4], float* __restrict__ zdec,
+                                          const float* __restrict__ tgt, const int* __restrict__ qat_bits, const float* __restrict__ grid,
+                                          int base, int lane, float* tl, float* vo, float* sums) {
     using Q = MfmaShape<S>;
     constexpr int NO = Q::kNout, C0 = S::kC0;
-    const int lane = tid_x() & 63, wave = __builtin_amdgcn_readfirstlane(tid_x() >> 6), i16 = lane & 15, g = lane >> 4;
-    constexpr bool kVOut = valu_out<S>();   // the output layer on the VALU: output g of pixel j in lane (g, j)
-    // each wave's LDS exchanges (in place of lane swaps): the tile operands, the VALU output layer's
-    // reduce-scatters of both candidates, the candidates' pixel sums
-    constexpr int kWaveLds = kTilesLds<S> + (kVOut ? 2 * kVoTile : 0) + kSumsLds;
-    __shared__ __attribute__((aligned(16))) float lds[4 * kWaveLds];
-    float* const tl = lds + wave * kWaveLds;
-    float* const vo = tl + kTilesLds<S>;
-    float* const sums = vo + (kVOut ? 2 * kVoTile : 0);
-    MfmaWeights<S> W;
-    mfma_load<S>(W, w, lane);
-    if constexpr (!Clamp) scale_output<S>(W, kNegLog2e);
-    if constexpr (Act == kActFold) scale_hidden<S>(W, fold_scale(m.leak));
-    const float ak = act_k_of<Act>(m);
-    float cw[4];
-    if constexpr (kVOut) {
-#pragma unroll
-        for (int r = 0; r < 4; r++) cw[r] = (r == 0 && g < NO) ? m.cw[g] : 0.0f;
-    } else {
-        lane_cw<S>(m.cw, g, cw);
-    }
-    const int base = bid_x() * 256 + wave * 64;   // tile t: pixels base + 16 t + j
+    constexpr bool kVOut = valu_out<S>();
+    const int i16 = lane & 15, g = lane >> 4;
     float f[S::kMaxIn];
     {
         const int pr = min(base + lane, m.npix - 1);
@@ -1132,6 +1113,218 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(qat_oc
             if (g == 0 && p < m.npix) zdec[m.lv[0].off + (size_t)p * m.lv[0].C + c] = win_v;
         }
     }
+}
+
+template <class S, int Act, bool Clamp, bool UnitCw = false>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(qat_occupancy<S, Act>()))) k_qat_mfma(DevModel m, const float* __restrict__ w, float* __restrict__ zdec,
+                                                 const float* __restrict__ tgt, const int* __restrict__ qat_bits,
+                                                 const float* __restrict__ grid) {
+    using Q = MfmaShape<S>;
+    constexpr int NO = Q::kNout;
+    const int lane = tid_x() & 63, wave = __builtin_amdgcn_readfirstlane(tid_x() >> 6), g = lane >> 4;
+    constexpr bool kVOut = valu_out<S>();   // the output layer on the VALU: output g of pixel j in lane (g, j)
+    // each wave's LDS exchanges (in place of lane swaps): the tile operands, the VALU output layer's
+    // reduce-scatters of both candidates, the candidates' pixel sums
+    constexpr int kWaveLds = kTilesLds<S> + (kVOut ? 2 * kVoTile : 0) + kSumsLds;
+    __shared__ __attribute__((aligned(16))) float lds[4 * kWaveLds];
+    float* const tl = lds + wave * kWaveLds;
+    float* const vo = tl + kTilesLds<S>;
+    float* const sums = vo + (kVOut ? 2 * kVoTile : 0);
+    MfmaWeights<S> W;
+    mfma_load<S>(W, w, lane);
+    if constexpr (!Clamp) scale_output<S>(W, kNegLog2e);
+    if constexpr (Act == kActFold) scale_hidden<S>(W, fold_scale(m.leak));
+    const float ak = act_k_of<Act>(m);
+    float cw[4];
+    if constexpr (kVOut) {
+#pragma unroll
+        for (int r = 0; r < 4; r++) cw[r] = (r == 0 && g < NO) ? m.cw[g] : 0.0f;
+    } else {
+        lane_cw<S>(m.cw, g, cw);
+    }
+    qat_round<S, Act, Clamp, UnitCw>(m, W, ak, cw, zdec, tgt, qat_bits, grid, bid_x() * 256 + wave * 64, lane, tl, vo, sums);
+}
+
+// ---- The selector search on the 16-bit matrix instructions with operands in two parts, for the shapes k_pop_split takes and
+// 0 <= leak <= 1. As k_qat_mfma, with blocks that stay on the chip as k_lat_split's: a wave takes 64 pixels at a time. The
+// searched inputs are left out of the first layer's operands (zeros in their places); each tile's first layer is formed once,
+// the other searched channels' terms and a candidate's are added to it in 32 bits, one fused multiply-add each. A candidate
+// then takes the layers after the first: 9 matrix instructions of 16 cycles for the 32-wide, 12-output models where the
+// 32-bit ones are 24 of 32. The winners are written when all of a round's losses are numbers; a round with a NaN is left as
+// it was and searched in 32 bits at the end (qat_round), the launch giving a wave at most 64 rounds.
+// material512, two channels of four values (MI355X): 73 -> 38 us.
+// (a wave per SIMD fewer than k_pop_split with more than one searched channel, whose first-layer weights are in registers too)
+constexpr int qat_waves(int nin, int H, int nout, int c0) { return split_waves(nin, H, nout) - (c0 > 1 && H <= 48 ? 1 : 0); }
+template <class S, bool Clamp, bool UnitCw>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(qat_waves(S::kNin, S::kH, S::kNout, S::kC0)))) k_qat_split(DevModel m, const float* __restrict__ w, float* __restrict__ zdec,
+                                                 const float* __restrict__ tgt, const int* __restrict__ qat_bits,
+                                                 const float* __restrict__ grid, int blocks) {
+    using Q = MfmaShape<S>;
+    using P = SplitShape<S>;
+    constexpr int NO = Q::kNout, RO = out_regs<S>(), C0 = S::kC0, kEx = 64 * split_inputs(Q::kIn);
+    constexpr bool kVOut = valu_out<S>();
+    constexpr int NT = kVOut ? NO : RO;
+    static_assert(kTilesLds<S> <= kEx, "the 32-bit search's tile operands fit");
+    __shared__ unsigned par_s[SplitLds<S>::kWords];
+    __shared__ __attribute__((aligned(16))) float lds[4][kEx + (kVOut ? 2 * kVoTile : 0) + kSumsLds];
+    const int lane = tid_x() & 63, wave = __builtin_amdgcn_readfirstlane(tid_x() >> 6), i16 = lane & 15, g = lane >> 4;
+    float* const ex = lds[wave];
+    float* const vo = ex + kEx;
+    float* const sums = vo + (kVOut ? 2 * kVoTile : 0);
+    const SplitScale sc = split_stage_plain<S>(m, w, Clamp ? 1.0 : kNegLog2eD, par_s);
+    SplitWeights<S> W;
+    split_load<S>(W, par_s, lane);
+    const float ak = in_vgpr(act_k_of<kActFold>(m)), neg = in_vgpr(-1.0f), inv = in_vgpr(sc.inv);
+    // the first layer's weights of the searched inputs for this lane's units, with the layer's factors
+    float w1[C0][Q::kHt][4];
+    {
+        const double b = split_factors(sc, m.fold_c, 1.0).w1 * kSplitFeat;
+#pragma unroll
+        for (int c = 0; c < C0; c++)
+#pragma unroll
+            for (int ot = 0; ot < Q::kHt; ot++)
+#pragma unroll
+                for (int r = 0; r < 4; r++) {
+                    const int u = unit_of<Q>(ot, 4 * g + r);
+                    const float v = (float)((double)w[min(u, Q::kH - 1) * Q::kIn + c] * b);
+                    w1[c][ot][r] = u < Q::kH ? v : 0.0f;
+                }
+    }
+    float cw[NT];
+#pragma unroll
+    for (int r = 0; r < NT; r++) {
+        cw[r] = 0.0f;
+#pragma unroll
+        for (int c = 0; c < NO; c++)
+            if ((kVOut ? r : out_at<S>(g, r)) == c) cw[r] = m.cw[c];
+    }
+    constexpr bool kUnit = UnitCw && (kVOut || NO == 4 * RO);
+    const int R = (m.npix + 63) >> 6;
+    unsigned long long again = 0;   // rounds that had a NaN
+    int n = 0;
+    for (int rd = bid_x() * 4 + wave; rd < R; rd += 4 * blocks, n++) {
+        const int base = 64 * rd;
+        float f[S::kMaxIn];
+        {
+            const int pr = min(base + lane, m.npix - 1);
+            features<S>(m, PlainLatent{ zdec }, pr % m.W, pr / m.W, f);
+        }
+        float own[C0];      // the lane's own pixel's channels and their grid indices
+        int cur_own[C0];
+#pragma unroll
+        for (int c = 0; c < C0; c++) {
+            own[c] = f[c]; cur_own[c] = qat_index(f[c], qat_bits[c]);
+            f[c] = 0.0f;
+        }
+        split_write<S>(f, neg, (u4v*)ex, lane);
+        wave_lds_fence();
+        float win[4][C0];
+        bool bad = false;
+#pragma unroll
+        for (int t = 0; t < 4; t++) {
+            float tt[NT];
+            const int pr = min(base + 16 * t + i16, m.npix - 1);
+#pragma unroll
+            for (int r = 0; r < NT; r++) tt[r] = tgt[(size_t)pr * NO + (kVOut ? r : max(out_at<S>(g, r), 0))];
+            const h8v b1 = split_read<S>((const u4v*)ex, 16 * t + i16, g);
+            f4v s0[Q::kHt];
+#pragma unroll
+            for (int ot = 0; ot < Q::kHt; ot++) {
+                s0[ot] = mfma_h(W.a1[ot][0], b1, W.c1[ot]);
+                if constexpr (P::kS1 > 1) s0[ot] = mfma_h(W.a1[ot][1], b1, s0[ot]);
+            }
+#pragma unroll
+            for (int c = 0; c < C0; c++) win[t][c] = __int_as_float(__builtin_amdgcn_ds_bpermute((16 * t + i16) << 2, __float_as_int(own[c])));
+#pragma unroll
+            for (int c = 0; c < C0; c++) {
+                const int levels = (1 << qat_bits[c]) - 1;
+                const float* gv = grid + qat_bits[c] * 257;
+                const int cur = __builtin_amdgcn_ds_bpermute((16 * t + i16) << 2, cur_own[c]);
+                f4v sb[Q::kHt];   // without channel c
+#pragma unroll
+                for (int ot = 0; ot < Q::kHt; ot++) {
+                    sb[ot] = s0[ot];
+#pragma unroll
+                    for (int q = 0; q < C0; q++)
+                        if (q != c)
+#pragma unroll
+                            for (int r = 0; r < 4; r++) sb[ot][r] = __builtin_fmaf(w1[q][ot][r], win[t][q], sb[ot][r]);
+                }
+                // the running minimum as in qat_round: the current value first, then the others in ascending order, strict <
+                float cur_l = 0.0f, best_l = __builtin_inff(), cur_v = 0.0f, best_v = 0.0f;
+                for (int kc = 0; kc <= levels; kc += 2) {
+                    const float gc[2] = { gv[kc], gv[kc + 1] };
+                    float lv[2];
+#pragma unroll
+                    for (int v = 0; v < 2; v++) {
+                        f4v a1[Q::kHt];
+#pragma unroll
+                        for (int ot = 0; ot < Q::kHt; ot++)
+#pragma unroll
+                            for (int r = 0; r < 4; r++) a1[ot][r] = __builtin_fmaf(w1[c][ot][r], gc[v], sb[ot][r]);
+                        h8v b[P::kB];
+                        split_act<S>(a1, ak, neg, b);
+                        if constexpr (Q::kNL > 1) {
+                            f4v a2[Q::kHt];
+#pragma unroll
+                            for (int ot = 0; ot < Q::kHt; ot++) a2[ot] = split_dot<S, true>(W.ah[ot], b, W.ch[ot]);
+                            split_act<S>(a2, ak, neg, b);
+                        }
+                        const f4v o = split_dot<S, true>(W.ao[0], b, W.co);   // (at most 4 outputs: lane group 0 holds them)
+                        lv[v] = 0.0f;
+#pragma unroll
+                        for (int r = 0; r < NT; r++) {
+                            const float s = o[r] * inv;
+                            if constexpr (Clamp) bad |= !not_nan_bits(s);
+                            const float d = out_of<S>(s, Clamp) - tt[r];
+                            lv[v] = kUnit ? __builtin_fmaf(d, d, lv[v]) : __builtin_fmaf(cw[r], __fmul_rn(d, d), lv[v]);
+                        }
+                    }
+                    float ls[2];
+                    if constexpr (kVOut) {
+#pragma unroll
+                        for (int v = 0; v < 2; v++) ls[v] = __int_as_float(__builtin_amdgcn_ds_bpermute(i16 << 2, __float_as_int(lv[v])));
+                    } else {
+                        group_sums(lv[0], lv[1], sums, g, i16, ls[0], ls[1]);
+                    }
+#pragma unroll
+                    for (int v = 0; v < 2; v++) {
+                        const float l = ls[v];
+                        const bool is_cur = kc + v == cur, better = !is_cur && l < best_l;
+                        bad |= !not_nan_bits(l);
+                        cur_l = is_cur ? l : cur_l;
+                        cur_v = is_cur ? gc[v] : cur_v;
+                        best_l = better ? l : best_l;
+                        best_v = better ? gc[v] : best_v;
+                    }
+                }
+                win[t][c] = best_l < cur_l ? best_v : cur_v;
+            }
+        }
+        wave_lds_fence();
+        if (__builtin_amdgcn_ballot_w64(bad) != 0) {
+            again |= 1ull << n;
+            continue;
+        }
+#pragma unroll
+        for (int t = 0; t < 4; t++) {
+            const int p = base + 16 * t + i16;
+            if (g == 0 && p < m.npix)
+#pragma unroll
+                for (int c = 0; c < C0; c++) zdec[m.lv[0].off + (size_t)p * m.lv[0].C + c] = win[t][c];
+        }
+    }
+    if (again == 0) return;
+    MfmaWeights<S> F;
+    mfma_load<S>(F, w, lane);
+    if constexpr (!Clamp) scale_output<S>(F, kNegLog2e);
+    scale_hidden<S>(F, fold_scale(m.leak));
+    float cw4[4];
+#pragma unroll
+    for (int r = 0; r < 4; r++) cw4[r] = kVOut ? ((r == 0 && g < NO) ? m.cw[min(g, NO - 1)] : 0.0f) : (r < NT ? cw[r < NT ? r : 0] : 0.0f);
+    n = 0;
+    for (int rd = bid_x() * 4 + wave; rd < R; rd += 4 * blocks, n++)
+        if ((again >> n) & 1ull) qat_round<S, kActFold, Clamp, false>(m, F, ak, cw4, zdec, tgt, qat_bits, grid, 64 * rd, lane, ex, vo, sums);
 }
 
 }   // namespace ntc_hip

@@ -234,6 +234,24 @@ void launch_lat_pair(Impl& I, int K, float sigma, unsigned mask) {
 }
 
 void launch_qat_mfma(Impl& I) {
+    if (split_pays(I.dm.nin, I.dm.nl) && I.dm.leak >= 0.0f && I.dm.leak <= 1.0f) {
+        // as many blocks as fit the chip; more where a wave would have over 64 rounds (its mask of rounds to search again)
+        const size_t rounds = (I.npix + 63) / 64;
+        const size_t fill = std::max((size_t)I.cus * qat_waves(I.dm.nin, I.dm.hidden[0], I.dm.nout, I.dm.lv[0].C), (rounds + 255) / 256);
+        const unsigned blocks = (unsigned)std::min(fill, (rounds + 3) / 4);
+        if (I.jit) {
+            jit_launch(k_qat_split<ShapeMaterial, false, false>, I, "k_qat_split", I.dm.clamp_out ? "true, false" : "false, false", dim3(blocks),
+                       dim3(256), 0, I.dm, I.w, I.zdec, I.tgt, I.qat_bits, I.qat_grid, (int)blocks);
+        } else dispatch_shape(I.dm, [&](auto s) {
+            using S = decltype(s);
+            if constexpr (SplitShape<S>::kOk) {
+                auto kern = I.dm.clamp_out ? k_qat_split<S, true, false> : (unit_cw(I) ? k_qat_split<S, false, true> : k_qat_split<S, false, false>);
+                hipLaunchKernelGGL(kern, dim3(blocks), dim3(256), 0, I.stream, I.dm, I.w, I.zdec, I.tgt, I.qat_bits, I.qat_grid, (int)blocks);
+            }
+        });
+        NTC_CHECK(hipGetLastError());
+        return;
+    }
     if (I.jit) {
         const float leak = I.dm.leak;
         const int act = leak >= 0.0f && leak <= 1.0f ? kActFold : kActAny;
@@ -247,12 +265,8 @@ void launch_qat_mfma(Impl& I) {
         using S = decltype(s);
         if constexpr (MfmaShape<S>::kOk)
         {
-            const float leak = I.dm.leak;
-            const bool fold = leak >= 0.0f && leak <= 1.0f, unit = unit_cw(I);
-            auto kern = I.dm.clamp_out ? (fold ? (unit ? k_qat_mfma<S, kActFold, true, true> : k_qat_mfma<S, kActFold, true, false>)
-                                               : k_qat_mfma<S, kActAny, true>)
-                                       : (fold ? (unit ? k_qat_mfma<S, kActFold, false, true> : k_qat_mfma<S, kActFold, false, false>)
-                                               : k_qat_mfma<S, kActAny, false>);
+            // (every listed shape with 0 <= leak <= 1 is the split kernel's)
+            auto kern = I.dm.clamp_out ? k_qat_mfma<S, kActAny, true> : k_qat_mfma<S, kActAny, false>;
             hipLaunchKernelGGL(kern, dim3((unsigned)((I.npix + 255) / 256)), dim3(256), 0, I.stream, I.dm, I.w, I.zdec, I.tgt,
                                I.qat_bits, I.qat_grid);
         }

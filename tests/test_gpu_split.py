@@ -150,3 +150,45 @@ def test_split_latent_range(orc, name):
     p[n1 + h * h:n2] *= s
     p[n2:n2 + lay.nout * h] /= s
     latent(orc, lay, z * s, p, tgt, 3, sigma=0.05 * 2.0 ** 14)
+
+
+@pytest.mark.parametrize("name", ["material", "material_clamp", "chief1_36", "mat_qat_36", "image3_27", "jit_mfma_28", "dct_plane"])
+@pytest.mark.parametrize("scale", [1.0, 2.0 ** 14])
+def test_split_selector_search(orc, name, scale):
+    """the selector search on the split kernel against the oracle's, over image sizes around a wave's 64 pixels, on ordinary
+    models and on ones whose hidden values pass the 16-bit range (large features of the other level): the same choices, but for
+    texels whose candidates' losses agree to 1e-6 (main.cpp:3143-3144)"""
+    from neural_block_textures_amd import synth
+    base = LAYOUTS[name]
+    for W, H in ((1, 1), (63, 1), (65, 3), (52, 41)):
+        lay = Layout(**{k: getattr(base, k) for k in base.__dataclass_fields__})
+        lay.W, lay.H = W, H
+        lay.levels = [(W, H, base.levels[0][2], True)] + [(max(1, W * w // base.W), max(1, H * h // base.H), c, near)
+                                                          for w, h, c, near in base.levels[1:]]
+        z, p, tgt = data(lay, 28)
+        grid, C0 = synth.qat_grid(), lay.levels[0][2]
+        bits = [2 + (c % 2) for c in range(C0)]
+        n0 = W * H * C0
+        lv0 = z[:n0].reshape(-1, C0)
+        for c in range(C0):
+            lv0[:, c] = synth.qat_snap(lv0[:, c], bits[c], grid)
+        if scale != 1.0:
+            nin, h, s = lay.nin, lay.hidden[0], np.float32(scale)
+            z[n0:] *= s
+            n1, n2 = h * nin + h, h * nin + h + h * h + h
+            w1 = p[:h * nin].reshape(h, nin)
+            w1[:, :C0] *= s                      # the searched inputs keep their share of the first layer
+            p[h * nin:n1] *= s
+            p[n1 + h * h:n2] *= s
+            p[n2:n2 + lay.nout * h] /= s
+        tr = trainer(lay, z, p, tgt, qat_bits=bits, qat_grid=grid)
+        tr.qat_search()
+        zg, zc = tr.download_model()[0], z.copy()
+        orc.qat_search(lay, p, zc, tgt, bits, grid)
+        assert np.array_equal(zg[n0:], z[n0:])
+        diff = np.nonzero((zg[:n0] != zc[:n0]).reshape(-1, C0).any(1))[0]
+        say("selectors", name, W, H, "scale", scale, "differ", diff.size, "of", W * H)
+        if diff.size:
+            ec, eg = orc.decode_err(lay, p, zc, tgt), orc.decode_err(lay, p, zg, tgt)
+            assert (np.abs(ec[diff] - eg[diff]) <= 1e-6 * np.maximum(ec[diff], eg[diff]) + 1e-12).all()
+        tr.close()
