@@ -113,7 +113,8 @@ void launch_pop_eval_fd(Impl& I, float h, int M, int chunk, int chunks) {
 }
 
 // The split population kernel takes every step that the matrix cores take, of the shapes it has an operand layout for
-// (split_pays). Against the 32-bit kernel on the MI355X: see k_pop_split. NTC_HIP_POP_PAIR=0 keeps k_pop_mfma for every step.
+// (split_pays). Against the 32-bit kernel on the MI355X: see k_pop_split. NTC_HIP_POP_PAIR=0 keeps the
+// 32-bit kernels for every step of a listed shape: k_pop_mfma, and k_lat_pair_mfma for its latent pairs.
 bool pop_split_possible(const Impl& I) {
     if (!pop_on_matrix_cores(I)) return false;
     const char* env = getenv("NTC_HIP_POP_PAIR");
@@ -198,8 +199,12 @@ static int lat_rounds_for(const Impl& I, int most, int K) {
     return most;
 }
 
-// (k_lat_pair_mfma, for the shapes the split kernel does not take, is compiled at init only)
-bool lat_pair_on_matrix_cores(const Impl& I) { return pop_on_matrix_cores(I) && (I.jit || split_pays(I.dm.nin, I.dm.nl)); }
+bool lat_pair_on_matrix_cores(const Impl& I) { return pop_on_matrix_cores(I); }
+
+// k_lat_split for the models whose population is split, and for every shape compiled at init that it takes (no other
+// latent pair kernel is compiled for those); k_lat_pair_mfma for the rest, which in a default run are shapes compiled at
+// init, and with NTC_HIP_POP_PAIR=0 the listed ones: that run's gradients then come from 32-bit kernels throughout.
+static bool lat_pair_split(const Impl& I) { return split_pays(I.dm.nin, I.dm.nl) && (I.jit || I.pop_split); }
 
 void launch_lat_pair(Impl& I, int K, float sigma, unsigned mask) {
     ProfScope ps(I, "lat_pair");
@@ -207,7 +212,7 @@ void launch_lat_pair(Impl& I, int K, float sigma, unsigned mask) {
         launch_lat_pair_valu(I, K, sigma, mask);
         return;
     }
-    if (split_pays(I.dm.nin, I.dm.nl)) {
+    if (lat_pair_split(I)) {
         // as many blocks as fit the chip, or as 64-pixel rounds fill
         const size_t rounds = (I.npix + 63) / 64 * (size_t)K;
         const unsigned blocks = (unsigned)std::min<size_t>((size_t)I.cus * split_waves(I.dm.nin, I.dm.hidden[0], I.dm.nout), (rounds + 3) / 4);
@@ -225,11 +230,20 @@ void launch_lat_pair(Impl& I, int K, float sigma, unsigned mask) {
         NTC_CHECK(hipGetLastError());
         return;
     }
-    // a shape compiled at init (every listed one is the split kernel's)
-    const int rounds = lat_rounds_for(I, lat_rounds_of(I.dm.nin), K), pix = 256 * rounds;
-    jit_launch(k_lat_pair_mfma<ShapeMaterial, kActFold, false>, I, "k_lat_pair_mfma",
-               std::to_string((int)kActFold) + (I.dm.clamp_out ? ", true" : ", false"), dim3((unsigned)((I.npix + pix - 1) / pix), K), dim3(256), 0,
-               I.dm, I.w, I.zdec, I.eps_lat, I.tgt, sigma, mask, I.dpix, rounds);
+    if (I.jit) {
+        const int rounds = lat_rounds_for(I, lat_rounds_of(I.dm.nin), K), pix = 256 * rounds;
+        jit_launch(k_lat_pair_mfma<ShapeMaterial, kActFold, false>, I, "k_lat_pair_mfma",
+                   std::to_string((int)kActFold) + (I.dm.clamp_out ? ", true" : ", false"), dim3((unsigned)((I.npix + pix - 1) / pix), K), dim3(256), 0,
+                   I.dm, I.w, I.zdec, I.eps_lat, I.tgt, sigma, mask, I.dpix, rounds);
+    } else dispatch_shape(I.dm, [&](auto s) {
+        using S = decltype(s);
+        if constexpr (MfmaShape<S>::kOk) {
+            const int rounds = lat_rounds_for(I, lat_rounds<S>(), K), pix = 256 * rounds;
+            auto kern = I.dm.clamp_out ? k_lat_pair_mfma<S, kActFold, true> : k_lat_pair_mfma<S, kActFold, false>;
+            hipLaunchKernelGGL(kern, dim3((unsigned)((I.npix + pix - 1) / pix), K), dim3(256), 0, I.stream, I.dm, I.w, I.zdec, I.eps_lat, I.tgt,
+                               sigma, mask, I.dpix, rounds);
+        }
+    });
     NTC_CHECK(hipGetLastError());
 }
 
