@@ -192,3 +192,16 @@ def test_split_selector_search(orc, name, scale):
             ec, eg = orc.decode_err(lay, p, zc, tgt), orc.decode_err(lay, p, zg, tgt)
             assert (np.abs(ec[diff] - eg[diff]) <= 1e-6 * np.maximum(ec[diff], eg[diff]) + 1e-12).all()
         tr.close()
+
+
+@pytest.mark.parametrize("name", ["rgb_16x2", "two_level", "material", "material_clamp", "chief1_36", "large"])
+def test_latent_pairs_on_the_32_bit_instructions(orc, monkeypatch, name):
+    """the same latent steps with NTC_HIP_POP_PAIR=0 (k_lat_pair_mfma on the listed shapes), at the same bar"""
+    monkeypatch.setenv("NTC_HIP_POP_PAIR", "0")
+    base = LAYOUTS[name]
+    for W, H, K in ((1, 1, 1), (65, 1, 1), (50, 41, 5)):
+        lay = Layout(**{k: getattr(base, k) for k in base.__dataclass_fields__})
+        lay.W, lay.H = W, H
+        lay.levels = [(max(1, W * w // base.W), max(1, H * h // base.H), c, near) for w, h, c, near in base.levels]
+        z, p, tgt = data(lay, 26)
+        latent(orc, lay, z, p, tgt, K)
