@@ -329,19 +329,16 @@ __device__ __forceinline__ void split_stage(const PopSource& src, const SplitFac
     }
 }
 
-// Flat parameter k of a member staged in LDS as the 32-bit evaluation takes it (the layers' factors without their powers of
-// two): both parts' sum; hi alone where that is an infinity.
-template <class S>
-struct SplitParam32 {
-    const unsigned* lds;
-    SplitScale sc;
+// Parameter k of a member in 32 bits: w0 + s eps, one fused operation (main.cpp:1852-1856); central differences: w0 with weight
+// `hit` at w + s (main.cpp:1905).
+template <int From>
+struct MemberAt {
+    const float *w0, *eps;
+    float s;
+    int hit;
     __device__ __forceinline__ float operator()(int k) const {
-        using L = SplitLds<S>;
-        const int l = L::layer(k);
-        const unsigned v = lds[L::pos(k)];
-        if (L::bias(k)) return __uint_as_float(v) / (kSplitFeat * sc.s1 * (l > 0 ? sc.s2 : 1.0f) * (l > 1 ? sc.s3 : 1.0f));
-        const float h = (float)__builtin_bit_cast(_Float16, (unsigned short)v), lo = (float)__builtin_bit_cast(_Float16, (unsigned short)(v >> 16));
-        return ((v & 0x7fffu) == 0x7c00u ? h : h + lo) / (l == 0 ? sc.s1 : (l == 1 ? sc.s2 : sc.s3));
+        if constexpr (From == kSets) return k == hit ? w0[k] + s : w0[k];
+        else return __builtin_fmaf(s, eps[k], w0[k]);
     }
 };
 
@@ -363,7 +360,7 @@ struct SplitParam32 {
 // -> 0.16, 64-wide with 8192 pairs on 262144 slots 386 -> 119.
 // A lane adds its channel terms cw (d d) in float over a pass's slots, then into a double, as the other population kernels.
 // Values past the 16-bit range make NaN outputs (split_mlp.hpp), so a wave whose sum is a NaN evaluates its slots again in
-// 32 bits as k_pop_mfma does; with --clamp, where a NaN output becomes 0, the output pre-activations are tested.
+// 32 bits, from the 32-bit weights, as k_pop_mfma does; with --clamp, where a NaN output becomes 0, the output pre-activations are tested.
 template <class S>
 constexpr int split_u() { return valu_out<S>() ? 4 : 2; }
 // Tiles whose layers are evaluated together, so that one tile's activations stand between another's matrix instructions: all
@@ -488,10 +485,23 @@ __global__ void __launch_bounds__(64 * kPopWaves) __attribute__((amdgpu_waves_pe
         if (q + 1 < mine) pass(in1, in0, q + 1);
     }
     if (__builtin_amdgcn_ballot_w64(bad || !not_nan_bits_d(e)) != 0) {
-        // 32 bits: the wave's slots again, a 16-slot tile at a time, from the minibatch's 32-bit feature rows
+        // 32 bits: the wave's slots again, a 16-slot tile at a time, from the minibatch's 32-bit feature rows and the member's
+        // 32-bit weights, as k_pop_mfma evaluates them
         e = 0.0;
+        constexpr int Act = From == kSets ? kActMax : kActFold;
+        const float k32 = act_k_of<Act>(m);
+        float* const eg = src.eps + (size_t)pair * Q::kP;
+        if constexpr (From == kDraw) {
+            if (ch != 0) {   // (the chunk-0 block, which may not have run, writes the same values)
+                const uint64_t head = noise_head(src.seed, NS_MLP, src.step, (uint32_t)pair);
+                for (int k = lane; k < Q::kP; k += 64) eg[k] = gauss_at(src.nt, head, (uint64_t)k);
+                __threadfence_block();
+            }
+        }
         MfmaWeights<S> F;
-        mfma_load_from<S>(F, SplitParam32<S>{ mine_s, sc }, lane);
+        mfma_load_from<S>(F, MemberAt<From>{ src.w0, eg, sgn ? -src.sigma : src.sigma, pair }, lane);
+        if constexpr (!Clamp) scale_output<S>(F, kNegLog2e);
+        if constexpr (Act == kActFold) scale_hidden<S>(F, fold_scale(m.leak));
         const __amdgpu_buffer_rsrc_t r32 = buffer_of(feat, 4u * ((uint32_t)minibatch_rows(NIN) * (uint32_t)Mcap + (uint32_t)kMinibatchSlack));
         for (int q = 0; q < mine; q++)
             for (int u = 0; u < U; u++) {
@@ -501,7 +511,7 @@ __global__ void __launch_bounds__(64 * kPopWaves) __attribute__((amdgpu_waves_pe
 #pragma unroll
                 for (int ks = 0; ks < Q::kKs1; ks++)
                     b1[0][ks] = buffer_f32(r32, 4u * ((uint32_t)(4 * ks + g) * (uint32_t)Mcap + (uint32_t)i16), 4u * (uint32_t)st);
-                mfma_hidden<S, 1, kActFold>(F, b1, ak, x);
+                mfma_hidden<S, 1, Act>(F, b1, k32, x);
                 float ts = 0.0f;
                 if constexpr (kVOut) {
                     const float d = out_of<S>(valu_out_g<S>(F, x[0], vo_s + wave * kVoTile, g, i16), Clamp) -
@@ -759,29 +769,31 @@ template <class S>
 __device__ __forceinline__ SplitScale split_stage_plain(const DevModel& m, const float* __restrict__ w, double out, unsigned* __restrict__ lds) {
     using L = SplitLds<S>;
     constexpr int kP = MfmaShape<S>::kP, kN = (kP + 255) / 256;
-    __shared__ float top[4][3];
-    float v[kN], mx[3] = { 0.0f, 0.0f, 0.0f };
+    __shared__ SplitRange top[4][3];
+    float v[kN];
+    SplitRange r[3] = { { 0, 0, 0 }, { 0, 0, 0 }, { 0, 0, 0 } };
 #pragma unroll
     for (int q = 0; q < kN; q++) v[q] = w[min(tid_x() + 256 * q, kP - 1)];
+    const float fold = fold_scale(m.leak);
 #pragma unroll
     for (int q = 0; q < kN; q++) {
-        const int k = min(tid_x() + 256 * q, kP - 1);
-        const float a = L::bias(k) ? 0.0f : fabsf(v[q]);
+        const int k = tid_x() + 256 * q;
+        const bool b = k >= kP || L::bias(k);
 #pragma unroll
-        for (int l = 0; l < 3; l++) mx[l] = fmaxf(mx[l], L::layer(k) == l ? a : 0.0f);
+        for (int l = 0; l < 3; l++) r[l].add(!b && L::layer(k) == l ? v[q] : 0.0f, 0.0f, l == 2 ? (float)fabs(out) : fold);
     }
 #pragma unroll
-    for (int l = 0; l < 3; l++)
-        for (int o = 32; o > 0; o >>= 1) mx[l] = fmaxf(mx[l], __shfl_xor(mx[l], o, 64));
-    if ((tid_x() & 63) == 0)
-#pragma unroll
-        for (int l = 0; l < 3; l++) top[tid_x() >> 6][l] = mx[l];
+    for (int l = 0; l < 3; l++) {
+        r[l].add_wave();
+        if ((tid_x() & 63) == 0) top[tid_x() >> 6][l] = r[l];
+    }
     __syncthreads();
 #pragma unroll
-    for (int l = 0; l < 3; l++) mx[l] = fmaxf(fmaxf(top[0][l], top[1][l]), fmaxf(top[2][l], top[3][l]));
-    const float fold = fold_scale(m.leak);
-    SplitScale sc{ split_pow2(mx[0] * fold, kSplitExp[0]), MfmaShape<S>::kNL > 1 ? split_pow2(mx[1] * fold, kSplitExp[1]) : 1.0f,
-                   split_pow2(mx[2] * (float)fabs(out), kSplitExp[2]), 0.0f };
+    for (int l = 0; l < 3; l++) {
+        r[l] = top[0][l];
+        for (int q = 1; q < 4; q++) r[l].add(top[q][l]);
+    }
+    SplitScale sc{ split_pow2(r[0], kSplitExp[0]), split_pow2(r[1], kSplitExp[1]), split_pow2(r[2], kSplitExp[2]), 0.0f };
     sc.inv = 1.0f / (kSplitFeat * sc.s1 * sc.s2 * sc.s3);
     const SplitFactors f = split_factors(sc, m.fold_c, out);
 #pragma unroll
@@ -834,7 +846,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(split_
     constexpr int NO = Q::kNout, RO = out_regs<S>(), kEx = 64 * split_inputs(Q::kIn);   // floats of one member's exchange
     constexpr bool kVOut = valu_out<S>();
     constexpr int NT = kVOut ? NO : RO;
-    static_assert(2 * kTilesLds<S> <= 2 * kEx && (!kVOut || 2 * kVoTile + kSumsLds <= 2 * kEx), "the 32-bit evaluation's exchanges fit");
+    static_assert(2 * kTilesLds<S> <= 2 * kEx && 2 * kVoTile + kSumsLds <= 2 * kEx, "the 32-bit evaluation's exchanges fit");
     __shared__ unsigned par_s[SplitLds<S>::kWords];
     __shared__ __attribute__((aligned(16))) float ex_s[4][2 * kEx];
     __shared__ __attribute__((aligned(16))) float sum_s[kVOut ? 1 : 4][kVOut ? 4 : 256];

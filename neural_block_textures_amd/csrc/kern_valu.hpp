@@ -27,9 +27,8 @@ struct EpsJob {
 };
 
 // The minibatch slot by slot for the split population kernel (device_common.hpp, split_inputs), and the layers' power-of-two
-// scales (split_mlp.hpp), which block `block` finds: scales[l] brings layer l's largest possible member weight (|w| + 6
-// sigma, more than the draw reaches, times the layer's factor: fold for hidden layers, out for the output layer) below
-// 2^kSplitExp[l]. feat null: none.
+// scales (split_mlp.hpp), which block `block` finds from the weights' SplitRange (factors: fold for hidden layers, out for the
+// output layer). feat null: none.
 struct SplitJob {
     uint4* feat;
     float* tgt;
@@ -40,22 +39,22 @@ struct SplitJob {
 };
 
 __device__ inline void split_scales(const DevModel& m, const SplitJob& sj) {
-    __shared__ float red[kTPB / 64];
+    __shared__ SplitRange red[kTPB / 64];
     float total = kSplitFeat;
     if (threadIdx.x == 0) sj.scales[1] = 1.0f;   // (a single hidden layer has no second)
     int p = 0, in = m.nin;
     for (int l = 0; l <= m.nl; l++) {
         const bool last = l == m.nl;
         const int out = last ? m.nout : m.hidden[l];
-        float v = 0.0f;
-        for (int k = (int)threadIdx.x; k < out * in; k += kTPB) v = fmaxf(v, fabsf(sj.w[p + k]));
-        for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o, 64));
-        if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
+        SplitRange r{ 0, 0, 0 };
+        for (int k = (int)threadIdx.x; k < out * in; k += kTPB) r.add(sj.w[p + k], sj.sigma, last ? sj.out : sj.fold);
+        r.add_wave();
+        if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = r;
         __syncthreads();
-        v = red[0];
-        for (int q = 1; q < kTPB / 64; q++) v = fmaxf(v, red[q]);
+        r = red[0];
+        for (int q = 1; q < kTPB / 64; q++) r.add(red[q]);
         __syncthreads();
-        const float s = split_pow2((v + 6.0f * fabsf(sj.sigma)) * fabsf(last ? sj.out : sj.fold), kSplitExp[last ? 2 : l]);
+        const float s = split_pow2(r, kSplitExp[last ? 2 : l]);
         total *= s;
         if (threadIdx.x == 0) sj.scales[last ? 2 : l] = s;
         p += out * in + out; in = out;

@@ -13,11 +13,11 @@
 // cycles of VALU instructions).
 //
 // Range. 16-bit parts span 2^-24 .. 65504, so the layers are scaled by powers of two (SplitScale): the features by
-// kSplitFeat, each layer's weights to a largest value of 2^kSplitExp. Powers of two commute with every rounding and
-// with the activation, so they change no result; the lo parts of weights down to 2^-8 of their layer's largest then
-// keep all their bits, and the hidden values have room up to a few hundred. A value past the range becomes
-// an infinity and its lo part the opposite one, so every unit it feeds is a NaN: the kernel sees the NaN and
-// evaluates its slots again in 32 bits. Nothing is ever clipped.
+// kSplitFeat, each layer's weights by split_pow2 to a typical size of 1 (hidden layers) or 2^9. Powers of two commute with every
+// rounding and with the activation, so they change no result; the hidden values have room up to a few hundred. A value past the
+// range becomes an infinity and its lo part the opposite one, so every unit it feeds is a NaN: the kernel sees the NaN and
+// evaluates its slots again in 32 bits, from the 32-bit weights. So it does where a layer's weights are too far apart for the
+// parts (split_pow2). Nothing is ever clipped.
 //
 // Operand layout (measured on gfx950): lane l, half j of A holds A[l % 16][8 (l / 16) + j], of B holds
 // B[8 (l / 16) + j][l % 16]; C/D as the 32-bit instruction's. The 32 contraction slots are free to hold any input and
