@@ -27,8 +27,8 @@ constexpr int kMaxLevels = 3, kMaxPos = 16, kMaxOut = 12, kMaxHidden = 8, kMaxWi
 constexpr int kMinibatchSlack = 256;
 __host__ __device__ constexpr int minibatch_rows(int nin) { return 4 * ((nin + 3) / 4); }
 
-// The minibatch as the split population kernel reads it (split_mlp.hpp), slot by slot: the features times kSplitFeat in
-// two 16-bit parts, split_inputs(nin) hi parts then as many lo parts (zero past nin), and the targets, split_targets(nout)
+// The minibatch as the split population kernel reads it (split_mlp.hpp), slot by slot: the features in two 16-bit parts,
+// split_inputs(nin) hi parts then as many lo parts times kSplitLo (zero past nin), and the targets, split_targets(nout)
 // floats. Both arrays carry kSplitSlack slots past the last one.
 // At most 16 inputs: a first layer of more would need another operand layout (no compiled shape has them). At most two
 // hidden layers: the values of a third, scaled as the first two are, would leave the 16-bit range.
@@ -36,7 +36,9 @@ __host__ __device__ constexpr bool split_pays(int nin, int nl) { return nin <= 1
 __host__ __device__ constexpr int split_inputs(int nin) { return nin <= 8 ? 8 : 16; }
 __host__ __device__ constexpr int split_targets(int nout) { return nout <= 4 ? nout : 4 * ((nout + 3) / 4); }
 constexpr int kSplitSlack = 256;
-constexpr float kSplitFeat = 1.0f;
+// (features' lo parts are held times this, so that they are no 16-bit subnormals down to features of 2^-14; the weights that
+// meet them are divided by it)
+constexpr float kSplitLo = 2048.0f;
 // the typical exponent (split_pow2) that the weights of the first hidden layer, the second and the output layer are scaled to
 constexpr int kSplitExp[3] = { 0, 0, 9 };
 

@@ -794,7 +794,7 @@ __device__ __forceinline__ SplitScale split_stage_plain(const DevModel& m, const
         for (int q = 1; q < 4; q++) r[l].add(top[q][l]);
     }
     SplitScale sc{ split_pow2(r[0], kSplitExp[0]), split_pow2(r[1], kSplitExp[1]), split_pow2(r[2], kSplitExp[2]), 0.0f };
-    sc.inv = 1.0f / (kSplitFeat * sc.s1 * sc.s2 * sc.s3);
+    sc.inv = 1.0f / (sc.s1 * sc.s2 * sc.s3);
     const SplitFactors f = split_factors(sc, m.fold_c, out);
 #pragma unroll
     for (int q = 0; q < kN; q++) {
@@ -810,18 +810,22 @@ __device__ __forceinline__ SplitScale split_stage_plain(const DevModel& m, const
     return sc;
 }
 
-// A wave's 64 pixels' features f (lane: one pixel) split to t: per pixel split_inputs hi parts, then as many lo parts
+// A wave's 64 pixels' features f (lane: one pixel) split to t: per pixel split_inputs hi parts, then as many lo parts times
+// kSplitLo
 template <class S>
 __device__ __forceinline__ void split_write(const float (&f)[S::kMaxIn], float neg, u4v* __restrict__ t, int lane) {
     constexpr int N = split_inputs(S::kNin), C = N / 8;   // 16-byte pieces per part
+    const float neg_lo = neg * kSplitLo;
 #pragma unroll
     for (int q = 0; q < C; q++) {
         h2v hi[4], lo[4];
 #pragma unroll
         for (int j = 0; j < 4; j++) {
             const int i = 8 * q + 2 * j;
-            const float x = i < S::kNin ? f[i < S::kNin ? i : 0] * kSplitFeat : 0.0f, y = i + 1 < S::kNin ? f[i + 1 < S::kNin ? i + 1 : 0] * kSplitFeat : 0.0f;
-            split2(x, y, neg, hi[j], lo[j]);
+            const float x = i < S::kNin ? f[i < S::kNin ? i : 0] : 0.0f, y = i + 1 < S::kNin ? f[i + 1 < S::kNin ? i + 1 : 0] : 0.0f;
+            hi[j] = __builtin_convertvector((f2v){ x, y }, h2v);
+            lo[j] = __builtin_convertvector((f2v){ __builtin_fmaf((float)hi[j][0], neg_lo, x * kSplitLo),
+                                                   __builtin_fmaf((float)hi[j][1], neg_lo, y * kSplitLo) }, h2v);
         }
         u4v a, b;
 #pragma unroll
@@ -1190,7 +1194,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(qat_wa
     // the first layer's weights of the searched inputs for this lane's units, with the layer's factors
     float w1[C0][Q::kHt][4];
     {
-        const double b = split_factors(sc, m.fold_c, 1.0).w1 * kSplitFeat;
+        const double b = split_factors(sc, m.fold_c, 1.0).w1;
 #pragma unroll
         for (int c = 0; c < C0; c++)
 #pragma unroll

@@ -40,7 +40,7 @@ struct SplitJob {
 
 __device__ inline void split_scales(const DevModel& m, const SplitJob& sj) {
     __shared__ SplitRange red[kTPB / 64];
-    float total = kSplitFeat;
+    float total = 1.0f;
     if (threadIdx.x == 0) sj.scales[1] = 1.0f;   // (a single hidden layer has no second)
     int p = 0, in = m.nin;
     for (int l = 0; l <= m.nl; l++) {
@@ -97,9 +97,9 @@ __global__ void __launch_bounds__(kTPB) k_batch(DevModel m, uint64_t head, int M
             union { _Float16 h[2 * N]; uint4 q[N / 4]; } v;
 #pragma unroll
             for (int i = 0; i < N; i++) {
-                const float x = i < S::kNin ? f[i < S::kNin ? i : 0] * kSplitFeat : 0.0f;
+                const float x = i < S::kNin ? f[i < S::kNin ? i : 0] : 0.0f;
                 v.h[i] = (_Float16)x;
-                v.h[N + i] = (_Float16)(x - (float)v.h[i]);
+                v.h[N + i] = (_Float16)((x - (float)v.h[i]) * kSplitLo);
             }
 #pragma unroll
             for (int i = 0; i < N / 4; i++) sj.feat[(size_t)s * (N / 4) + i] = v.q[i];

@@ -12,10 +12,12 @@
 // of matrix and VALU instructions is close to the sum of both (measured: a matrix instruction of 16 cycles hides about 5
 // cycles of VALU instructions).
 //
-// Range. 16-bit parts span 2^-24 .. 65504, so the layers are scaled by powers of two (SplitScale): the features by
-// kSplitFeat, each layer's weights by split_pow2 to a typical size of 1 (hidden layers) or 2^9. Powers of two commute with every
-// rounding and with the activation, so they change no result; the hidden values have room up to a few hundred. A value past the
-// range becomes an infinity and its lo part the opposite one, so every unit it feeds is a NaN: the kernel sees the NaN and
+// Range. 16-bit parts span 2^-24 .. 65504, so the layers' weights are scaled by powers of two (SplitScale, split_pow2) to a
+// typical size of 1 (hidden layers) or 2^9. Powers of two commute with every rounding and with the activation, so they change no
+// result; the hidden values have room up to a few hundred, and keep both parts' bits down to 1/4. Features are not scaled, but
+// their lo parts are (kSplitLo), against weights divided by as much: with the lo parts of small features subnormal, latents of 0.01
+// gave gradients up to 1.7 and per-pixel latent differences up to 2.9 times as far from 64 bits as the 32-bit kernels. A value
+// past the range becomes an infinity and its lo part the opposite one, so every unit it feeds is a NaN: the kernel sees the NaN and
 // evaluates its slots again in 32 bits, from the 32-bit weights. So it does where a layer's weights are too far apart for the
 // parts (split_pow2). Nothing is ever clipped.
 //
@@ -121,7 +123,7 @@ struct SplitLds {
 // layers' powers of two, a bias with those of the layers before it.
 struct SplitFactors { double w1, w2, w3, b1, b2, b3; };
 __device__ __forceinline__ SplitFactors split_factors(const SplitScale& sc, float fold_c, double out) {
-    const double b = 1.0 / (1.0 + (double)fold_c), t1 = (double)sc.s1 * kSplitFeat, t2 = t1 * sc.s2;
+    const double b = 1.0 / (1.0 + (double)fold_c), t1 = sc.s1, t2 = t1 * sc.s2;
     return { b * sc.s1, b * sc.s2, out * sc.s3, b * t1, b * t2, out * t2 * sc.s3 };
 }
 
@@ -164,6 +166,9 @@ __device__ __forceinline__ void split_load(SplitWeights<S>& W, const unsigned* _
     const int i16 = lane & 15, g = lane >> 4;
     auto at = [&](bool ok, int k) { const unsigned v = lds[k]; return ok ? v : 0u; };
     auto bias = [&](bool ok, int k) { return __uint_as_float(at(ok, k)); };
+    // the weights of features' lo parts: of a power of two, so exact down to a scaled weight of 2^-3, then within 2^-25
+    const bool low = P::kS1 == 1 ? (g & 1) != 0 : g >= 2;
+    auto for_features = [&](h8v& a) { a *= (_Float16)(low ? 1.0f / kSplitLo : 1.0f); };
     // slots 2 j and 2 j + 1 of an operand from two parameters
     auto put = [&](h8v& a, int j, unsigned x, unsigned y, unsigned half) {
         u4v v = __builtin_bit_cast(u4v, a);
@@ -188,6 +193,8 @@ __device__ __forceinline__ void split_load(SplitWeights<S>& W, const unsigned* _
                 put(W.a1[ot][1], j, w[2 * j], w[2 * j + 1], kLo);
             }
         }
+#pragma unroll
+        for (int s = 0; s < P::kS1; s++) for_features(W.a1[ot][s]);
 #pragma unroll
         for (int r = 0; r < 4; r++) {
             const int ur = unit_of<Q>(ot, 4 * g + r);

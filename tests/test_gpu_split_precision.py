@@ -92,7 +92,7 @@ def population_errors(orc, monkeypatch, name, regime, path, seeds, batch):
     return e
 
 
-REGIMES = ["outlier_dead"]
+REGIMES = ["small", "outlier_dead"]
 
 
 def cases(names):
@@ -109,7 +109,7 @@ def test_population_no_further_from_64_bits(orc, monkeypatch, name, regime):
 @pytest.mark.parametrize("name,regime", cases(["rgb_16x2", "two_level", "material", "chief1_36", "jit_mfma_28", "one_24"]))
 def test_central_differences_no_further_from_64_bits(orc, monkeypatch, name, regime):
     split, full = population_errors(orc, monkeypatch, name, regime, "fd", 2, 1500)
-    assert split <= 1.1 * full
+    assert split <= 1.2 * full
 
 
 def latent_errors(orc, monkeypatch, name, regime, seeds, K=4):
