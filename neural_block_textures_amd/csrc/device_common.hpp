@@ -27,9 +27,8 @@ constexpr int kMaxLevels = 3, kMaxPos = 16, kMaxOut = 12, kMaxHidden = 8, kMaxWi
 constexpr int kMinibatchSlack = 256;
 __host__ __device__ constexpr int minibatch_rows(int nin) { return 4 * ((nin + 3) / 4); }
 
-// The minibatch as the split population kernel reads it (split_mlp.hpp), slot by slot: the features in two 16-bit parts,
-// split_inputs(nin) hi parts then as many lo parts times kSplitLo (zero past nin), and the targets, split_targets(nout)
-// floats. Both arrays carry kSplitSlack slots past the last one.
+// The minibatch as the split population kernel reads it (split_mlp.hpp), slot by slot: the features in two 16-bit parts, hi and
+// lo times kSplitLo (zero past nin), in the order of split_piece, and the targets, split_targets(nout) floats. Both arrays carry kSplitSlack slots past the last one.
 // At most 16 inputs: a first layer of more would need another operand layout (no compiled shape has them). At most two
 // hidden layers: the values of a third, scaled as the first two are, would leave the 16-bit range.
 __host__ __device__ constexpr bool split_pays(int nin, int nl) { return nin <= 16 && nl <= 2; }
@@ -39,8 +38,11 @@ constexpr int kSplitSlack = 256;
 // (features' lo parts are held times this, so that they are no 16-bit subnormals down to features of 2^-14; the weights that
 // meet them are divided by it)
 constexpr float kSplitLo = 2048.0f;
+// What half h of a slot's features holds, N = split_inputs(nin): below N the hi part of that input, N + i the lo part of input i.
+// 8 inputs: the hi parts, then the lo parts; 16: four hi parts and their lo parts at a time (a lane group's).
+__host__ __device__ constexpr int split_piece(int N, int h) { return N == 8 ? h : (h & 4 ? N : 0) + 4 * (h / 8) + (h & 3); }
 // the typical exponent (split_pow2) that the weights of the first hidden layer, the second and the output layer are scaled to
-constexpr int kSplitExp[3] = { 0, 0, 9 };
+constexpr int kSplitExp[3] = { 2, 0, 9 };
 
 // ---------------------------------------------------------------- model description
 struct DevLevel {
@@ -106,8 +108,18 @@ struct SplitRange {
         top = max(top, (int)(v >> 23));   // (255 for an infinity or a NaN)
     }
     __device__ __forceinline__ void add(const SplitRange& o) { sum += o.sum; n += o.n; top = max(top, o.top); }
-    __device__ __forceinline__ void add_wave() {   // over the wave's lanes
-        for (int o = 32; o > 0; o >>= 1) add(SplitRange{ __shfl_xor(sum, o, 64), __shfl_xor(n, o, 64), __shfl_xor(top, o, 64) });
+    // over the wave's lanes, each of at most 25 weights (sum and n then fit one word), without LDS
+    __device__ __forceinline__ void add_wave() {
+        int v = sum | n << 20, t = top;
+        add_lanes<0x111, 0xf>(v, t); add_lanes<0x112, 0xf>(v, t); add_lanes<0x114, 0xf>(v, t); add_lanes<0x118, 0xf>(v, t);   // row_shr 1, 2, 4, 8
+        add_lanes<0x142, 0xa>(v, t); add_lanes<0x143, 0xc>(v, t);                                                             // row_bcast 15, 31
+        v = __builtin_amdgcn_readlane(v, 63);
+        sum = v & 0xfffff; n = v >> 20; top = __builtin_amdgcn_readlane(t, 63);
+    }
+    template <int Ctrl, int Rows>
+    __device__ __forceinline__ static void add_lanes(int& v, int& t) {
+        v += __builtin_amdgcn_update_dpp(0, v, Ctrl, Rows, 0xf, false);
+        t = max(t, __builtin_amdgcn_update_dpp(0, t, Ctrl, Rows, 0xf, false));
     }
 };
 // The power of two in 2^-30 .. 2^30 that scales the layer: its mean exponent to e, or less where its largest weight would pass

@@ -4,9 +4,9 @@
 // The population evaluation (MlpTrainer::step's member losses, main.cpp:1848-1861) on the
 // matrix cores of gfx950, for the fixed shapes the matrix cores pay off for (MfmaShape::kOk) and
 // 0 <= leak <= 1; other models use the VALU kernel of kernels_mlp.hip. In an ES step the kernel
-// stages the pair's perturbed weights itself (no member weight sets in memory). ES steps of the shapes split_pays
-// takes run on k_pop_split (16-bit instructions, operands in two parts); central differences, and the ES steps of
-// the other shapes, on k_pop_mfma (32-bit instructions), which the following is about.
+// stages the pair's perturbed weights itself (no member weight sets in memory). The shapes split_pays takes run on k_pop_split
+// (16-bit instructions, operands in parts), ES steps and central differences; the other shapes on k_pop_mfma (32-bit
+// instructions), which the following is about.
 //
 // On this chip an FP32 matrix instruction and a VALU instruction do not run concurrently on a
 // SIMD (a 16x16x4 f32 step costs 32 cycles, a VALU instruction 4, and their mixes take the sum),
@@ -288,10 +288,16 @@ __global__ void __launch_bounds__(64 * kPopWaves) __attribute__((amdgpu_waves_pe
     }
 }
 
-// waves per SIMD the split kernel's register allocation aims at (more would spill)
+// Waves per SIMD that the split kernels' register allocation aims at. k_lat_split and k_qat_split: split_waves, at which several
+// shapes keep values in scratch. k_pop_split holds three parts of the weights: at three waves its loop over tiles reloads up to
+// 28 values a pass from scratch for the 36-wide models of more than 8 inputs and the 48-wide ones, at two none (512 pairs on 4096
+// slots, MI355X: 10-36-36-12 299 -> 118 us, 14-48-48-12 771 -> 147 us).
 constexpr int split_waves(int nin, int H, int nout) { return H > 48 ? 2 : ((nin <= 8 && H <= 32 && (nout > 4 || H <= 16)) ? 4 : 3); }
+constexpr int pop_split_waves(int nin, int H, int nout) { return H > 40 || (H > 32 && nin > 8) ? 2 : split_waves(nin, H, nout); }
 template <class S>
 constexpr int split_occupancy() { return split_waves(MfmaShape<S>::kIn, MfmaShape<S>::kH, MfmaShape<S>::kNout); }
+template <class S>
+constexpr int pop_split_occupancy() { return pop_split_waves(MfmaShape<S>::kIn, MfmaShape<S>::kH, MfmaShape<S>::kNout); }
 // the minibatch slot by slot (device_common.hpp, split_inputs) and the step's layer scales (split_mlp.hpp)
 struct SplitIn {
     const u4v* feat;
@@ -299,12 +305,13 @@ struct SplitIn {
     const float* scales;
 };
 
-// Stages both members of an ES pair in LDS (SplitLds): w0 + sigma eps, then w0 - sigma eps (main.cpp:1852-1856), in two
+// Stages both members of an ES pair in LDS (SplitLds): w0 + sigma eps, then w0 - sigma eps (main.cpp:1852-1856), in three
 // parts with their factors. The Gaussians are drawn here (kDraw: the chunk-0 block writes them for the update) or read
 // (kReadEps). Central differences (kSets): pair j < P is w0 with weight j at w + h and w - h (h = sigma; the 32-bit sums,
 // main.cpp:1905), pair P two copies of w0.
 template <class S, int From>
-__device__ __forceinline__ void split_stage(const PopSource& src, const SplitFactors f, int pair, int ch, unsigned* __restrict__ lds) {
+__device__ __forceinline__ void split_stage(const PopSource& src, const SplitFactors f, int pair, int ch, unsigned* __restrict__ lds,
+                                            unsigned short* __restrict__ last) {
     using L = SplitLds<S>;
     constexpr int kP = MfmaShape<S>::kP;
     const uint64_t head = noise_head(src.seed, NS_MLP, src.step, (uint32_t)pair);
@@ -324,8 +331,8 @@ __device__ __forceinline__ void split_stage(const PopSource& src, const SplitFac
         const int l = L::layer(k), at = L::pos(k);
         const bool b = L::bias(k);
         const double fw = l == 0 ? f.w1 : (l == 1 ? f.w2 : f.w3), fb = l == 0 ? f.b1 : (l == 1 ? f.b2 : f.b3), ff = b ? fb : fw;
-        lds[at] = split_param(wp, s, e, ff, b);
-        lds[L::kWords + at] = split_param(wm, -s, e, ff, b);
+        lds[at] = split_param(wp, s, e, ff, b, last[at]);
+        lds[L::kWords + at] = split_param(wm, -s, e, ff, b, last[L::kWords + at]);
     }
 }
 
@@ -342,25 +349,29 @@ struct MemberAt {
     }
 };
 
-// ---- The population on the 16-bit matrix instructions with 32-bit operands in two parts (split_mlp.hpp), for the shapes
-// of at most 16 inputs and two hidden layers: ES steps, and central differences (kSets), whose members it forms from the
-// weights themselves (no weight sets in memory).
+// ---- The population on the 16-bit matrix instructions with 32-bit operands in parts (split_mlp.hpp: weights in three, values in
+// two), for the shapes of at most 16 inputs and two hidden layers: ES steps, and central differences (kSets), whose members it
+// forms from the weights themselves (no weight sets in memory).
 //
 // Block (pair, chunk) has four waves: wave w evaluates member 2 pair + (w & 1) on the passes 2 q + (w >> 1) of the chunk's
 // slots, 32 slots a pass (two 16-slot tiles) for the models with more than 4 outputs, 64 (four tiles) for the others, whose
 // four output tiles meet in one accumulator so that every lane ends with the outputs of its own slot. A member's operands and
-// biases stay in VGPRs for the whole chunk (both parts of every weight: 32 VGPRs for the 32-wide models, 112 for the 64-wide
-// ones), so a pass reads only its inputs, the next pass's while it computes: 16 bytes of features per lane and tile and the
-// lane's targets, both laid out slot by slot by the minibatch launch.
-// What bounds it is the issue of matrix and VALU instructions, which hardly overlap: a 32-wide, 12-output tile takes 11
-// matrix instructions of 16 cycles and about 75 VALU ones (300 cycles: 2.5 each, conversions 4.5, exp2 and the reciprocal 8.6),
-// where the 32-bit instructions of k_pop_mfma take 28 of 32 cycles beside their VALU work; material512's population takes 530
-// cycles a tile, the staging of its members' weights among them. Whole launches against the 32-bit kernels (MI355X, ms):
-// material512 0.95 -> 0.47, two levels with 512 pairs on 65536 slots 1.57 -> 0.72, 36-wide with 777 pairs on 5001 slots 0.38
-// -> 0.16, 64-wide with 8192 pairs on 262144 slots 386 -> 119.
-// A lane adds its channel terms cw (d d) in float over a pass's slots, then into a double, as the other population kernels.
+// biases stay in VGPRs for the whole chunk, but for those of the widest models that SplitShape keeps in LDS, so a pass reads only
+// its inputs, the next pass's while it computes: 16 bytes of features per lane and tile and the lane's targets, both laid out slot
+// by slot by the minibatch launch.
+// What bounds it is the issue of matrix and VALU instructions, which hardly overlap: a 32-wide, 12-output tile takes 14
+// matrix instructions of 16 cycles and about 66 VALU ones (2.5 cycles each, conversions 4.5, exp2 and the reciprocal 8.6), where
+// the 32-bit instructions of k_pop_mfma take 28 of 32 cycles beside their VALU work. Whole launches, k_pop_mfma and
+// k_pop_split with weights in two parts and in three (MI355X, ms): material512 0.97 (its former pair-sharing kernel), 0.48, 0.51;
+// two levels with 512 pairs on 65536 slots 1.58, 0.72, 0.82; 36-wide with 777 pairs on 5001 slots 0.37, 0.145, 0.16; 64-wide with
+// 8192 pairs on 262144 slots 386, 119, 143.
+// A lane adds its channel terms cw (d d) in float over a pass's slots, then into a double, as the other population kernels;
+// central differences in double throughout (in float, their loss differences were 1.02 to 1.13 times as far from 64 bits as
+// k_pop_mfma's).
 // Values past the 16-bit range make NaN outputs (split_mlp.hpp), so a wave whose sum is a NaN evaluates its slots again in
-// 32 bits, from the 32-bit weights, as k_pop_mfma does; with --clamp, where a NaN output becomes 0, the output pre-activations are tested.
+// 32 bits, from the 32-bit weights, as k_pop_mfma does; with --clamp, where a NaN output becomes 0, the output pre-activations
+// are tested. A model of such values pays for both evaluations in every step: its hidden values, scaled as the weights are
+// (split_pow2), pass 65504.
 template <class S>
 constexpr int split_u() { return valu_out<S>() ? 4 : 2; }
 // Tiles whose layers are evaluated together, so that one tile's activations stand between another's matrix instructions: all
@@ -369,12 +380,19 @@ constexpr int split_u() { return valu_out<S>() ? 4 : 2; }
 template <class S>
 constexpr int split_together() { return MfmaShape<S>::kHt == 1 ? split_u<S>() : (MfmaShape<S>::kHt == 2 ? 2 : 1); }
 
+template <int From>
+struct SlotSum { using T = float; };
+template <>
+struct SlotSum<kSets> { using T = double; };
+
 template <class S, bool Clamp, int From, bool UnitCw>
-__global__ void __launch_bounds__(64 * kPopWaves) __attribute__((amdgpu_waves_per_eu(split_occupancy<S>()))) k_pop_split(DevModel m, PopSource src, int M, int Mcap,
+__global__ void __launch_bounds__(64 * kPopWaves) __attribute__((amdgpu_waves_per_eu(pop_split_occupancy<S>()))) k_pop_split(DevModel m, PopSource src, int M, int Mcap,
                                                             int chunk, int chunks, SplitIn in, const float* __restrict__ feat,
                                                             double* __restrict__ part) {
     using Q = MfmaShape<S>;
-    using P = SplitShape<S>;
+    // central differences: members one weight apart, so the reference's activation (see launch_pop_matrix)
+    constexpr int Act = From == kSets ? kActMax : kActFold;
+    using P = SplitShape<S, 3>;
     static_assert(P::kOk, "a shape the split kernel takes");
     constexpr int NIN = Q::kIn, NO = Q::kNout, RO = out_regs<S>(), U = split_u<S>();
     constexpr bool kVOut = valu_out<S>();
@@ -382,7 +400,10 @@ __global__ void __launch_bounds__(64 * kPopWaves) __attribute__((amdgpu_waves_pe
     constexpr int NT = kVOut ? NO : RO;                                  // target values a lane takes per read
     constexpr int TT = kVOut ? 1 : U;                                    // reads per pass
     __shared__ double red[kPopWaves];
-    __shared__ unsigned par_s[2 * SplitLds<S>::kWords];                  // the + member's parameters, then the - member's
+    // the + member's parameters, then the - member's, and their weights' last parts; then their operands that stay in LDS
+    constexpr int kWords = SplitLds<S>::kWords, kMem = 3 * kWords > 512 * P::kLdsOps ? 3 * kWords : 512 * P::kLdsOps;
+    __shared__ __attribute__((aligned(16))) unsigned par_s[kMem];
+    unsigned short* const last_s = (unsigned short*)(par_s + 2 * kWords);
     __shared__ __attribute__((aligned(16))) float vo_s[kVOut ? kPopWaves * kVoTile : 4];   // the 32-bit evaluation's output sums
     const int lane = tid_x() & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid_x() >> 6);
@@ -393,7 +414,7 @@ __global__ void __launch_bounds__(64 * kPopWaves) __attribute__((amdgpu_waves_pe
     const int mine = ((s1 - s0 + PS - 1) / PS - half + 1) >> 1;          // this wave's passes: 2 q + half, q < mine
     const uint32_t slots = (uint32_t)Mcap + (uint32_t)kSplitSlack;
     const __amdgpu_buffer_rsrc_t rf = buffer_of((const float*)in.feat, slots * (uint32_t)FB), rt = buffer_of(in.tgt, slots * 4u * TS);
-    const uint32_t fo = (uint32_t)(FB * i16 + 16 * (P::kS1 == 1 ? (g & 1) : g));
+    const uint32_t fo = (uint32_t)(FB * i16 + 16 * (P::kS1 == 1 ? (g == 1 ? 1 : 0) : g));
     const uint32_t to = kVOut ? 4u * (uint32_t)(TS * lane) : 4u * (uint32_t)(TS * i16 + RO * g);
     struct In { h8v f[U]; float t[TT][NT]; };
     auto load = [&](In& n, int q) {
@@ -408,12 +429,19 @@ __global__ void __launch_bounds__(64 * kPopWaves) __attribute__((amdgpu_waves_pe
     In in0, in1;
     load(in0, 0);
     const SplitScale sc = split_scale(in.scales);
-    split_stage<S, From>(src, split_factors(sc, m.fold_c, Clamp ? 1.0 : kNegLog2eD), pair, ch, par_s);
+    split_stage<S, From>(src, split_factors(sc, Act == kActMax ? 0.0f : m.fold_c, Clamp ? 1.0 : kNegLog2eD), pair, ch, par_s, last_s);
     __syncthreads();
-    const unsigned* const mine_s = par_s + sgn * SplitLds<S>::kWords;
-    SplitWeights<S> W;
-    split_load<S>(W, mine_s, lane);
-    const float ak = in_vgpr(act_k_of<kActFold>(m)), neg = in_vgpr(-1.0f), inv = in_vgpr(sc.inv);
+    SplitWeights<S, 3> W;
+    {
+        h8v kept[P::kLdsOps + 1];
+        split_load<S, 3>(W, par_s + sgn * kWords, last_s + sgn * kWords, lane, kept);
+        if constexpr (P::kLdsOps > 0) {
+            __syncthreads();
+            split_keep<S, 3>(W, kept, (h8v*)par_s + sgn * 64 * P::kLdsOps, half == 0, lane);
+            __syncthreads();
+        }
+    }
+    const float ak = in_vgpr(act_k_of<Act>(m)), neg = in_vgpr(-1.0f), inv = in_vgpr(sc.inv);
     // the channel weight of each of this lane's output registers (0 past the last output)
     float cw[NT];
 #pragma unroll
@@ -426,19 +454,24 @@ __global__ void __launch_bounds__(64 * kPopWaves) __attribute__((amdgpu_waves_pe
     constexpr bool kUnit = UnitCw && (kVOut || NO == 4 * RO);   // (padding outputs need their zero weight)
     double e = 0.0;
     bool bad = false;   // --clamp: an output pre-activation was a NaN
-    auto terms = [&](const f4v& o, const float (&t)[NT], float sum) {
+    // sum plus this lane's channel terms, in 32 bits; central differences, whose loss differences are small against the
+    // losses: in 64
+    using Sum = typename SlotSum<From>::T;
+    auto terms = [&](const f4v& o, const float (&t)[NT], Sum sum) {
 #pragma unroll
         for (int r = 0; r < NT; r++) {
             const float s = o[r] * inv;
             if constexpr (Clamp) bad |= !not_nan_bits(s);
             const float d = out_of<S>(s, Clamp) - t[r];
-            sum = __builtin_fmaf(kUnit ? d : __fmul_rn(cw[r], d), d, sum);
+            if constexpr (From == kSets) sum = __builtin_fma(kUnit ? (double)d : (double)cw[r] * (double)d, (double)d, sum);
+            else sum = __builtin_fmaf(kUnit ? d : __fmul_rn(cw[r], d), d, sum);
         }
         return sum;
     };
     auto pass = [&](In& c, In& n, int q) {
         q = __builtin_amdgcn_readfirstlane(q);
         load(n, q + 1 < mine ? q + 1 : q);
+        W.reload();
         const int s = s0 + PS * (2 * q + half);   // the pass's first slot
         if constexpr (kVOut) {
             f4v o = W.co;
@@ -448,11 +481,11 @@ __global__ void __launch_bounds__(64 * kPopWaves) __attribute__((amdgpu_waves_pe
                 h8v b[N][P::kB], fs[N];
 #pragma unroll
                 for (int n = 0; n < N; n++) fs[n] = c.f[u + n];
-                split_hidden_n<S, N>(W, fs, ak, neg, b);
+                split_hidden_n<S, 3, Act, N>(W, fs, ak, neg, b);
 #pragma unroll
-                for (int n = 0; n < N; n++) o = split_dot<S>(W.ao[u + n], b[n], o);
+                for (int n = 0; n < N; n++) o = split_dot_out<S, 3>(W, u + n, b[n], o);
             }
-            const float ts = terms(o, c.t[0], 0.0f);
+            const Sum ts = terms(o, c.t[0], 0);
             if (s + lane < s1) e += (double)ts;
         } else {
             f4v o[U];
@@ -462,19 +495,19 @@ __global__ void __launch_bounds__(64 * kPopWaves) __attribute__((amdgpu_waves_pe
                 h8v b[N][P::kB], fs[N];
 #pragma unroll
                 for (int n = 0; n < N; n++) fs[n] = c.f[u + n];
-                split_hidden_n<S, N>(W, fs, ak, neg, b);
+                split_hidden_n<S, 3, Act, N>(W, fs, ak, neg, b);
 #pragma unroll
-                for (int n = 0; n < N; n++) o[u + n] = split_dot<S>(W.ao[0], b[n], W.co);
+                for (int n = 0; n < N; n++) o[u + n] = split_dot_out<S, 3>(W, 0, b[n], W.co);
             }
             if (s + PS <= s1) {   // every slot inside the chunk (uniform)
-                float ts = 0.0f;
+                Sum ts = 0;
 #pragma unroll
                 for (int u = 0; u < U; u++) ts = terms(o[u], c.t[u], ts);
                 e += (double)ts;
             } else {
 #pragma unroll
                 for (int u = 0; u < U; u++) {
-                    const float ts = terms(o[u], c.t[u], 0.0f);
+                    const Sum ts = terms(o[u], c.t[u], 0);
                     if (s + 16 * u + i16 < s1) e += (double)ts;
                 }
             }
@@ -488,8 +521,6 @@ __global__ void __launch_bounds__(64 * kPopWaves) __attribute__((amdgpu_waves_pe
         // 32 bits: the wave's slots again, a 16-slot tile at a time, from the minibatch's 32-bit feature rows and the member's
         // 32-bit weights, as k_pop_mfma evaluates them
         e = 0.0;
-        constexpr int Act = From == kSets ? kActMax : kActFold;
-        const float k32 = act_k_of<Act>(m);
         float* const eg = src.eps + (size_t)pair * Q::kP;
         if constexpr (From == kDraw) {
             if (ch != 0) {   // (the chunk-0 block, which may not have run, writes the same values)
@@ -498,10 +529,10 @@ __global__ void __launch_bounds__(64 * kPopWaves) __attribute__((amdgpu_waves_pe
                 __threadfence_block();
             }
         }
-        MfmaWeights<S> F;
-        mfma_load_from<S>(F, MemberAt<From>{ src.w0, eg, sgn ? -src.sigma : src.sigma, pair }, lane);
-        if constexpr (!Clamp) scale_output<S>(F, kNegLog2e);
-        if constexpr (Act == kActFold) scale_hidden<S>(F, fold_scale(m.leak));
+        MfmaWeights<S> W32;
+        mfma_load_from<S>(W32, MemberAt<From>{ src.w0, eg, sgn ? -src.sigma : src.sigma, pair }, lane);
+        if constexpr (!Clamp) scale_output<S>(W32, kNegLog2e);
+        if constexpr (Act == kActFold) scale_hidden<S>(W32, fold_scale(m.leak));
         const __amdgpu_buffer_rsrc_t r32 = buffer_of(feat, 4u * ((uint32_t)minibatch_rows(NIN) * (uint32_t)Mcap + (uint32_t)kMinibatchSlack));
         for (int q = 0; q < mine; q++)
             for (int u = 0; u < U; u++) {
@@ -511,15 +542,15 @@ __global__ void __launch_bounds__(64 * kPopWaves) __attribute__((amdgpu_waves_pe
 #pragma unroll
                 for (int ks = 0; ks < Q::kKs1; ks++)
                     b1[0][ks] = buffer_f32(r32, 4u * ((uint32_t)(4 * ks + g) * (uint32_t)Mcap + (uint32_t)i16), 4u * (uint32_t)st);
-                mfma_hidden<S, 1, Act>(F, b1, k32, x);
+                mfma_hidden<S, 1, Act>(W32, b1, ak, x);
                 float ts = 0.0f;
                 if constexpr (kVOut) {
-                    const float d = out_of<S>(valu_out_g<S>(F, x[0], vo_s + wave * kVoTile, g, i16), Clamp) -
+                    const float d = out_of<S>(valu_out_g<S>(W32, x[0], vo_s + wave * kVoTile, g, i16), Clamp) -
                                     buffer_f32(rt, 4u * (uint32_t)(TS * i16 + min(g, NO - 1)), (uint32_t)st * (4u * TS));
                     ts = g < NO ? __fmul_rn(__fmul_rn(m.cw[min(g, NO - 1)], d), d) : 0.0f;
                 } else {
                     f4v o[1];
-                    mfma_output<S, 1>(F, x, o);
+                    mfma_output<S, 1>(W32, x, o);
 #pragma unroll
                     for (int r = 0; r < RO; r++) {
                         const float d = out_of<S>(o[0][r], Clamp) - buffer_f32(rt, to + 4u * r, (uint32_t)st * (4u * TS));
@@ -764,7 +795,8 @@ __global__ void __launch_bounds__(256) k_lat_pair_mfma(DevModel m, const float* 
 // What bounds it is instruction issue, as in k_pop_split, with the feature loads (two floats a tap and channel) beside it.
 // Against k_lat_pair_mfma (MI355X): 512 x 512, four maps, a searched and a 4-channel level, 4 pairs: 71 -> 40 us; RGB, levels of 8 and 4 channels,
 // 16 pairs: 292 -> 165 us. All four products of the two parts are taken (1% of the step): over seven models of three seeds the
-// gradient's error against 64 bits is 1.002 times the 32-bit kernel's, 1.004 without the product of the lo parts.
+// gradient's error against 64 bits was 1.002 times the 32-bit kernel's, 1.004 without the product of the lo parts; with the small
+// products first, the per-pixel differences' is 0.68 to 0.98 times it (split_mlp.hpp).
 template <class S>
 __device__ __forceinline__ SplitScale split_stage_plain(const DevModel& m, const float* __restrict__ w, double out, unsigned* __restrict__ lds) {
     using L = SplitLds<S>;
@@ -803,35 +835,37 @@ __device__ __forceinline__ SplitScale split_stage_plain(const DevModel& m, const
             const int l = L::layer(k);
             const bool b = L::bias(k);
             const double fw = l == 0 ? f.w1 : (l == 1 ? f.w2 : f.w3), fb = l == 0 ? f.b1 : (l == 1 ? f.b2 : f.b3);
-            lds[L::pos(k)] = split_param(v[q], 0.0f, 0.0f, b ? fb : fw, b);
+            unsigned short last;
+            lds[L::pos(k)] = split_param(v[q], 0.0f, 0.0f, b ? fb : fw, b, last);
         }
     }
     __syncthreads();
     return sc;
 }
 
-// A wave's 64 pixels' features f (lane: one pixel) split to t: per pixel split_inputs hi parts, then as many lo parts times
-// kSplitLo
+// A wave's 64 pixels' features f (lane: one pixel) split to t, as split_piece orders them
 template <class S>
 __device__ __forceinline__ void split_write(const float (&f)[S::kMaxIn], float neg, u4v* __restrict__ t, int lane) {
     constexpr int N = split_inputs(S::kNin), C = N / 8;   // 16-byte pieces per part
     const float neg_lo = neg * kSplitLo;
+    h2v hi[N / 2], lo[N / 2];
 #pragma unroll
-    for (int q = 0; q < C; q++) {
-        h2v hi[4], lo[4];
+    for (int j = 0; j < N / 2; j++) {
+        const int i = 2 * j;
+        const float x = i < S::kNin ? f[i < S::kNin ? i : 0] : 0.0f, y = i + 1 < S::kNin ? f[i + 1 < S::kNin ? i + 1 : 0] : 0.0f;
+        hi[j] = __builtin_convertvector((f2v){ x, y }, h2v);
+        lo[j] = __builtin_convertvector((f2v){ __builtin_fmaf((float)hi[j][0], neg_lo, x * kSplitLo),
+                                               __builtin_fmaf((float)hi[j][1], neg_lo, y * kSplitLo) }, h2v);
+    }
+#pragma unroll
+    for (int q = 0; q < 2 * C; q++) {
+        u4v a;
 #pragma unroll
         for (int j = 0; j < 4; j++) {
-            const int i = 8 * q + 2 * j;
-            const float x = i < S::kNin ? f[i < S::kNin ? i : 0] : 0.0f, y = i + 1 < S::kNin ? f[i + 1 < S::kNin ? i + 1 : 0] : 0.0f;
-            hi[j] = __builtin_convertvector((f2v){ x, y }, h2v);
-            lo[j] = __builtin_convertvector((f2v){ __builtin_fmaf((float)hi[j][0], neg_lo, x * kSplitLo),
-                                                   __builtin_fmaf((float)hi[j][1], neg_lo, y * kSplitLo) }, h2v);
+            const int p = split_piece(N, 8 * q + 2 * j);   // (an even half and the next one are parts of neighbouring inputs)
+            a[j] = __builtin_bit_cast(unsigned, p < N ? hi[p / 2 % (N / 2)] : lo[p / 2 % (N / 2)]);
         }
-        u4v a, b;
-#pragma unroll
-        for (int j = 0; j < 4; j++) { a[j] = __builtin_bit_cast(unsigned, hi[j]); b[j] = __builtin_bit_cast(unsigned, lo[j]); }
         t[lane * 2 * C + q] = a;
-        t[lane * 2 * C + C + q] = b;
     }
 }
 // the first-layer operand of pixel `px` (of the wave's 64) for lane group g
@@ -846,7 +880,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(split_
                                                       const float* __restrict__ eps, const float* __restrict__ tgt, float sg,
                                                       unsigned mask, float* __restrict__ dpix, int K, int blocks) {
     using Q = MfmaShape<S>;
-    using P = SplitShape<S>;
+    using P = SplitShape<S, 2>;
     constexpr int NO = Q::kNout, RO = out_regs<S>(), kEx = 64 * split_inputs(Q::kIn);   // floats of one member's exchange
     constexpr bool kVOut = valu_out<S>();
     constexpr int NT = kVOut ? NO : RO;
@@ -856,8 +890,11 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(split_
     __shared__ __attribute__((aligned(16))) float sum_s[kVOut ? 1 : 4][kVOut ? 4 : 256];
     const int lane = tid_x() & 63, wave = __builtin_amdgcn_readfirstlane(tid_x() >> 6), i16 = lane & 15, g = lane >> 4;
     const SplitScale sc = split_stage_plain<S>(m, w, Clamp ? 1.0 : kNegLog2eD, par_s);
-    SplitWeights<S> W;
-    split_load<S>(W, par_s, lane);
+    SplitWeights<S, 2> W;
+    {
+        h8v kept[1];
+        split_load<S, 2>(W, par_s, nullptr, lane, kept);
+    }
     const float ak = in_vgpr(act_k_of<kActFold>(m)), neg = in_vgpr(-1.0f), inv = in_vgpr(sc.inv);
     float cw[NT];
 #pragma unroll
@@ -921,8 +958,8 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(split_
 #pragma unroll
                 for (int v = 0; v < 2; v++) {
                     h8v b[P::kB];
-                    split_hidden<S, true>(W, split_read<S>((const u4v*)(ex + v * kEx), 16 * u + i16, g), ak, neg, b);
-                    o[v] = split_dot<S, true>(W.ao[u], b, o[v]);
+                    split_hidden<S, 2, kActFold>(W, split_read<S>((const u4v*)(ex + v * kEx), 16 * u + i16, g), ak, neg, b);
+                    o[v] = split_dot_out<S, 2>(W, u, b, o[v]);
                 }
             diff = terms(o[0], o[1], t);
         } else {
@@ -937,8 +974,8 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(split_
 #pragma unroll
                 for (int v = 0; v < 2; v++) {
                     h8v b[P::kB];
-                    split_hidden<S, true>(W, split_read<S>((const u4v*)(ex + v * kEx), 16 * u + i16, g), ak, neg, b);
-                    o[v] = split_dot<S, true>(W.ao[0], b, W.co);
+                    split_hidden<S, 2, kActFold>(W, split_read<S>((const u4v*)(ex + v * kEx), 16 * u + i16, g), ak, neg, b);
+                    o[v] = split_dot_out<S, 2>(W, 0, b, W.co);
                 }
                 sums[(16 * u + i16) * 4 + g] = terms(o[0], o[1], t);
             }
@@ -1176,7 +1213,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(qat_wa
                                                  const float* __restrict__ tgt, const int* __restrict__ qat_bits,
                                                  const float* __restrict__ grid, int blocks) {
     using Q = MfmaShape<S>;
-    using P = SplitShape<S>;
+    using P = SplitShape<S, 2>;
     constexpr int NO = Q::kNout, RO = out_regs<S>(), C0 = S::kC0, kEx = 64 * split_inputs(Q::kIn);
     constexpr bool kVOut = valu_out<S>();
     constexpr int NT = kVOut ? NO : RO;
@@ -1188,8 +1225,11 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(qat_wa
     float* const vo = ex + kEx;
     float* const sums = vo + (kVOut ? 2 * kVoTile : 0);
     const SplitScale sc = split_stage_plain<S>(m, w, Clamp ? 1.0 : kNegLog2eD, par_s);
-    SplitWeights<S> W;
-    split_load<S>(W, par_s, lane);
+    SplitWeights<S, 2> W;
+    {
+        h8v kept[1];
+        split_load<S, 2>(W, par_s, nullptr, lane, kept);
+    }
     const float ak = in_vgpr(act_k_of<kActFold>(m)), neg = in_vgpr(-1.0f), inv = in_vgpr(sc.inv);
     // the first layer's weights of the searched inputs for this lane's units, with the layer's factors
     float w1[C0][Q::kHt][4];
@@ -1246,8 +1286,9 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(qat_wa
             f4v s0[Q::kHt];
 #pragma unroll
             for (int ot = 0; ot < Q::kHt; ot++) {
-                s0[ot] = mfma_h(W.a1[ot][0], b1, W.c1[ot]);
-                if constexpr (P::kS1 > 1) s0[ot] = mfma_h(W.a1[ot][1], b1, s0[ot]);
+                s0[ot] = W.c1[ot];
+#pragma unroll
+                for (int s = P::kS1 - 1; s >= 0; s--) s0[ot] = mfma_h(W.a1[ot][s], b1, s0[ot]);
             }
 #pragma unroll
             for (int c = 0; c < C0; c++) win[t][c] = __int_as_float(__builtin_amdgcn_ds_bpermute((16 * t + i16) << 2, __float_as_int(own[c])));
@@ -1279,14 +1320,14 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(qat_wa
 #pragma unroll
                             for (int r = 0; r < 4; r++) a1[ot][r] = __builtin_fmaf(w1[c][ot][r], gc[v], sb[ot][r]);
                         h8v b[P::kB];
-                        split_act<S>(a1, ak, neg, b);
+                        split_act<S, 2, kActFold>(a1, ak, neg, b);
                         if constexpr (Q::kNL > 1) {
                             f4v a2[Q::kHt];
 #pragma unroll
-                            for (int ot = 0; ot < Q::kHt; ot++) a2[ot] = split_dot<S, true>(W.ah[ot], b, W.ch[ot]);
-                            split_act<S>(a2, ak, neg, b);
+                            for (int ot = 0; ot < Q::kHt; ot++) a2[ot] = split_dot_hidden<S, 2>(W, ot, b);
+                            split_act<S, 2, kActFold>(a2, ak, neg, b);
                         }
-                        const f4v o = split_dot<S, true>(W.ao[0], b, W.co);   // (at most 4 outputs: lane group 0 holds them)
+                        const f4v o = split_dot_out<S, 2>(W, 0, b, W.co);   // (at most 4 outputs: lane group 0 holds them)
                         lv[v] = 0.0f;
 #pragma unroll
                         for (int r = 0; r < NT; r++) {

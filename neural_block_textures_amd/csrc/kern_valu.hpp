@@ -96,10 +96,11 @@ __global__ void __launch_bounds__(kTPB) k_batch(DevModel m, uint64_t head, int M
             constexpr int N = split_inputs(S::kNin), TS = split_targets(S::kNout);
             union { _Float16 h[2 * N]; uint4 q[N / 4]; } v;
 #pragma unroll
-            for (int i = 0; i < N; i++) {
+            for (int h = 0; h < 2 * N; h++) {
+                const int q = split_piece(N, h), i = q % N;
                 const float x = i < S::kNin ? f[i < S::kNin ? i : 0] : 0.0f;
-                v.h[i] = (_Float16)x;
-                v.h[N + i] = (_Float16)((x - (float)v.h[i]) * kSplitLo);
+                const _Float16 hi = (_Float16)x;
+                v.h[h] = q < N ? hi : (_Float16)((x - (float)hi) * kSplitLo);
             }
 #pragma unroll
             for (int i = 0; i < N / 4; i++) sj.feat[(size_t)s * (N / 4) + i] = v.q[i];

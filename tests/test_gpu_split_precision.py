@@ -92,24 +92,26 @@ def population_errors(orc, monkeypatch, name, regime, path, seeds, batch):
     return e
 
 
-REGIMES = ["small", "outlier_dead"]
+REGIMES = ["plain", "small", "outlier", "wide", "outlier_dead"]
 
 
 def cases(names):
     return [(n, r) for n in sorted(names) for r in REGIMES if r != "outlier_dead" or MODELS[n].leak == 0.0]
 
 
-# A wrong range costs orders of magnitude; the members' own roundings are within a factor of two of each other's.
+# The members' roundings are independent: 192 loss differences give each error to 5% and the ratio of two to 7%. Measured 0.38 to
+# 0.97 (with the weights in two parts up to 1.75).
 @pytest.mark.parametrize("name,regime", cases(MODELS))
 def test_population_no_further_from_64_bits(orc, monkeypatch, name, regime):
     split, full = population_errors(orc, monkeypatch, name, regime, "es", 4, 1500)
-    assert split <= 2.0 * full
+    assert split <= 1.1 * full
 
 
+# Thousands of differences each. Measured 0.81 to 1.02.
 @pytest.mark.parametrize("name,regime", cases(["rgb_16x2", "two_level", "material", "chief1_36", "jit_mfma_28", "one_24"]))
 def test_central_differences_no_further_from_64_bits(orc, monkeypatch, name, regime):
     split, full = population_errors(orc, monkeypatch, name, regime, "fd", 2, 1500)
-    assert split <= 1.2 * full
+    assert split <= 1.1 * full
 
 
 def latent_errors(orc, monkeypatch, name, regime, seeds, K=4):
@@ -140,11 +142,12 @@ def latent_errors(orc, monkeypatch, name, regime, seeds, K=4):
     return e
 
 
-# (a shape compiled at init has no 32-bit latent pair kernel beside the split one)
+# Measured 0.68 to 1.0; 1.13 for the 16-wide model of large weights, whose 32-bit sums round few times where its hidden values
+# have 22 bits. (A shape compiled at init has no 32-bit latent pair kernel beside the split one.)
 @pytest.mark.parametrize("name,regime", cases(n for n in MODELS if n not in ("jit_mfma_28", "rgb_20", "one_24")))
 def test_latent_pairs_no_further_from_64_bits(orc, monkeypatch, name, regime):
     split, full = latent_errors(orc, monkeypatch, name, regime, 1)
-    assert split <= 1.1 * full
+    assert split <= (1.2 if regime == "wide" else 1.1) * full
 
 
 @pytest.mark.parametrize("name", ["rgb_16x2", "material", "material_clamp", "large", "chief1_36"])
