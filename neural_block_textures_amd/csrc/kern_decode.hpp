@@ -20,15 +20,36 @@
 
 namespace ntc_hip {
 
-// Matrix instructions of a 16-pixel tile, every output a row of one output tile, and whether they pay: 32 cycles each
-// against about 1.1 cycles of a multiply-add on the VALU (4.5 cycles for 64 pixels). 16-wide decoders and wider ones do
-// (16: 320 cycles against 450), 17-wide ones do not (their second tile holds one unit: 608 against 516).
+// Matrix instructions of a 16-pixel tile, every output a row of one output tile.
 __host__ __device__ constexpr int decode_mfmas(int nin, int H, int NL) {
     const int ht = (H + 15) / 16, ks = 4 * (ht - 1) + (H - 16 * (ht - 1) + 3) / 4;
     return ht * ((nin + 3) / 4) + (NL - 1) * ht * ks + ks;
 }
+// The registers it takes (within 4 of the compiler's count for 6 and 14 inputs, 16 to 64 wide, one to six layers): weights and
+// biases of every layer, which stay in them, the tiles in flight and the first layer's operands. And the waves per SIMD that
+// they leave room for, at most 4.
+__host__ __device__ constexpr int decode_regs(int nin, int H, int NL) {
+    const int ht = (H + 15) / 16, ks = 4 * (ht - 1) + (H - 16 * (ht - 1) + 3) / 4, ks1 = (nin + 3) / 4;
+    return ht * ks1 + 4 * ht + ks + 4 + (NL - 1) * ht * (ks + 4) + 42 + 8 * ks1;
+}
+__host__ __device__ constexpr int decode_waves(int nin, int H, int NL) {
+    const int r = decode_regs(nin, H, NL), w = H > 48 ? 2 : (H > 32 ? 3 : 4);
+    return r <= 128 && w > 3 ? 4 : (r <= 168 && w > 2 ? 3 : (r <= 256 ? 2 : 1));
+}
+// Whether it pays: a matrix instruction takes 32 cycles against about 1.1 of a multiply-add on the VALU (4.5 cycles for 64
+// pixels). 16-wide decoders and wider ones do (16: 320 cycles against 450), 17-wide ones do not (their second tile holds one
+// unit: 608 against 516). And its registers must fit with two waves or more.
 __host__ __device__ constexpr bool decode_pays(int nin, int H, int NL, int nout) {
-    return nout <= 16 && NL >= 1 && 32 * decode_mfmas(nin, H, NL) < nin * H + (NL - 1) * H * H + H * nout;
+    return nout <= 16 && NL >= 1 && 32 * decode_mfmas(nin, H, NL) < nin * H + (NL - 1) * H * H + H * nout && decode_waves(nin, H, NL) >= 2;
+}
+// Whether it also pays for at most 4 outputs as floats on `groups` 256-pixel groups, `fill` of them a full chip: their stores are
+// a float a lane, and a full chip hides the VALU kernel's latencies. Below a full chip it does (MI355X, us, VALU -> here: 16-wide
+// 256 x 256 9.5 -> 7.8, 24-wide 11.9 -> 9.7); above, where the matrix instructions are a quarter ahead (32-wide 1024 x 1024 60.6 ->
+// 55.2, 2048 x 2048 218 -> 188) and not where less (16-wide 27.5 -> 29.3 and 87.8 -> 97.1, 24-wide 41.0 -> 43.5 and 141 -> 149), nor
+// on just a full chip (32-wide 512 x 512 21.7 -> 22.9).
+__host__ __device__ constexpr bool decode_float_pays(int nin, int H, int NL, int nout, size_t groups, size_t fill) {
+    return nout > 4 || groups < fill ||
+           (groups >= 2 * fill && 4 * 32 * decode_mfmas(nin, H, NL) <= 3 * (nin * H + (NL - 1) * H * H + H * nout));
 }
 template <class S, bool = S::kFixed && S::kUniform>
 struct DecodeOk { static constexpr bool value = false; };
@@ -38,8 +59,6 @@ struct DecodeOk<S, true> { static constexpr bool value = decode_pays(S::kNin, S:
 enum DecodeTo : int { kToFloat = 0, kToBytes = 1, kToError = 2 };
 
 __host__ __device__ constexpr int dec_unit(int ot, int row) { return 16 * ot + 4 * (row & 3) + (row >> 2); }
-// waves per SIMD that the registers allow
-__host__ __device__ constexpr int decode_waves(int H) { return H > 48 ? 2 : (H > 32 ? 3 : 4); }
 // 16-pixel tiles evaluated at once, so that enough chains of matrix instructions are independent
 constexpr int dec_tiles(int ht) { return ht == 1 ? 4 : (ht == 2 ? 2 : 1); }
 
@@ -144,7 +163,7 @@ __device__ __forceinline__ int to_byte(float v) { return (int)roundf(__fmul_rn(f
 // Pixels 0 .. ew eh - 1 of the extent (raster order within it) to out: W H nout floats (kToFloat) or bytes (kToBytes), the
 // extent then being the image; or four sums of squared 8-bit differences from tgt per block (kToError).
 template <class S, int To>
-__global__ void __launch_bounds__(kTPB) __attribute__((amdgpu_waves_per_eu(decode_waves(S::kH)))) k_decode_mfma(DevModel m, const float* __restrict__ w, const float* __restrict__ z,
+__global__ void __launch_bounds__(kTPB) __attribute__((amdgpu_waves_per_eu(decode_waves(S::kNin, S::kH, S::kNL)))) k_decode_mfma(DevModel m, const float* __restrict__ w, const float* __restrict__ z,
                                                                       const float* __restrict__ tgt, int ew, int eh, void* __restrict__ out) {
     using D = DecWeights<S>;
     constexpr int NO = S::kNout, U = dec_tiles(D::kHt);

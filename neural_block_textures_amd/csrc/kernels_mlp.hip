@@ -405,7 +405,8 @@ static size_t launch_decode_mfma(Impl& I, const float* z, int ew, int eh, void* 
     const int H = I.dm.hidden[0];
     for (int l = 1; l < I.dm.nl; l++) if (I.dm.hidden[l] != H) return 0;
     if (!decode_pays(I.dm.nin, H, I.dm.nl, I.dm.nout)) return 0;
-    const size_t groups = ((size_t)ew * eh + kTPB - 1) / kTPB, fill = (size_t)I.cus * decode_waves(H);
+    const size_t groups = ((size_t)ew * eh + kTPB - 1) / kTPB, fill = (size_t)I.cus * decode_waves(I.dm.nin, H, I.dm.nl);
+    if (To == kToFloat && !decode_float_pays(I.dm.nin, H, I.dm.nl, I.dm.nout, groups, fill)) return 0;
     const size_t rounds = (groups + fill - 1) / fill, blocks = (groups + rounds - 1) / rounds;
     bool done = false;
     if (I.jit) {

@@ -71,3 +71,22 @@ def test_decode_leak(leak, clamp):
     lay = Layout(70, 9, [(18, 3, 4, False)], [24, 24], T=2, leak=leak, clamp_out=clamp)
     z, p, tgt = data(lay, 34)
     same(lay, z, p, tgt)
+
+
+@pytest.mark.parametrize("hidden,T", [([32], 1), ([64], 4), ([24] * 3, 1), ([32] * 4, 4), ([64] * 3, 1), ([64] * 4, 4)])
+def test_decode_layers(hidden, T):
+    """one, three and four hidden layers: kernels of fewer waves, and (the last two) models whose layers do not fit the registers,
+    which the VALU decode takes"""
+    lay = Layout(131, 37, [(33, 10, 4, False), (9, 3, 4, False)], hidden, T=T, leak=0.01)
+    z, p, tgt = data(lay, 35)
+    say("decode layers", hidden, T)
+    same(lay, z, p, tgt)
+
+
+@pytest.mark.parametrize("W,H", [(512, 511), (512, 513), (1030, 520)])
+def test_decode_floats_on_a_full_chip(W, H):
+    """at most 4 outputs as floats: images below a full chip, on one and on two (the matrix cores on the first and last)"""
+    lay = Layout(W, H, [(-(-W // 4), -(-H // 4), 8, False), (-(-W // 16), -(-H // 16), 4, False)], [32, 32], leak=0.0)
+    z, p, tgt = data(lay, 36)
+    say("decode floats", W, H)
+    same(lay, z, p, tgt)
