@@ -48,10 +48,12 @@ __global__ void __launch_bounds__(kTPB) k_lat_eps(NoiseFix nt, DevModel m, uint6
 // row: lane group q of a wave sums pair q of the wave's four, lane j of it texel j. The sum is one chain of rounded adds, so
 // its length is fixed; what can be fast is what feeds it.
 // kNarrow (rectangles of at most 16 columns): each lane reads its run from memory, the 16 lanes of a pair a few lines.
-// kWide: texels lie further apart than a line, so a wave copies its pairs' rows to LDS, whole lines at a time and the next
-// row in flight while one is added, and every lane reads its texel's run from there; with four waves all 16 pairs' chains
+// Wider ones, kRows: texels lie further apart than a line, so a wave copies its pairs' rows to LDS, whole lines at a time and the
+// next row in flight while one is added, and every lane reads its texel's run from there; with four waves all 16 pairs' chains
 // run at once. Levels of 128 x 128 x 8 and 32 x 32 x 4 under 512 x 512 pixels, 16 pairs (MI355X): 190 -> 78 us (104 with the four rows a multiple of 64
 // floats apart: sixteen lanes on a bank).
+// Wider ones with at most four pairs, kRuns: one wave's rows to LDS take longer than each lane's own runs of 16 from memory, the
+// next run in flight while one is added. The same levels, 1, 2, 4 and 8 pairs: 43, 46, 53 and 99 us against 57, 57, 58 and 63.
 // kUnit (a level 0 of one pixel per texel): a thread per texel, its pairs in order; a 512 x 512 x 1 plane and a 128 x 128 x 4
 // level, 4 pairs: 31 -> 23 us.
 //
@@ -64,7 +66,7 @@ __global__ void __launch_bounds__(kTPB) k_lat_eps(NoiseFix nt, DevModel m, uint6
 // lv[i]); the rate term goes to level 0, and zq_copy[i] (or null) is level lv[i]'s decode copy.
 constexpr int kGatherTex = 16, kGatherPairs = 4, kGatherWaves = 4, kGatherRun = 32, kWideCols = 320,
               kWideRow = kWideCols + 4;   // (the four pairs' rows in LDS: texels 16 columns apart then share a bank four at a time, not sixteen)
-enum GatherMode : int { kNarrow = 0, kUnit = 1, kWide = 2 };
+enum GatherMode : int { kNarrow = 0, kUnit = 1, kRows = 2, kRuns = 3 };
 struct LatAhead {
     NoiseFix nt; uint64_t seed; uint32_t next_step; unsigned mask;
     float* eps_next; int eb; long long lo, hi;
@@ -76,8 +78,8 @@ struct GatherLevels {
     int mode[kMaxLevels];
     float* zq_copy[kMaxLevels];
 };
-// Wide: whether a level of the launch is kWide
-template <bool Wide>
+// Wide: kRows or kRuns if a level of the launch is, else kNarrow
+template <int Wide>
 __global__ void __launch_bounds__(64 * kGatherWaves) k_lat_gather(DevModel m, GatherLevels G, int K, float scale,
                                                                   const float* __restrict__ dpix,
                                                                   const float* __restrict__ eps, const int* __restrict__ ranges,
@@ -95,7 +97,7 @@ __global__ void __launch_bounds__(64 * kGatherWaves) k_lat_gather(DevModel m, Ga
         return;
     }
     __shared__ float dsum[kGatherWaves * kGatherPairs][kGatherTex];
-    extern __shared__ float stage_s[];   // with a wide level: kGatherPairs x kWideRow floats per wave
+    extern __shared__ float stage_s[];   // with a level of kRows: kGatherPairs x kWideRow floats per wave
     int li = 0;   // this block's level (uniform)
     while (li + 1 < G.n && (int)blockIdx.x >= G.start[li + 1]) li++;
     const int level = G.lv[li], blk0 = (int)blockIdx.x - G.start[li];
@@ -140,7 +142,7 @@ __global__ void __launch_bounds__(64 * kGatherWaves) k_lat_gather(DevModel m, Ga
     for (int k0 = 0; k0 < K; k0 += round) {
         const int kw = k0 + kGatherPairs * wave, k = kw + q;   // this wave's first pair, this lane's
         float d = 0.0f;
-        if (!Wide || G.mode[li] == kNarrow) {
+        if (Wide == kNarrow || G.mode[li] == kNarrow) {
             if (k < K && x0 < x1 && y0 < y1) {
                 // the rectangle's values in raster order, loaded in groups of kGatherRun across row ends and then added in
                 // order (the loads of a group overlap; the sum stays one chain). A slot past the rectangle's end adds +0, which
@@ -164,6 +166,32 @@ __global__ void __launch_bounds__(64 * kGatherWaves) k_lat_gather(DevModel m, Ga
 #pragma unroll
                         for (int i = 0; i < kGatherRun; i++) d += v[i];
                     }
+                }
+            }
+        } else if constexpr (Wide == kRuns) {
+            if (k < K && x0 < x1 && y0 < y1) {
+                // runs of 16 in raster order (a row's last run padded with +0), two buffers
+                const float* dp = dpix + (size_t)k * m.npix;
+                float va[16], vb[16];
+                auto load_run = [&](float (&v)[16], int py, int px) {
+                    const float* rw = dp + (size_t)py * m.W;
+#pragma unroll
+                    for (int i = 0; i < 16; i++) v[i] = px + i < x1 ? rw[px + i] : 0.0f;
+                };
+                auto step = [&](int& py, int& px) { px += 16; if (px >= x1) { px = x0; py++; } };
+                int py = y0, px = x0;
+                load_run(va, py, px);
+                while (true) {
+                    step(py, px);
+                    if (py < y1) load_run(vb, py, px);
+#pragma unroll
+                    for (int i = 0; i < 16; i++) d += va[i];
+                    if (py >= y1) break;
+                    step(py, px);
+                    if (py < y1) load_run(va, py, px);
+#pragma unroll
+                    for (int i = 0; i < 16; i++) d += vb[i];
+                    if (py >= y1) break;
                 }
             }
         } else if (kw < K) {
@@ -252,16 +280,16 @@ void launch_lat_gather(Impl& I, unsigned mask, int k0, int K, float scale, bool 
     const float c1 = t > 0 ? 1.0f - powf(0.9f, (float)t) : 1.0f, c2 = t > 0 ? 1.0f - powf(0.999f, (float)t) : 1.0f;
     GatherLevels G{};
     size_t grid = 0;
-    bool wide = false;
+    int wide = kNarrow;
     const int threads = 64 * std::min(kGatherWaves, (K + kGatherPairs - 1) / kGatherPairs);
-    auto mode = [&](int l) { return l == 0 && I.lv0_unit_cells ? kUnit : (I.lv_cols[l] > 16 ? kWide : kNarrow); };
+    auto mode = [&](int l) { return l == 0 && I.lv0_unit_cells ? kUnit : (I.lv_cols[l] > 16 ? (K > kGatherPairs ? kRows : kRuns) : kNarrow); };
     for (int pass = 0; pass < 2; pass++)   // the wide levels' blocks first: they take longest
         for (int l = 0; l < I.d.nlev; l++)
-            if (((mask >> l) & 1u) && (mode(l) == kWide) == (pass == 0)) {
+            if (((mask >> l) & 1u) && (mode(l) >= kRows) == (pass == 0)) {
                 G.lv[G.n] = l;
                 G.start[G.n] = (int)grid;
                 G.mode[G.n] = mode(l);
-                wide = wide || pass == 0;
+                if (pass == 0) wide = mode(l);
                 G.zq_copy[G.n] = l > 0 ? zq_rest : nullptr;
                 grid += mode(l) == kUnit ? (size_t)blocks_for((size_t)I.d.lv[l].W * I.d.lv[l].H, threads)
                                          : (size_t)blocks_for((size_t)I.d.lv[l].W, kGatherTex) * (size_t)I.d.lv[l].H;
@@ -286,8 +314,8 @@ void launch_lat_gather(Impl& I, unsigned mask, int k0, int K, float scale, bool 
         exit(1);
     }
     ProfScope ps(I, "lat_gather");
-    hipLaunchKernelGGL((wide ? k_lat_gather<true> : k_lat_gather<false>), dim3((unsigned)grid), dim3(threads),
-                       wide ? (size_t)threads / 64 * kGatherPairs * kWideRow * sizeof(float) : 0, I.stream, I.dm, G, K,
+    hipLaunchKernelGGL((wide == kRows ? k_lat_gather<kRows> : wide == kRuns ? k_lat_gather<kRuns> : k_lat_gather<kNarrow>), dim3((unsigned)grid), dim3(threads),
+                       wide == kRows ? (size_t)threads / 64 * kGatherPairs * kWideRow * sizeof(float) : 0, I.stream, I.dm, G, K,
                        scale, I.dpix, I.eps_lat,
                        I.ranges, rate ? 1 : 0, I.ddct.rate_scale, I.ddct.BW, I.ddct.n, rate ? I.dct_dbits + (size_t)k0 * I.ddct.n : nullptr,
                        I.zgrad, k0 == 0 ? 1 : 0, t > 0 ? 1 : 0, I.z, I.zm,
