@@ -32,6 +32,8 @@ __host__ __device__ constexpr int minibatch_rows(int nin) { return 4 * ((nin + 3
 // At most 16 inputs: a first layer of more would need another operand layout (no compiled shape has them). At most two
 // hidden layers: the values of a third, scaled as the first two are, would leave the 16-bit range.
 __host__ __device__ constexpr bool split_pays(int nin, int nl) { return nin <= 16 && nl <= 2; }
+// whether the selector search does too (k_qat_split)
+__host__ __device__ constexpr bool split_qat_pays(int nin, int nl, int nout) { return split_pays(nin, nl) && (nl > 1 || nout > 4); }
 __host__ __device__ constexpr int split_inputs(int nin) { return nin <= 8 ? 8 : 16; }
 __host__ __device__ constexpr int split_targets(int nout) { return nout <= 4 ? nout : 4 * ((nout + 3) / 4); }
 constexpr int kSplitSlack = 256;

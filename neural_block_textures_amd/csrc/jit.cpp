@@ -99,7 +99,7 @@ std::vector<std::string> expressions(const std::string& shape, const DevModel& m
         if (split_pays(m.nin, m.nl)) v.push_back(e("k_lat_split", c + ", false"));
         else v.push_back(e("k_lat_pair_mfma", std::to_string(a_es) + ", " + c));
     }
-    if (unit && split_pays(m.nin, m.nl)) v.push_back(e("k_qat_split", c + ", false"));
+    if (unit && split_qat_pays(m.nin, m.nl, m.nout)) v.push_back(e("k_qat_split", c + ", false"));
     else v.push_back(e("k_qat_mfma", std::to_string(unit ? kActFold : kActAny) + ", " + c));
     return v;
 }

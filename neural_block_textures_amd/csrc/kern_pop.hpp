@@ -1206,6 +1206,8 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(qat_oc
 // 32-bit ones are 24 of 32. The winners are written when all of a round's losses are numbers; a round with a NaN is left as
 // it was and searched in 32 bits at the end (qat_round), the launch giving a wave at most 64 rounds.
 // material512, two channels of four values (MI355X): 73 -> 38 us.
+// With one hidden layer a candidate is the output layer alone, of which at most 4 outputs are a small part of a matrix tile: those
+// models stay on k_qat_mfma, whose output layer is on the VALU (7-32-3, one channel, 512 x 512: 26 us against 31).
 // (a wave per SIMD fewer than k_pop_split with more than one searched channel, whose first-layer weights are in registers too)
 constexpr int qat_waves(int nin, int H, int nout, int c0) { return split_waves(nin, H, nout) - (c0 > 1 && H <= 48 ? 1 : 0); }
 template <class S, bool Clamp, bool UnitCw>

@@ -248,7 +248,7 @@ void launch_lat_pair(Impl& I, int K, float sigma, unsigned mask) {
 }
 
 void launch_qat_mfma(Impl& I) {
-    if (split_pays(I.dm.nin, I.dm.nl) && I.dm.leak >= 0.0f && I.dm.leak <= 1.0f) {
+    if (split_qat_pays(I.dm.nin, I.dm.nl, I.dm.nout) && I.dm.leak >= 0.0f && I.dm.leak <= 1.0f) {
         // as many blocks as fit the chip; more where a wave would have over 64 rounds (its mask of rounds to search again)
         const size_t rounds = (I.npix + 63) / 64;
         const size_t fill = std::max((size_t)I.cus * qat_waves(I.dm.nin, I.dm.hidden[0], I.dm.nout, I.dm.lv[0].C), (rounds + 255) / 256);

@@ -205,3 +205,24 @@ def test_latent_pairs_on_the_32_bit_instructions(orc, monkeypatch, name):
         lay.levels = [(max(1, W * w // base.W), max(1, H * h // base.H), c, near) for w, h, c, near in base.levels]
         z, p, tgt = data(lay, 26)
         latent(orc, lay, z, p, tgt, K)
+
+
+@pytest.mark.parametrize("T", [1, 4])
+def test_selector_search_one_hidden_layer(orc, T):
+    """one hidden layer: at most 4 outputs on k_qat_mfma, more on k_qat_split; the oracle's choices but for ties"""
+    from neural_block_textures_amd import synth
+    lay = Layout(65, 21, [(65, 21, 2, True), (17, 6, 4, False)], [32], T=T, leak=0.01)
+    z, p, tgt = data(lay, 30)
+    grid, bits, n0 = synth.qat_grid(), [2, 3], 65 * 21 * 2
+    for c in range(2):
+        z[:n0].reshape(-1, 2)[:, c] = synth.qat_snap(z[:n0].reshape(-1, 2)[:, c], bits[c], grid)
+    tr = trainer(lay, z, p, tgt, qat_bits=bits, qat_grid=grid)
+    tr.qat_search()
+    zg, zc = tr.download_model()[0], z.copy()
+    tr.close()
+    orc.qat_search(lay, p, zc, tgt, bits, grid)
+    assert np.array_equal(zg[n0:], z[n0:])
+    diff = np.nonzero((zg[:n0] != zc[:n0]).reshape(-1, 2).any(1))[0]
+    say("selectors, one hidden layer", T, "differ", diff.size)
+    ec, eg = orc.decode_err(lay, p, zc, tgt), orc.decode_err(lay, p, zg, tgt)
+    assert (np.abs(ec[diff] - eg[diff]) <= 1e-6 * np.maximum(ec[diff], eg[diff]) + 1e-12).all()
