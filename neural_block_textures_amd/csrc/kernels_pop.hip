@@ -118,7 +118,10 @@ void launch_pop_eval_fd(Impl& I, float h, int M, int chunk, int chunks) {
 bool pop_split_possible(const Impl& I) {
     if (!pop_on_matrix_cores(I)) return false;
     const char* env = getenv("NTC_HIP_POP_PAIR");
-    return !(env && env[0] == '0') && split_pays(I.dm.nin, I.dm.nl);
+    // (its arrays are read through 32-bit offsets: for 9 to 12 inputs 67 million slots, where k_pop_mfma's hold 89 million)
+    const uint64_t slots = (uint64_t)I.Mcap + kSplitSlack, most = (uint64_t)1 << 32;
+    const bool fits = slots * 4u * split_inputs(I.dm.nin) < most && slots * 4u * split_targets(I.dm.nout) < most;
+    return !(env && env[0] == '0') && split_pays(I.dm.nin, I.dm.nl) && fits;
 }
 bool pop_split_step(const Impl& I) { return I.pop_split && pop_on_matrix_cores(I); }
 

@@ -226,3 +226,21 @@ def test_selector_search_one_hidden_layer(orc, T):
     say("selectors, one hidden layer", T, "differ", diff.size)
     ec, eg = orc.decode_err(lay, p, zc, tgt), orc.decode_err(lay, p, zg, tgt)
     assert (np.abs(ec[diff] - eg[diff]) <= 1e-6 * np.maximum(ec[diff], eg[diff]) + 1e-12).all()
+
+
+def test_split_population_past_32_bit_offsets():
+    """a minibatch whose split arrays pass 4 GiB (9 to 12 inputs: 67 million slots) evaluates on the 32-bit kernel, whose rows
+    still fit. The oracle would take minutes over its slots: the members are the weights themselves (sigma 0), and their loss is
+    the mean of the pixels' losses within five of its standard deviations."""
+    lay = Layout(16, 16, [(4, 4, 4, False), (2, 2, 4, False)], [36, 36], T=4, leak=0.01)
+    z, p, tgt = data(lay, 31)
+    for M, split in ((1 << 20, True), (68 << 20, False)):
+        tr = trainer(lay, z, p, tgt, max_pairs=1, max_batch=M)
+        assert tr.on_matrix_cores("pop_eval") and tr.on_matrix_cores("pop_split") == split
+        say("split sizes", M)
+        d = (tr.decode_full().astype(np.float64) - tgt).reshape(-1, lay.nout)
+        tr.mlp_step(1, 0.0, 0.0, 1, M)
+        loss = tr.mlp_stats()[0]
+        tr.close()
+        e = (d * d).sum(1) / (3.0 * lay.T)
+        assert abs(loss - e.mean()) <= 5 * e.std() / np.sqrt(M) + 1e-6 * e.mean()
