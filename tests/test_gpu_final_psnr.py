@@ -42,10 +42,11 @@ def dct_desc(w, lay, s):
     return d, steps, (W0 // 8) * (H0 // 8) * C0
 
 
-def run_schedule(orc, name, fx, probes=None):
+def run_schedule(orc, name, fx, probes=None, nudge=0):
     """the fixture's schedule on a fresh device trainer: (final PSNR, {checkpoint: PSNR}); probes: a list that gets, at
     the DCT switch and at every refit, the number of blocks whose device probe codes differ from the oracle's probe of
-    the same device state"""
+    the same device state; nudge: at the DCT switch every weight moves by one unit in its last place, up or down by that
+    seed"""
     s = SCHEDULES[name]
     w, lay, tr, z, p, tgt = full_trainer(name)
     assert np.array_equal(digest(z, p, tgt), fx["digest"]), "the synthetic inputs differ from the reference run's"
@@ -66,6 +67,10 @@ def run_schedule(orc, name, fx, probes=None):
     for it in range(1, iters + 1):
         if w.dct_q:
             if not live and it == s["dct_start"]:                 # the DCT switch (main.cpp:4100-4109)
+                if nudge:
+                    zn, pn = tr.download_model()
+                    to = np.where(np.random.default_rng(nudge).random(pn.size) < 0.5, np.float32(-np.inf), np.float32(np.inf))
+                    tr.upload_model(zn, np.nextafter(pn, to.astype(np.float32)))
                 code, _ = tr.dct_probe()                          # the probe of the clamped shadow, then the snap
                 if H is not None:
                     probes.append(int((code != oracle_codes()).sum()))
@@ -122,11 +127,15 @@ def test_dct512_final_psnr_against_reference_loop(orc, monkeypatch):
     After the switch the run depends on rounding: a shadow value a rounding away from a quantizer boundary snaps to
     the other lattice point, and the rate term counts the symbols. The reference itself shows it. Its loop built for
     x86-64-v4 (AVX-512, the same -O3 -ffast-math flags; final_psnr_dct512_v4.npz) follows its x86-64-v3 build to
-    1e-4 dB up to the switch and ends 0.057 dB away from it. The device's two population kernels (k_pop_pair, and
-    k_pop_mfma with NTC_HIP_POP_PAIR=0) differ only in the rounding of the member losses; they end 0.095 dB apart.
-    Bars: each device run within 0.1 dB of the x86-64-v3 build's end and within 0.05 dB of one of the reference's
-    two builds (k_pop_pair 0.022 dB from the x86-64-v4 build, k_pop_mfma 0.017 dB from the x86-64-v3 build when
-    measured); the x86-64-v3 build's end inside the two device runs' range widened by 0.05 dB."""
+    1e-4 dB up to the switch and ends 0.057 dB away from it; the device's runs with every weight moved by one unit in its
+    last place at the switch end with a standard deviation of 0.05 dB. A single end so says little, and two ends of two
+    kernels bracketing the reference's say little too: so they did with earlier kernels, did not when the latent pairs
+    moved to k_lat_split (47.308 and 47.319 dB against 47.241), and would by chance.
+    Bars: the kernels as shipped and the 32-bit ones (NTC_HIP_POP_PAIR=0: k_pop_mfma, k_lat_pair_mfma), each within
+    0.1 dB of the x86-64-v3 build's end and within 0.05 dB of one of the reference's two builds; and the mean of eight
+    shipped runs, seven of them nudged at the switch, within 0.05 dB of the mean of the reference's two builds (when
+    written: 47.282 against 47.270; the same eight on the 32-bit kernels 47.275), the x86-64-v3 build's end inside their range
+    widened by 0.05 dB."""
     fx = fixture("dct512")
     s = SCHEDULES["dct512"]
     ps_c = float(fx["final_psnr"])
@@ -143,7 +152,7 @@ def test_dct512_final_psnr_against_reference_loop(orc, monkeypatch):
             f"after it {post4}; final {float(v4['final_psnr']):.4f} dB, delta {float(v4['final_psnr']) - ps_c:+.4f}")
         refs.append(float(v4["final_psnr"]))
     finals = []
-    for kernel, env in (("k_pop_pair", None), ("k_pop_mfma", "0")):
+    for kernel, env in (("k_pop_mfma, k_lat_pair_mfma", "0"), ("k_pop_split, k_lat_split", None)):
         if env is None:
             monkeypatch.delenv("NTC_HIP_POP_PAIR", raising=False)
         else:
@@ -163,4 +172,8 @@ def test_dct512_final_psnr_against_reference_loop(orc, monkeypatch):
             assert nearest <= 0.05
         finals.append(ps_g)
     assert ps_c > float(fx["start_psnr"]) + 0.5
-    assert min(finals) - 0.05 <= ps_c <= max(finals) + 0.05
+    shipped = [finals[-1]] + [run_schedule(orc, "dct512", fx, nudge=n)[0] for n in range(1, 8)]
+    say(f"dct512 as shipped, eight runs a unit in the last place apart at the switch: {' '.join(f'{p:.4f}' for p in shipped)}; "
+        f"mean {np.mean(shipped):.4f} dB, reference builds {np.mean(refs):.4f} dB")
+    assert abs(np.mean(shipped) - np.mean(refs)) <= 0.05
+    assert min(shipped) - 0.05 <= ps_c <= max(shipped) + 0.05
