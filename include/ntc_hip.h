@@ -192,10 +192,8 @@ void ntc_trainer_set_profiling_only(ntc_trainer* t, const char* names);
 void ntc_trainer_set_profiling_every(ntc_trainer* t, int n);
 int ntc_trainer_kernel_time(ntc_trainer* t, const char* name, double* total_ms, long long* launches);
 // 1 if the stage ("pop_eval": the ES and central-difference populations, "lat_pair", "qat_search") runs on
-// the matrix cores for this model, else 0; "pop_split": 1 if its ES steps take the population kernel on the 16-bit
-// matrix instructions with 32-bit operands in two parts (k_pop_split); "pop_pair": 1 if the model is one of the library's
-// shapes of one or two whole 16-unit hidden tiles and, with the pairs and minibatch sized at init, a chunk's first layer
-// takes at most 2 MiB; "pop_pair_own": 1 if moreover it has one such tile and at most 4 outputs
+// the matrix cores for this model, else 0; "pop_split", "lat_split", "qat_split": 1 if it does on the 16-bit matrix
+// instructions with 32-bit operands in parts (k_pop_split, k_lat_split, k_qat_split)
 int ntc_trainer_on_matrix_cores(ntc_trainer* t, const char* stage);
 /* on = 0: every stage of this trainer runs on the VALU kernels from the next call on (the matrix-core
  * kernels' parity and speed are then measured against them); on = 1 (the default): the matrix cores

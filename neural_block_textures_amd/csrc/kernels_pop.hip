@@ -113,8 +113,9 @@ void launch_pop_eval_fd(Impl& I, float h, int M, int chunk, int chunks) {
 }
 
 // The split population kernel takes every step that the matrix cores take, of the shapes it has an operand layout for
-// (split_pays). Against the 32-bit kernel on the MI355X: see k_pop_split. NTC_HIP_POP_PAIR=0 keeps the
-// 32-bit kernels for every step of a listed shape: k_pop_mfma, and k_lat_pair_mfma for its latent pairs.
+// (split_pays) and minibatches its offsets hold. Against the 32-bit kernel on the MI355X: see k_pop_split. NTC_HIP_POP_PAIR=0
+// (read at init) keeps k_pop_mfma for the population, and k_lat_pair_mfma for the latent pairs of the listed shapes: the 32-bit
+// kernels that the tests compare the split ones with.
 bool pop_split_possible(const Impl& I) {
     if (!pop_on_matrix_cores(I)) return false;
     const char* env = getenv("NTC_HIP_POP_PAIR");
@@ -124,32 +125,6 @@ bool pop_split_possible(const Impl& I) {
     return !(env && env[0] == '0') && split_pays(I.dm.nin, I.dm.nl) && fits;
 }
 bool pop_split_step(const Impl& I) { return I.pop_split && pop_on_matrix_cores(I); }
-
-// ntc_trainer_on_matrix_cores' "pop_pair" and "pop_pair_own": the fixed shapes of one or two whole 16-unit hidden tiles
-// whose chunks' first layers take at most 2 MiB, and those of them with at most 4 outputs and one tile.
-template <class S, bool = MfmaShape<S>::kOk>
-struct PairShape { static constexpr bool kOk = false, kOwn = false; };
-template <class S>
-struct PairShape<S, true> {
-    using Q = MfmaShape<S>;
-    static constexpr bool kOk = Q::kHt <= 2 && Q::kH % 16 == 0, kOwn = kOk && pop_own<S>();
-};
-bool pop_pair_possible(const Impl& I) {
-    if (I.jit || I.valu_only || !(I.dm.leak >= 0.0f && I.dm.leak <= 1.0f)) return false;
-    const char* env = getenv("NTC_HIP_POP_PAIR");
-    if (env && env[0] == '0') return false;
-    bool ok = false;
-    dispatch_shape(I.dm, [&](auto s) { ok = PairShape<decltype(s)>::kOk; });
-    return ok;
-}
-bool pop_pair_own_shape(const Impl& I) {
-    bool own = false;
-    dispatch_shape(I.dm, [&](auto s) { own = PairShape<decltype(s)>::kOwn; });
-    return own;
-}
-bool pop_pair_step(const Impl& I, int chunk) {
-    return I.pop_pair && pop_on_matrix_cores(I) && (size_t)I.d.hidden[0] * (size_t)chunk * sizeof(float) <= ((size_t)2 << 20);
-}
 
 template <int From>
 static void launch_pop_split(Impl& I, const PopSource& src, int N, int M, int chunk, int chunks) {
@@ -206,8 +181,12 @@ bool lat_pair_on_matrix_cores(const Impl& I) { return pop_on_matrix_cores(I); }
 
 // k_lat_split for the models whose population is split, and for every shape compiled at init that it takes (no other
 // latent pair kernel is compiled for those); k_lat_pair_mfma for the rest, which in a default run are shapes compiled at
-// init, and with NTC_HIP_POP_PAIR=0 the listed ones: that run's gradients then come from 32-bit kernels throughout.
-static bool lat_pair_split(const Impl& I) { return split_pays(I.dm.nin, I.dm.nl) && (I.jit || I.pop_split); }
+// init, and with NTC_HIP_POP_PAIR=0 the listed ones.
+bool lat_split_step(const Impl& I) { return lat_pair_on_matrix_cores(I) && split_pays(I.dm.nin, I.dm.nl) && (I.jit || I.pop_split); }
+// k_qat_split for the shapes it pays for and 0 <= leak <= 1, whatever NTC_HIP_POP_PAIR is; k_qat_mfma for the rest
+bool qat_split_step(const Impl& I) {
+    return qat_on_matrix_cores(I) && split_qat_pays(I.dm.nin, I.dm.nl, I.dm.nout) && I.dm.leak >= 0.0f && I.dm.leak <= 1.0f;
+}
 
 void launch_lat_pair(Impl& I, int K, float sigma, unsigned mask) {
     ProfScope ps(I, "lat_pair");
@@ -215,7 +194,7 @@ void launch_lat_pair(Impl& I, int K, float sigma, unsigned mask) {
         launch_lat_pair_valu(I, K, sigma, mask);
         return;
     }
-    if (lat_pair_split(I)) {
+    if (lat_split_step(I)) {
         // as many blocks as fit the chip, or as 64-pixel rounds fill
         const size_t rounds = (I.npix + 63) / 64 * (size_t)K;
         const unsigned blocks = (unsigned)std::min<size_t>((size_t)I.cus * split_waves(I.dm.nin, I.dm.hidden[0], I.dm.nout), (rounds + 3) / 4);
@@ -251,7 +230,7 @@ void launch_lat_pair(Impl& I, int K, float sigma, unsigned mask) {
 }
 
 void launch_qat_mfma(Impl& I) {
-    if (split_qat_pays(I.dm.nin, I.dm.nl, I.dm.nout) && I.dm.leak >= 0.0f && I.dm.leak <= 1.0f) {
+    if (qat_split_step(I)) {
         // as many blocks as fit the chip; more where a wave would have over 64 rounds (its mask of rounds to search again)
         const size_t rounds = (I.npix + 63) / 64;
         const size_t fill = std::max((size_t)I.cus * qat_waves(I.dm.nin, I.dm.hidden[0], I.dm.nout, I.dm.lv[0].C), (rounds + 255) / 256);

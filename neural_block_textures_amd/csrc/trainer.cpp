@@ -395,7 +395,6 @@ bool Trainer::init(const ModelDesc& d, const float* z, const float* p, const flo
             fprintf(stderr, "ntc_hip backend: the runtime-shaped kernels run this model (%s)\n", jwhy.c_str());
         }
     }
-    I.pop_pair = pop_pair_possible(I);
     I.pop_split = pop_split_possible(I);
     if (I.pop_split) {
         const size_t slots = (size_t)I.Mcap + kSplitSlack, nf = slots * (split_inputs(d.nin) / 4), nt = slots * split_targets(d.nout);

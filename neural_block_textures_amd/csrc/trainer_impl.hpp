@@ -92,7 +92,7 @@ struct ntc_cuda::Trainer::Impl {
     // the 4 scales, as many slots of split_targets(nout) floats
     uint4* sfeat = nullptr;
     float *stgt = nullptr, *sscale = nullptr;
-    bool pop_split = false, pop_pair = false;
+    bool pop_split = false;
     float* wsets = nullptr;
     size_t wsets_cap = 0;      // floats
     float* eps_mlp = nullptr;
@@ -236,10 +236,9 @@ void launch_batch(Impl& I, int it, int M, int eps_pairs = 0, bool split = false,
 // its arrays), and whether the next one does
 bool pop_split_possible(const Impl& I);
 bool pop_split_step(const Impl& I);
-// ntc_trainer_on_matrix_cores' "pop_pair" and "pop_pair_own"
-bool pop_pair_possible(const Impl& I);
-bool pop_pair_step(const Impl& I, int chunk);
-bool pop_pair_own_shape(const Impl& I);
+// whether the latent pairs and the selector search do
+bool lat_split_step(const Impl& I);
+bool qat_split_step(const Impl& I);
 void launch_perturb(Impl& I, int it, float sigma, int N);
 // the Gaussians of one ES step (NS_MLP, it, pair, k) into eps_mlp, N x P
 void launch_fd_sets(Impl& I, float h);

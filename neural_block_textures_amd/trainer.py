@@ -479,8 +479,8 @@ class Trainer:
         self._lib.ntc_trainer_set_profiling(self._h, 1 if on else 0)
 
     def on_matrix_cores(self, stage: str) -> bool:
-        """whether the stage ("pop_eval", "lat_pair", "qat_search") runs on the matrix cores; "pop_split": whether ES steps
-        take the split population kernel; "pop_pair", "pop_pair_own": the shapes and sizes that include/ntc_hip.h gives"""
+        """whether the stage ("pop_eval", "lat_pair", "qat_search") runs on the matrix cores; "pop_split", "lat_split",
+        "qat_split": whether on their 16-bit instructions with operands in parts"""
         return bool(self._lib.ntc_trainer_on_matrix_cores(self._h, stage.encode()))
 
     def set_matrix_cores(self, on: bool):

@@ -10,6 +10,7 @@ import numpy as np
 import pytest
 
 from neural_block_textures_amd import synth
+from neural_block_textures_amd.trainer import Layout
 from tests.gpu_common import LAYOUTS, data, rel, say, trainer
 
 pytestmark = pytest.mark.gpu
@@ -248,30 +249,39 @@ def test_matrix_core_choice(orc, name, mfma):
     assert tr.on_matrix_cores("lat_pair") == mfma
 
 
-@pytest.mark.parametrize("name,pair", [("material", True), ("dct_plane", True), ("two_level", True), ("rgb_16x2", True),
-                                       ("large", False), ("dct_17", False), ("material_valu", False)])
-def test_pair_population_kernel_choice(orc, name, pair):
-    """ES steps share a pair's first layer on the fixed shapes with one or two 16-unit hidden tiles (k_pop_pair: the
-    12-output material and the 3-output 32-wide ones; k_pop_pair_own: the pixel-per-lane 16-wide one); not the 64-wide
-    one, a 17-wide one or the VALU kernels"""
+@pytest.mark.parametrize("name,split", [("material", True), ("material_clamp", True), ("dct_plane", True), ("two_level", True),
+                                        ("rgb_16x2", True), ("large", True), ("dct_17", True), ("chief1_36", True), ("run8x3", True),
+                                        ("jit_mfma_28", True), ("jit_valu_7", False), ("material_valu", False), ("runtime", False)])
+def test_split_kernel_choice(orc, monkeypatch, name, split):
+    """the population (ES steps and central differences) and the latent pairs run on the 16-bit instructions with operands in
+    parts on every shape of at most 16 inputs and two hidden layers that the matrix cores take; not on the VALU kernels, and not
+    with NTC_HIP_POP_PAIR=0, but for the latent pairs of a shape compiled at init"""
     lay = LAYOUTS[name]
     z, p, tgt = data(lay, 8)
-    tr = trainer(lay, z, p, tgt)
-    assert tr.on_matrix_cores("pop_pair") == pair
-    assert tr.on_matrix_cores("pop_pair_own") == (pair and name == "rgb_16x2")
-    tr.close()
-
-
-def test_pair_population_kernel_chunk_in_l2(orc):
-    """the pair kernels read each chunk's first layer (H x chunk floats) from the L2: a step whose chunk would take more
-    than 2 MiB evaluates on k_pop_mfma (2048 pairs of 65536 slots: one chunk, 8 MiB for 32 units), a step of the same
-    model with fewer pairs (smaller chunks) on k_pop_pair"""
-    lay = LAYOUTS["dct_plane"]
-    z, p, tgt = data(lay, 8)
-    for pairs, pair in ((2048, False), (64, True)):
-        tr = trainer(lay, z, p, tgt, max_pairs=pairs, max_batch=65536)
-        assert tr.on_matrix_cores("pop_pair") == pair, pairs
+    for env in (None, "0"):
+        if env:
+            monkeypatch.setenv("NTC_HIP_POP_PAIR", env)
+        tr = trainer(lay, z, p, tgt)
+        assert tr.on_matrix_cores("pop_split") == (split and not env)
+        assert tr.on_matrix_cores("lat_split") == (split and (not env or name.startswith("jit")))
+        unit = lay.levels[0][:2] == (lay.W, lay.H)
+        assert tr.on_matrix_cores("qat_split") == (split and unit)
+        tr.set_matrix_cores(False)
+        assert not any(tr.on_matrix_cores(s) for s in ("pop_split", "lat_split", "qat_split"))
         tr.close()
+
+
+@pytest.mark.parametrize("channels,hidden,T,split,qat", [(14, [24, 24], 1, True, True), (15, [24, 24], 1, False, False), (6, [24] * 3, 1, False, False),
+                                                        (6, [24], 1, True, False), (6, [24], 4, True, True)])
+def test_split_kernel_limits(orc, channels, hidden, T, split, qat):
+    """16 inputs are the most and two hidden layers; the selector search with one only of more than 4 outputs"""
+    lay = Layout(32, 24, [(32, 24, channels, True)], hidden, T=T, leak=0.01)
+    z, p, tgt = data(lay, 8)
+    tr = trainer(lay, z, p, tgt)
+    assert tr.on_matrix_cores("pop_eval")
+    assert tr.on_matrix_cores("pop_split") == split and tr.on_matrix_cores("lat_split") == split
+    assert tr.on_matrix_cores("qat_search") and tr.on_matrix_cores("qat_split") == qat
+    tr.close()
 
 
 @pytest.mark.parametrize("name", ["jit_valu_7", "jit_mfma_28", "jit_widths", "runtime"])
