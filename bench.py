@@ -371,7 +371,7 @@ def run_gpu(w, steps, warmup, fd_steps=0, seconds=0.0, settle=0.0):
         fd = {"iters_per_s": fd_steps / fd_el, "ms_per_iter": 1e3 * fd_el / fd_steps,
               "evals_per_s": (2 * (w.layout.nparams + 1) * w.mlp_batch) * fd_steps / fd_el,
               "pop_eval_ms": round(fd_pop_ms / max(fd_pop_n, 1), 4),
-              "pop_kernel": "k_pop_mfma" if tr.on_matrix_cores("pop_eval") else "k_pop_eval"}
+              "pop_kernel": "k_pop_split" if tr.on_matrix_cores("pop_split") else "k_pop_mfma" if tr.on_matrix_cores("pop_eval") else "k_pop_eval"}
     refit = None
     if w.dct_q:   # the device refit (probe + re-snap) against the reference's host path for the same step
         tr.synchronize()
@@ -407,8 +407,8 @@ def roofline_of(w, r):
     achieved = pop_flop / (pe["ms_mean"] * 1e-3) / 1e12
     # the VALU kernels (--valu) against the FP32 VALU peak without packed instructions
     bound, peak = ("mfma", FP32_PEAK_TFLOPS) if r["pop_kernel"] != "k_pop_eval" else ("valu", VALU_F32_PEAK_TFLOPS)
-    if r["pop_kernel"] == "k_pop_split":   # each multiply-add is three 16-bit products
-        peak = round(F16_PEAK_TFLOPS / 3, 1)
+    if r["pop_kernel"] == "k_pop_split":   # each multiply-add is four 16-bit products
+        peak = round(F16_PEAK_TFLOPS / 4, 1)
     roof = {"bound": bound, "achieved": round(achieved, 3), "peak": peak, "unit": "TFLOP/s",
             "frac": round(achieved / peak, 4), "traffic": None, "kernel": r["pop_kernel"],
             "flop_per_launch": pop_flop, "ms_per_launch": pe["ms_mean"]}
