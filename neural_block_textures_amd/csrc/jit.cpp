@@ -75,8 +75,9 @@ void make_dirs(const std::string& path) {
         if (i == path.size() || path[i] == '/') mkdir(path.substr(0, i).c_str(), 0755);
 }
 
-// the name expressions one program instantiates; pop: the matrix-core kernels, else the VALU ones
-std::vector<std::string> expressions(const std::string& shape, const DevModel& m, bool pop) {
+// the name expressions one program instantiates; pop: the matrix-core kernels, else the VALU ones; split: the trainer's population
+// runs on k_pop_split (pop_split_fits), so the 32-bit population kernels, which it never launches, are left out
+std::vector<std::string> expressions(const std::string& shape, const DevModel& m, bool pop, bool split) {
     auto e = [&](const char* k, const std::string& t) { return std::string("ntc_hip::") + k + "<" + shape + (t.empty() ? "" : ", " + t) + ">"; };
     std::vector<std::string> v;
     if (!pop) {
@@ -91,11 +92,10 @@ std::vector<std::string> expressions(const std::string& shape, const DevModel& m
     const bool unit = m.leak >= 0.0f && m.leak <= 1.0f;
     if (unit) {
         const int a_fd = kActMax, a_es = kActFold;
-        v.push_back(e("k_pop_mfma", std::to_string(a_fd) + ", " + c + ", 0"));
-        v.push_back(e("k_pop_mfma", std::to_string(a_es) + ", " + c + ", 1"));
-        v.push_back(e("k_pop_mfma", std::to_string(a_es) + ", " + c + ", 2"));
-        if (split_pays(m.nin, m.nl))
-            for (int from : { 0, 1, 2 }) v.push_back(e("k_pop_split", c + ", " + std::to_string(from) + ", false"));
+        for (int from : { 0, 1, 2 }) {
+            if (split) v.push_back(e("k_pop_split", c + ", " + std::to_string(from) + ", false"));
+            else v.push_back(e("k_pop_mfma", std::to_string(from == 0 ? a_fd : a_es) + ", " + c + ", " + std::to_string(from)));
+        }
         if (split_pays(m.nin, m.nl)) v.push_back(e("k_lat_split", c + ", false"));
         else v.push_back(e("k_lat_pair_mfma", std::to_string(a_es) + ", " + c));
     }
@@ -224,16 +224,16 @@ bool jit_prepare(Impl& I, std::string& why) {
     hiprtcVersion(&rv_major, &rv_minor);
     key_src += "|hiprtc " + std::to_string(rv_major) + "." + std::to_string(rv_minor);
     const std::string arch = I.arch.substr(0, I.arch.find(':'));
-    const bool mfma = jit_shape_mfma(js);
+    const bool mfma = jit_shape_mfma(js), split = pop_split_fits(I);
     const std::string setkey = std::to_string(I.device) + "|" + shape + "|" + std::to_string(I.dm.leak) + "|" + std::to_string(I.dm.clamp_out) +
-                               "|" + std::to_string(fnv1a(key_src));
+                               "|" + std::to_string(split) + "|" + std::to_string(fnv1a(key_src));
     std::lock_guard<std::mutex> lock(g_mu);
     if (auto it = g_sets.find(setkey); it != g_sets.end()) { I.jit = it->second; return true; }
     auto* set = new JitModuleSet();
     set->shape = shape;
     set->mfma = mfma;
     for (int pop = 0; pop < (mfma ? 2 : 1); pop++) {
-        const auto exprs = expressions(shape, I.dm, pop != 0);
+        const auto exprs = expressions(shape, I.dm, pop != 0, split);
         std::string code;
         std::vector<std::string> lowered;
         if (!build_program(csrc, arch, pop ? "kern_pop.hpp" : "kern_decode.hpp", exprs, pop != 0, key_src, code, lowered, why)) {
@@ -264,8 +264,8 @@ bool jit_compile_only(const DevModel& m, const std::string& arch, std::string& w
     for (int pop = 0; pop < (mfma ? 2 : 1); pop++) {
         std::string code;
         std::vector<std::string> lowered;
-        if (!build_program(csrc, arch, pop ? "kern_pop.hpp" : "kern_decode.hpp", expressions(shape, m, pop != 0), pop != 0, "", code, lowered,
-                           why, false))   // compiled every time, never cached
+        if (!build_program(csrc, arch, pop ? "kern_pop.hpp" : "kern_decode.hpp", expressions(shape, m, pop != 0, split_pays(m.nin, m.nl)), pop != 0,
+                           "", code, lowered, why, false))   // compiled every time, never cached
             return false;
         if (code.empty()) { why = "empty code object"; return false; }
     }

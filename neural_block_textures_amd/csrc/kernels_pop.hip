@@ -116,14 +116,14 @@ void launch_pop_eval_fd(Impl& I, float h, int M, int chunk, int chunks) {
 // (split_pays) and minibatches its offsets hold. Against the 32-bit kernel on the MI355X: see k_pop_split. NTC_HIP_POP_PAIR=0
 // (read at init) keeps k_pop_mfma for the population, and k_lat_pair_mfma for the latent pairs of the listed shapes: the 32-bit
 // kernels that the tests compare the split ones with.
-bool pop_split_possible(const Impl& I) {
-    if (!pop_on_matrix_cores(I)) return false;
+bool pop_split_fits(const Impl& I) {
     const char* env = getenv("NTC_HIP_POP_PAIR");
     // (its arrays are read through 32-bit offsets: for 9 to 12 inputs 67 million slots, where k_pop_mfma's hold 89 million)
     const uint64_t slots = (uint64_t)I.Mcap + kSplitSlack, most = (uint64_t)1 << 32;
     const bool fits = slots * 4u * split_inputs(I.dm.nin) < most && slots * 4u * split_targets(I.dm.nout) < most;
     return !(env && env[0] == '0') && split_pays(I.dm.nin, I.dm.nl) && fits;
 }
+bool pop_split_possible(const Impl& I) { return pop_on_matrix_cores(I) && pop_split_fits(I); }
 bool pop_split_step(const Impl& I) { return I.pop_split && pop_on_matrix_cores(I); }
 
 template <int From>

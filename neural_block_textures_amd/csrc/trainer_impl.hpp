@@ -235,6 +235,7 @@ void launch_batch(Impl& I, int it, int M, int eps_pairs = 0, bool split = false,
 // whether this model's ES steps take the split population kernel (k_pop_split; decided at init, the trainer then keeps
 // its arrays), and whether the next one does
 bool pop_split_possible(const Impl& I);
+bool pop_split_fits(const Impl& I);   // the same of a model that the matrix cores take, before its kernels are compiled
 bool pop_split_step(const Impl& I);
 // whether the latent pairs and the selector search do
 bool lat_split_step(const Impl& I);

@@ -244,3 +244,23 @@ def test_split_population_past_32_bit_offsets():
         tr.close()
         e = (d * d).sum(1) / (3.0 * lay.T)
         assert abs(loss - e.mean()) <= 5 * e.std() / np.sqrt(M) + 1e-6 * e.mean()
+
+
+@pytest.mark.parametrize("hidden,leak", [([23, 23], 0.03), ([29], 0.0)])
+def test_specialised_shapes_compile_one_population(orc, monkeypatch, tmp_path, hidden, leak):
+    """a shape compiled at init holds the population kernels its trainer launches and no others: k_pop_split's, or with
+    NTC_HIP_POP_PAIR=0 k_pop_mfma's (the three of both take a third longer to compile); one process runs both"""
+    monkeypatch.setenv("NTC_HIP_JIT_CACHE", str(tmp_path))
+    lay = Layout(40, 24, [(10, 6, 4, False)], hidden, T=4, leak=leak)
+    z, p, tgt = data(lay, 32)
+    for env, kernel, other in ((None, "k_pop_split", "k_pop_mfma"), ("0", "k_pop_mfma", "k_pop_split")):
+        if env:
+            monkeypatch.setenv("NTC_HIP_POP_PAIR", env)
+        old = set(tmp_path.glob("*.names"))
+        for pairs, batch in ((3, 100), (2, 1200)):
+            check(orc, lay, z, p, tgt, pairs, batch)
+        names = "".join(f.read_text() for f in set(tmp_path.glob("*.names")) - old)
+        assert names.count(kernel) == 3 and other not in names
+        tr = trainer(lay, z, p, tgt, max_pairs=4, max_batch=100)
+        tr.mlp_step_fd(1, 1e-3, 0.0, 100)
+        tr.close()
