@@ -1208,7 +1208,7 @@ __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(qat_oc
 // material512, two channels of four values (MI355X): 73 -> 38 us.
 // With one hidden layer a candidate is the output layer alone, of which at most 4 outputs are a small part of a matrix tile: those
 // models stay on k_qat_mfma, whose output layer is on the VALU (7-32-3, one channel, 512 x 512: 26 us against 31).
-// (a wave per SIMD fewer than k_pop_split with more than one searched channel, whose first-layer weights are in registers too)
+// (a wave per SIMD fewer than k_lat_split with more than one searched channel, whose first-layer weights are in registers too)
 constexpr int qat_waves(int nin, int H, int nout, int c0) { return split_waves(nin, H, nout) - (c0 > 1 && H <= 48 ? 1 : 0); }
 template <class S, bool Clamp, bool UnitCw>
 __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(qat_waves(S::kNin, S::kH, S::kNout, S::kC0)))) k_qat_split(DevModel m, const float* __restrict__ w, float* __restrict__ zdec,
