@@ -78,16 +78,19 @@ struct GatherLevels {
     int mode[kMaxLevels];
     float* zq_copy[kMaxLevels];
 };
-// Wide: kRows or kRuns if a level of the launch is, else kNarrow
-template <int Wide>
-__global__ void __launch_bounds__(64 * kGatherWaves) k_lat_gather(DevModel m, GatherLevels G, int K, float scale,
+// Wide: kRows or kRuns if a level of the launch is, else kNarrow. Waves: a block's most. Steps of at most four pairs, which need
+// one, are compiled for one (barriers and the wave's index go: levels of 128 x 128 x 8 and 32 x 32 x 4 under 512 x 512 pixels, 4
+// pairs, 56.2 -> 54.7 us). The loop over pairs in `channel` is not unrolled: by four it took 104 scalar registers, which leave 7
+// waves a SIMD for 8 (1024 x 1024 x 4 and 256 x 256 x 8 under 2048 x 2048 pixels, 4 pairs, 381 -> 376 us).
+template <int Wide, int Waves>
+__global__ void __launch_bounds__(64 * Waves) k_lat_gather(DevModel m, GatherLevels G, int K, float scale,
                                                                   const float* __restrict__ dpix,
                                                                   const float* __restrict__ eps, const int* __restrict__ ranges,
                                                                   int rate0, float rate_scale, int dct_bw, int dct_n,
                                                                   const int32_t* __restrict__ dbits, float* __restrict__ grad,
                                                                   int first, int adam, float* __restrict__ z, float* __restrict__ zm,
                                                                   float* __restrict__ zv, float lr, float c1, float c2, LatAhead ah) {
-    const int threads = (int)blockDim.x;
+    const int threads = Waves == 1 ? 64 : (int)blockDim.x;
     if ((int)blockIdx.x >= G.start[G.n]) {   // a draw-ahead block (uniform: the whole block returns here)
         const int d = (int)blockIdx.x - G.start[G.n], k = d / ah.eb;
         const uint64_t head = noise_head(ah.seed, NS_LAT, ah.next_step, (uint32_t)k);
@@ -96,7 +99,7 @@ __global__ void __launch_bounds__(64 * kGatherWaves) k_lat_gather(DevModel m, Ga
             if ((ah.mask >> level_of(m, i)) & 1u) ah.eps_next[(size_t)k * m.nz + i] = gauss_at(ah.nt, head, (uint64_t)i);
         return;
     }
-    __shared__ float dsum[kGatherWaves * kGatherPairs][kGatherTex];
+    __shared__ float dsum[Waves * kGatherPairs][kGatherTex];
     extern __shared__ float stage_s[];   // with a level of kRows: kGatherPairs x kWideRow floats per wave
     int li = 0;   // this block's level (uniform)
     while (li + 1 < G.n && (int)blockIdx.x >= G.start[li + 1]) li++;
@@ -110,7 +113,6 @@ __global__ void __launch_bounds__(64 * kGatherWaves) k_lat_gather(DevModel m, Ga
         const size_t i = (size_t)(L.off + ((long long)ty * L.W + tx) * L.C + c);
         const int blk = (ty / 8) * dct_bw + tx / 8;
         float gc = (first && k0 == 0) ? 0.0f : grad[i];
-#pragma unroll 4
         for (int kk = 0; kk < kn; kk++) {
             const float ei = eps[(size_t)(k0 + kk) * m.nz + i];
             gc = __builtin_fmaf(d(kk) * scale, ei, gc);
@@ -132,7 +134,7 @@ __global__ void __launch_bounds__(64 * kGatherWaves) k_lat_gather(DevModel m, Ga
             channel(t % L.W, t / L.W, c, 0, K, [&](int kk) { return 0.0f + dpix[(size_t)kk * m.npix + t]; });
         return;
     }
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, j = lane % kGatherTex, q = lane / kGatherTex;
+    const int lane = threadIdx.x & 63, wave = Waves == 1 ? 0 : threadIdx.x >> 6, j = lane % kGatherTex, q = lane / kGatherTex;
     const int tiles = (L.W + kGatherTex - 1) / kGatherTex, ty = blk0 / tiles, tx = (blk0 - ty * tiles) * kGatherTex + j;
     const bool live = tx < L.W;
     const int* R = ranges + L.rng;
@@ -314,7 +316,11 @@ void launch_lat_gather(Impl& I, unsigned mask, int k0, int K, float scale, bool 
         exit(1);
     }
     ProfScope ps(I, "lat_gather");
-    hipLaunchKernelGGL((wide == kRows ? k_lat_gather<kRows> : wide == kRuns ? k_lat_gather<kRuns> : k_lat_gather<kNarrow>), dim3((unsigned)grid), dim3(threads),
+    auto* const kern = wide == kRows   ? k_lat_gather<kRows, kGatherWaves>
+                       : wide == kRuns ? k_lat_gather<kRuns, 1>
+                       : threads == 64 ? k_lat_gather<kNarrow, 1>
+                                       : k_lat_gather<kNarrow, kGatherWaves>;
+    hipLaunchKernelGGL(kern, dim3((unsigned)grid), dim3(threads),
                        wide == kRows ? (size_t)threads / 64 * kGatherPairs * kWideRow * sizeof(float) : 0, I.stream, I.dm, G, K,
                        scale, I.dpix, I.eps_lat,
                        I.ranges, rate ? 1 : 0, I.ddct.rate_scale, I.ddct.BW, I.ddct.n, rate ? I.dct_dbits + (size_t)k0 * I.ddct.n : nullptr,
